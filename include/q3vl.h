@@ -492,9 +492,13 @@ int q3_batched_gemm_backward(const void* x, const void* w, const void* dy, void*
  * (B, Hq, Sq, D), k, v, grad_k, grad_v (B, Hkv, Sk, D), all contiguous; lse
  * (B, Hq, Sq) fp32 natural-log row log-sum-exp of the scaled scores (as
  * q3_flash_attention writes it); D <= 128; causal masks key j > query i.
- * Workspace: q3_flash_attention_backward_workspace_bytes (one fp32 per query
- * row). */
+ * Workspace: at least q3_flash_attention_backward_workspace_bytes (one fp32 per
+ * query row); with q3_flash_attention_backward_mfma_workspace_bytes (row
+ * statistics and fp32 partials) bf16 tensors of D = 64, 72, 80, 96 or 128 run on
+ * the matrix cores, otherwise on the SIMT kernels. */
 int64_t q3_flash_attention_backward_workspace_bytes(int64_t B, int64_t Hq, int64_t Sq);
+int64_t q3_flash_attention_backward_mfma_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t Sk,
+                                                         int64_t D, int dtype);
 int q3_flash_attention_backward(const void* q, const void* k, const void* v, const void* o, const float* lse,
                                 const void* grad_out, void* grad_q, void* grad_k, void* grad_v, int64_t B, int64_t Hq,
                                 int64_t Hkv, int64_t Sq, int64_t Sk, int64_t D, float scale, int is_causal,

@@ -99,6 +99,7 @@ _SIGS: dict[str, tuple] = {
     "q3_batched_gemm_backward_workspace_bytes": (c_int64, [_I, _I, _I, _I, c_int]),
     "q3_batched_gemm_backward": (c_int, [_V, _V, _V, _V, _V, _I, _I, _I, _I, c_int, _V, _I, _V]),
     "q3_flash_attention_backward_workspace_bytes": (c_int64, [_I, _I, _I]),
+    "q3_flash_attention_backward_mfma_workspace_bytes": (c_int64, [_I, _I, _I, _I, _I, _I, c_int]),
     "q3_flash_attention_backward": (c_int, [_V, _V, _V, _V, _f32p, _V, _V, _V, _V, _I, _I, _I, _I, _I, _I, c_float,
                                             c_int, c_int, _V, _I, _V]),
 }

@@ -33,10 +33,11 @@ HIPFLAGS = [
 ]
 
 
-# Per-source extra flags. attention.hip: MFMA results in arch VGPRs rather than
+# Per-source extra flags. The attention sources: MFMA results in arch VGPRs rather than
 # AGPRs (its kernels' whole state fits the 256 registers of 2 waves per SIMD;
 # with AGPRs the softmax copied every score tile out of them).
-EXTRA_FLAGS: dict[str, list[str]] = {"attention.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+EXTRA_FLAGS: dict[str, list[str]] = {src: ["-mllvm", "-amdgpu-mfma-vgpr-form"]
+                                     for src in ("attention.hip", "attention_bwd.hip")}
 
 
 def _hipcc() -> str:

@@ -104,7 +104,8 @@ class FlashAttentionFunction(torch.autograd.Function):
         B, Hq, Sq, D = q.shape
         Hkv, Sk = k.shape[1], k.shape[2]
         dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-        ws, nws = _lib.workspace(_lib.lib().q3_flash_attention_backward_workspace_bytes(B, Hq, Sq), q.device)
+        ws, nws = _lib.workspace(_lib.lib().q3_flash_attention_backward_mfma_workspace_bytes(
+            B, Hq, Hkv, Sq, Sk, D, _dt(q)), q.device)
         _lib.call("q3_flash_attention_backward", q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
                   lse.data_ptr(), _c(do).to(q.dtype).data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), B, Hq,
                   Hkv, Sq, Sk, D, ctx.scale, int(ctx.is_causal), _dt(q), _lib.ptr(ws), nws, _lib.stream())

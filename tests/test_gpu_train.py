@@ -277,6 +277,45 @@ def test_flash_attention_backward_bf16(B, Hq, Hkv, Sq, Sk, D, causal):
     twice_equal(lambda: run_grads(_fa(Hq // Hkv, causal, s), [q, k, v], dy)[1])
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,D,causal", [
+    (1, 4, 1, 1, 1, 128, True), (2, 2, 2, 31, 33, 64, False), (1, 8, 2, 129, 129, 128, True),
+    (1, 8, 2, 64, 200, 128, True), (1, 8, 2, 200, 64, 128, True), (1, 6, 2, 97, 127, 96, False),
+    (2, 3, 3, 128, 128, 72, False), (1, 16, 1, 257, 257, 80, True), (3, 4, 4, 33, 96, 72, True),
+    (1, 32, 8, 640, 640, 128, True),
+])
+def test_flash_attention_backward_mfma_against_simt(B, Hq, Hkv, Sq, Sk, D, causal):
+    """The MFMA backward (tile, split and causal edges) against the fp32 oracle, and against the SIMT kernels (which
+    a workspace of one float per row selects) on the same o and lse. Both keep P and dS in fp32 (the MFMA kernels as
+    two bf16 terms, 2^-17 relative) and round once, so an element may differ by one bf16 rounding of its own value
+    (2^-7 of it), the fp32 sums' error over terms up to the largest result (2^-14 of it), and, where dP - Dv cancels
+    (one key: dS is 0 up to rounding), the fp32 rounding of dP and Dv (a few 2^-24 of the largest dP, here 2^-21)
+    times the largest |scale * q| or |scale * k|."""
+    from qwen3_5_vl_cuda_custom_amd import _lib
+    from qwen3_5_vl_cuda_custom_amd.kernels.flash_attention import flash_attention_lse
+    q, k, v = (rnd(B, Hq, Sq, D, seed=64).bfloat16(), rnd(B, Hkv, Sk, D, seed=65).bfloat16(),
+               rnd(B, Hkv, Sk, D, seed=66).bfloat16())
+    dy = rnd(B, Hq, Sq, D, seed=67).bfloat16()
+    s = D ** -0.5
+    _, got = run_grads(_fa(Hq // Hkv, causal, s), [q, k, v], dy)
+    _, ref = ref_grads(_fa_ref(Hq // Hkv, causal, s), [q, k, v], dy)
+    qd, kd, vd, dyd = (t.to(DEV) for t in (q, k, v, dy))
+    o, lse = flash_attention_lse(qd, kd, vd, s, causal, Hq // Hkv)
+    simt = [torch.empty_like(t) for t in (qd, kd, vd)]
+    nws = _lib.lib().q3_flash_attention_backward_workspace_bytes(B, Hq, Sq)
+    ws = torch.empty(nws, dtype=torch.uint8, device=DEV)
+    _lib.call("q3_flash_attention_backward", *(t.data_ptr() for t in (qd, kd, vd, o, lse, dyd, *simt)), B, Hq, Hkv,
+              Sq, Sk, D, s, int(causal), _lib.dtype_code(q.dtype), ws.data_ptr(), nws, _lib.stream())
+    dp = (dy.float() @ v.float().repeat_interleave(Hq // Hkv, dim=1).transpose(-1, -2)).abs().max()
+    noise = 2.0 ** -21 * float(dp * torch.maximum(q.abs().max(), k.abs().max())) * s
+    for a, r, b, n in zip(got, ref, simt, ("dq", "dk", "dv")):
+        x, y = a.float(), b.float()
+        tol = 2.0 ** -7 * torch.maximum(x.abs(), y.abs()) + 2.0 ** -14 * y.abs().max() + noise
+        over = float(((x - y).abs() - tol).max())
+        assert over <= 0, f"{n} vs SIMT: {over:.3e} over"
+        if float(r.abs().max()) > 1e-6:  # one key: P = 1, dS = 0 up to rounding
+            assert_grad_close(a, r, f"flash {n} D={D}")
+
+
 # ------------------------------------------------------------------ embedding, rotary, routing
 @pytest.mark.parametrize("dtype,padding_idx", [(torch.float32, None), (torch.bfloat16, 3)])
 def test_embedding_backward(dtype, padding_idx):
