@@ -471,8 +471,11 @@ int q3_transpose(const void* a, void* b, int64_t E, int64_t R, int64_t C, int dt
  * the three may be null. The operands are transposed into `workspace`
  * (q3_matmul_backward_workspace_bytes) and multiplied by q3_matmul, which may
  * use `gemm_ws` as q3_matmul's workspace (zero-filled before first use, as
- * there; size at least q3_matmul_workspace_bytes of both products). */
+ * there; size at least q3_matmul_workspace_bytes of both products;
+ * q3_matmul_backward_gemm_workspace_bytes also covers the weight gradient's
+ * product over the padded row count it runs at). */
 int64_t q3_matmul_backward_workspace_bytes(int64_t M, int64_t N, int64_t K, int dtype);
+int64_t q3_matmul_backward_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int dtype);
 int q3_matmul_backward(const void* x, const void* w, const void* dy, void* gx, void* gw, void* gb, int64_t M,
                        int64_t N, int64_t K, int dtype, void* workspace, int64_t workspace_bytes, void* gemm_ws,
                        int64_t gemm_ws_bytes, void* stream);

@@ -466,54 +466,112 @@ __global__ __launch_bounds__(kT) void topk_bwd_kernel(const T* __restrict__ gv, 
 }
 
 // ===================================================================== transpose
-// (E, R, C) -> (E, C, R) through a 64 x 65 LDS tile.
+// (E, R, C) -> (E, C, ldb), columns R .. ldb - 1 of the result zero. Bound by
+// memory: one read and one write of each element.
+//
+// bf16 with 16-byte rows on both sides: a 64 x 64 tile through LDS (rows 72
+// elements apart, so the 4 rows of a transposed read fall into distinct
+// banks); 16-byte loads, and ds_read_b64_tr_b16 hands each lane 4 rows of its
+// column, two of them one 16-byte piece of an output row (64-byte runs per
+// wave and row). Against 2-byte accesses through a 64 x 65 tile: the 21
+// transposes of a dense layer's backward at S=2048 583 -> 311 us, the three of
+// a 151936 x 4096 head's at 1023 rows 1306 -> 623 us (4.6 TB/s).
+typedef short tr_short4 __attribute__((ext_vector_type(4)));
+typedef short tr_short8 __attribute__((ext_vector_type(8)));
+constexpr int kTrLd = 72;
+
+__global__ __launch_bounds__(kT) void transpose_vec_kernel(const bf16* __restrict__ a, bf16* __restrict__ b,
+                                                           int64_t R, int64_t C, int64_t ldb) {
+  __shared__ __attribute__((aligned(16))) bf16 tile[64 * kTrLd];
+  const int64_t e = blockIdx.z;
+  const bf16* ae = a + e * R * C;
+  bf16* be = b + e * C * ldb;
+  const int64_t c0 = (int64_t)blockIdx.x * 64, r0 = (int64_t)blockIdx.y * 64;
+  const int tid = threadIdx.x;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int r = (tid >> 3) + 32 * i, c = (tid & 7) * 8;
+    bf16x8 v = bf16x8{};
+    if (r0 + r < R && c0 + c < C) v = *reinterpret_cast<const bf16x8*>(ae + (r0 + r) * C + c0 + c);
+    *reinterpret_cast<bf16x8*>(tile + r * kTrLd + c) = v;
+  }
+  __syncthreads();
+  // wave w takes columns 16 w .. 16 w + 15; lane group g (16 lanes) rows 32 i + 8 g .. + 7
+  const int lane = tid & 63, w = tid >> 6, g = lane >> 4, rr = (lane & 15) >> 2, qq = lane & 3;
+  const int64_t c = c0 + 16 * w + (lane & 15);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int r = 32 * i + 8 * g;
+    auto rd = [&](int row) {
+      return __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_short4 __attribute__((address_space(3)))*)(
+          reinterpret_cast<uintptr_t>(tile + (row + rr) * kTrLd + 16 * w + 4 * qq)));
+    };
+    const tr_short4 lo = rd(r), hi = rd(r + 4);
+    const tr_short8 v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    if (c < C && r0 + r < ldb) *reinterpret_cast<tr_short8*>(be + c * ldb + r0 + r) = v;
+  }
+}
+
+// Any type and row length, through a 64 x 65 LDS tile.
 template <typename T>
 __global__ __launch_bounds__(kT) void transpose_kernel(const T* __restrict__ a, T* __restrict__ b, int64_t R,
-                                                       int64_t C) {
+                                                       int64_t C, int64_t ldb) {
   __shared__ T tile[64][65];
   const int64_t e = blockIdx.z;
   const T* ae = a + e * R * C;
-  T* be = b + e * R * C;
+  T* be = b + e * C * ldb;
   const int64_t c0 = (int64_t)blockIdx.x * 64, r0 = (int64_t)blockIdx.y * 64;
   const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
   for (int i = ty; i < 64; i += kT / 64) {
     const int64_t r = r0 + i, c = c0 + tx;
-    if (r < R && c < C) tile[i][tx] = ae[r * C + c];
+    tile[i][tx] = r < R && c < C ? ae[r * C + c] : from_f<T>(0.f);
   }
   __syncthreads();
   for (int i = ty; i < 64; i += kT / 64) {
     const int64_t c = c0 + i, r = r0 + tx;
-    if (r < R && c < C) be[c * R + r] = tile[tx][i];
+    if (r < ldb && c < C) be[c * ldb + r] = tile[tx][i];
   }
 }
 
-int transpose(const void* a, void* b, int64_t E, int64_t R, int64_t C, int dtype, hipStream_t st) {
+int transpose(const void* a, void* b, int64_t E, int64_t R, int64_t C, int64_t ldb, int dtype, hipStream_t st) {
   if (E == 0 || R == 0 || C == 0) return Q3_OK;
-  const dim3 grid((unsigned)q3_cdiv(C, 64), (unsigned)q3_cdiv(R, 64), (unsigned)E);
-  if (dtype == Q3_BF16)
-    hipLaunchKernelGGL(transpose_kernel<bf16>, grid, dim3(kT), 0, st, static_cast<const bf16*>(a),
-                       static_cast<bf16*>(b), R, C);
-  else
+  const dim3 grid((unsigned)q3_cdiv(C, 64), (unsigned)q3_cdiv(ldb, 64), (unsigned)E);
+  if (dtype == Q3_BF16) {
+    const bf16* s = static_cast<const bf16*>(a);
+    bf16* d = static_cast<bf16*>(b);
+    if (C % 8 == 0 && ldb % 8 == 0 && q3_aligned(a, 16) && q3_aligned(b, 16))
+      hipLaunchKernelGGL(transpose_vec_kernel, grid, dim3(kT), 0, st, s, d, R, C, ldb);
+    else
+      hipLaunchKernelGGL(transpose_kernel<bf16>, grid, dim3(kT), 0, st, s, d, R, C, ldb);
+  } else {
     hipLaunchKernelGGL(transpose_kernel<float>, grid, dim3(kT), 0, st, static_cast<const float*>(a),
-                       static_cast<float*>(b), R, C);
+                       static_cast<float*>(b), R, C, ldb);
+  }
   Q3_LAUNCH_CHECK();
   return Q3_OK;
 }
 
+// Row length of the transposed activations (dY^T and X^T of M rows), the
+// reduction length of the weight gradient's GEMM: the MFMA kernels take rows
+// of a multiple of 8 elements (any other M would leave the GEMM to the SIMT
+// kernel: M = 1023, N = 151936, K = 4096 70.2 ms), and whole 64-element stages
+// start on cache lines; the padding columns are zeros on both sides.
+int64_t padded_rows(int64_t M, int dtype) { return dtype == Q3_BF16 ? q3_cdiv(M, 64) * 64 : M; }
+
 int64_t align256(int64_t n) { return (n + 255) / 256 * 256; }
 
-// Workspace of the matmul backward: W^T (K, N), dY^T (N, M), X^T (K, M) and
-// the bias gradient's partial sums.
+// Workspace of the matmul backward: W^T (K, N), dY^T (N, Mp), X^T (K, Mp) with
+// Mp = padded_rows(M), and the bias gradient's partial sums.
 struct MmBwdLayout {
   int64_t wt, dyt, xt, part, total;
 };
 MmBwdLayout mm_bwd_layout(int64_t M, int64_t N, int64_t K, int dtype) {
-  const int64_t es = dtype == Q3_BF16 ? 2 : 4;
+  const int64_t es = dtype == Q3_BF16 ? 2 : 4, Mp = padded_rows(M, dtype);
   MmBwdLayout l{};
   l.wt = 0;
   l.dyt = l.wt + align256(K * N * es);
-  l.xt = l.dyt + align256(N * M * es);
-  l.part = l.xt + align256(K * M * es);
+  l.xt = l.dyt + align256(N * Mp * es);
+  l.part = l.xt + align256(K * Mp * es);
   l.total = l.part + align256(q3_cdiv(M, kColRows) * N * 4);
   return l;
 }
@@ -661,12 +719,18 @@ int q3_transpose(const void* a, void* b, int64_t E, int64_t R, int64_t C, int dt
   Q3_REQUIRE(a && b, Q3_ERR_NULL);
   Q3_REQUIRE(E >= 0 && R >= 0 && C >= 0 && E < 65536, Q3_ERR_SHAPE);
   Q3_REQUIRE(dtype == Q3_BF16 || dtype == Q3_F32, Q3_ERR_DTYPE);
-  return transpose(a, b, E, R, C, dtype, static_cast<hipStream_t>(stream));
+  return transpose(a, b, E, R, C, R, dtype, static_cast<hipStream_t>(stream));
 }
 
 int64_t q3_matmul_backward_workspace_bytes(int64_t M, int64_t N, int64_t K, int dtype) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   return mm_bwd_layout(M, N, K, dtype).total;
+}
+
+int64_t q3_matmul_backward_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int dtype) {
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  return std::max(q3_matmul_workspace_bytes(M, K, N, dtype, 0),
+                  q3_matmul_workspace_bytes(N, K, padded_rows(M, dtype), dtype, 0));
 }
 
 int q3_matmul_backward(const void* x, const void* w, const void* dy, void* gx, void* gw, void* gb, int64_t M,
@@ -685,7 +749,7 @@ int q3_matmul_backward(const void* x, const void* w, const void* dy, void* gx, v
   if (gx) {  // gx (M, K) = dY (M, N) . W (N, K) = dY . (W^T)^T with W^T (K, N) as the GEMM's weight
     const int64_t need = q3_matmul_workspace_bytes(M, K, N, dtype, 0);
     Q3_REQUIRE(need <= 0 || (gemm_ws && gemm_ws_bytes >= need), Q3_ERR_WORKSPACE);
-    if ((rc = transpose(w, ws + l.wt, 1, N, K, dtype, st)) != Q3_OK) return rc;
+    if ((rc = transpose(w, ws + l.wt, 1, N, K, N, dtype, st)) != Q3_OK) return rc;
     if ((rc = q3_matmul(dy, ws + l.wt, nullptr, nullptr, gx, M, K, N, N, N, 0, K, dtype, gemm_ws, gemm_ws_bytes,
                         stream)) != Q3_OK)
       return rc;
@@ -693,9 +757,12 @@ int q3_matmul_backward(const void* x, const void* w, const void* dy, void* gx, v
   if (gw) {  // gw (N, K) = dY^T (N, M) . X (M, K) = dY^T . (X^T)^T with X^T (K, M) as the weight
     const int64_t need = q3_matmul_workspace_bytes(N, K, M, dtype, 0);
     Q3_REQUIRE(need <= 0 || (gemm_ws && gemm_ws_bytes >= need), Q3_ERR_WORKSPACE);
-    if ((rc = transpose(dy, ws + l.dyt, 1, M, N, dtype, st)) != Q3_OK) return rc;
-    if ((rc = transpose(x, ws + l.xt, 1, M, K, dtype, st)) != Q3_OK) return rc;
-    if ((rc = q3_matmul(ws + l.dyt, ws + l.xt, nullptr, nullptr, gw, N, K, M, M, M, 0, K, dtype, gemm_ws,
+    // A tiled GEMM whose workspace covers only the unpadded length runs unsplit; the GEMV (N <= 32) needs all of it.
+    int64_t Mp = padded_rows(M, dtype);
+    if (N <= 32 && gemm_ws_bytes < q3_matmul_workspace_bytes(N, K, Mp, dtype, 0)) Mp = M;
+    if ((rc = transpose(dy, ws + l.dyt, 1, M, N, Mp, dtype, st)) != Q3_OK) return rc;
+    if ((rc = transpose(x, ws + l.xt, 1, M, K, Mp, dtype, st)) != Q3_OK) return rc;
+    if ((rc = q3_matmul(ws + l.dyt, ws + l.xt, nullptr, nullptr, gw, N, K, Mp, Mp, Mp, 0, K, dtype, gemm_ws,
                         gemm_ws_bytes, stream)) != Q3_OK)
       return rc;
   }
@@ -709,8 +776,8 @@ int q3_matmul_backward(const void* x, const void* w, const void* dy, void* gx, v
 
 int64_t q3_batched_gemm_backward_workspace_bytes(int64_t E, int64_t M, int64_t N, int64_t K, int dtype) {
   if (E <= 0 || M <= 0 || N <= 0 || K <= 0) return 0;
-  const int64_t es = dtype == Q3_BF16 ? 2 : 4;
-  return align256(E * K * N * es) + align256(E * N * M * es) + align256(E * K * M * es);
+  const int64_t es = dtype == Q3_BF16 ? 2 : 4, Mp = padded_rows(M, dtype);
+  return align256(E * K * N * es) + align256(E * N * Mp * es) + align256(E * K * Mp * es);
 }
 
 int q3_batched_gemm_backward(const void* x, const void* w, const void* dy, void* gx, void* gw, int64_t E, int64_t M,
@@ -720,23 +787,23 @@ int q3_batched_gemm_backward(const void* x, const void* w, const void* dy, void*
   Q3_REQUIRE(E >= 0 && M >= 0 && N >= 0 && K >= 0 && E < 65536, Q3_ERR_SHAPE);
   Q3_REQUIRE(dtype == Q3_BF16 || dtype == Q3_F32, Q3_ERR_DTYPE);
   if (E == 0 || M == 0 || N == 0 || K == 0) return Q3_OK;
-  const int64_t es = dtype == Q3_BF16 ? 2 : 4;
+  const int64_t es = dtype == Q3_BF16 ? 2 : 4, Mp = padded_rows(M, dtype);
   Q3_REQUIRE(workspace && workspace_bytes >= q3_batched_gemm_backward_workspace_bytes(E, M, N, K, dtype),
              Q3_ERR_WORKSPACE);
   Q3_REQUIRE(q3_aligned(workspace, 256), Q3_ERR_ALIGN);
   char* wt = static_cast<char*>(workspace);
   char* dyt = wt + align256(E * K * N * es);
-  char* xt = dyt + align256(E * N * M * es);
+  char* xt = dyt + align256(E * N * Mp * es);
   hipStream_t st = static_cast<hipStream_t>(stream);
   int rc;
   if (gx) {  // gx[e] (M, K) = dY[e] (M, N) . W[e] (N, K)
-    if ((rc = transpose(w, wt, E, N, K, dtype, st)) != Q3_OK) return rc;
+    if ((rc = transpose(w, wt, E, N, K, N, dtype, st)) != Q3_OK) return rc;
     if ((rc = q3_batched_gemm(dy, wt, gx, E, M, K, N, dtype, stream)) != Q3_OK) return rc;
   }
   if (gw) {  // gw[e] (N, K) = dY[e]^T (N, M) . X[e] (M, K)
-    if ((rc = transpose(dy, dyt, E, M, N, dtype, st)) != Q3_OK) return rc;
-    if ((rc = transpose(x, xt, E, M, K, dtype, st)) != Q3_OK) return rc;
-    if ((rc = q3_batched_gemm(dyt, xt, gw, E, N, K, M, dtype, stream)) != Q3_OK) return rc;
+    if ((rc = transpose(dy, dyt, E, M, N, Mp, dtype, st)) != Q3_OK) return rc;
+    if ((rc = transpose(x, xt, E, M, K, Mp, dtype, st)) != Q3_OK) return rc;
+    if ((rc = q3_batched_gemm(dyt, xt, gw, E, N, K, Mp, dtype, stream)) != Q3_OK) return rc;
   }
   return Q3_OK;
 }

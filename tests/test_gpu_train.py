@@ -216,6 +216,29 @@ def test_matmul_backward_bf16(shape):
     twice_equal(lambda: run_grads(K.matmul, [x, w, b], dy)[1])
 
 
+@pytest.mark.parametrize("M,N,K_", [(33, 72, 64), (63, 64, 136), (65, 200, 72), (127, 24, 40), (1023, 264, 520),
+                                    (77, 61, 64)])
+def test_matmul_backward_odd_rows_bf16(M, N, K_):
+    """Token counts that are no multiple of 8 (the padded transposes), on both sides of the 64-row tiles, and an
+    output width that is none (the scalar transpose and SIMT GEMM)."""
+    x, w = rnd(M, K_, seed=44).bfloat16(), rnd(N, K_, seed=45, std=0.1).bfloat16()
+    b, dy = rnd(N, seed=46, std=0.1).bfloat16(), rnd(M, N, seed=47).bfloat16()
+    _, (gx, gw, gb) = run_grads(K.matmul, [x, w, b], dy)
+    _, (rx, rw, rb) = ref_grads(O.linear, [x, w, b], dy)
+    for a, r, n in ((gx, rx, "dx"), (gw, rw, "dw"), (gb, rb, "db")):
+        assert_grad_close(a, r, f"matmul {n} bf16 {(M, N, K_)}")
+
+
+@pytest.mark.parametrize("R,C", [(64, 64), (8, 200), (200, 8), (72, 136), (65, 64), (64, 65), (1, 7)])
+def test_transpose_is_exact(R, C):
+    """q3_transpose, whole 16-byte rows (the vector kernel) and not: bit-exact."""
+    from qwen3_5_vl_cuda_custom_amd import _lib
+    a = rnd(3, R, C, seed=95).bfloat16().to(DEV)
+    b = torch.empty(3, C, R, dtype=a.dtype, device=DEV)
+    _lib.call("q3_transpose", a.data_ptr(), b.data_ptr(), 3, R, C, _lib.dtype_code(a.dtype), _lib.stream())
+    assert torch.equal(b, a.transpose(1, 2))
+
+
 def test_matmul_residual_gradient_passes_through():
     x, w, r, dy = rnd(40, 64, seed=48), rnd(24, 64, seed=49), rnd(40, 24, seed=50), rnd(40, 24, seed=51)
     _, (gx, gw, gr) = run_grads(lambda a, c, d: K.matmul(a, c, residual=d), [x, w, r], dy)
