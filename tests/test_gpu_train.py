@@ -165,6 +165,47 @@ def test_layernorm_backward(rows, cols, dtype):
             assert_grad_close(a, r, f"layernorm {n} bf16")
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,cols", [(1, 8), (70, 128), (17, 136), (9, 520), (30, 1032), (5, 1152), (6, 2048),
+                                       (3, 2056), (700, 4096), (2, 4104), (3, 8192), (2, 8200), (40, 127)])
+def test_norm_backward_row_lengths(rows, cols, dtype):
+    """Every instance of the norm backward (a row in 16 lanes, a wave, a block; rows it leaves to the scalar kernel)
+    at both sides of its range, more rows than one pass of the grid, and both norms."""
+    x, dy = rnd(rows, cols, seed=26, dtype=dtype), rnd(rows, cols, seed=29, dtype=dtype)
+    w, b = (1 + 0.1 * rnd(cols, seed=27)).to(dtype), (0.1 * rnd(cols, seed=28)).to(dtype)
+    got = list(run_grads(lambda a, c: K.rmsnorm(a, c, 1e-6), [x, w], dy)[1])
+    got += run_grads(lambda a, c, d: K.layernorm(a, c, d, 1e-6), [x, w, b], dy)[1]
+    ref = list(ref_grads(lambda a, c: O.rmsnorm(a, c, 1e-6), [x, w], dy)[1])
+    ref += ref_grads(lambda a, c, d: O.layernorm(a, c, d, 1e-6), [x, w, b], dy)[1]
+    for a, r, n in zip(got, ref, ("rms dx", "rms dw", "ln dx", "ln dw", "ln db")):
+        if dtype == torch.float32:  # sums of up to 8200 (columns) or 700 (rows) fp32 terms of magnitude ~1
+            assert_close(a, r, atol=1e-4, what=n)
+        else:
+            assert_grad_close(a, r, f"{n} bf16 {rows}x{cols}")
+
+
+@pytest.mark.parametrize("N,V", [(3, 8), (5, 2048 * 4 + 24), (7, 1001), (2, 70000)])
+def test_cross_entropy_rows_and_masked_logits_bf16(N, V):
+    """Vector and scalar rows, a row shorter than a block, and logits masked with -inf (also a whole thread's share)."""
+    x = rnd(N, V, seed=96, std=3.0).bfloat16()
+    x[:, : V // 2] = float("-inf")
+    tg = torch.full((N,), V - 1)
+    if N > 2:
+        tg[1] = -100
+    with torch.enable_grad():
+        a = x.to(DEV).requires_grad_(True)
+        loss = K.cross_entropy(a, tg.to(DEV))
+        loss.backward()
+        r = x.double().requires_grad_(True)
+        want = F.cross_entropy(r, tg)
+        want.backward()
+    assert abs(float(loss) - float(want)) <= 1e-5 * abs(float(want))
+    assert torch.isfinite(a.grad).all()
+    # one bf16 rounding of each value, and fp32 rounding of probabilities up to 1
+    err = (a.grad.double().cpu() - r.grad).abs()
+    assert bool((err <= 2.0 ** -8 * r.grad.abs() + 2.0 ** -20).all())
+
+
 @pytest.mark.parametrize("rows,cols,dtype", [(8, 256, torch.float32), (4096, 128, torch.bfloat16)])
 def test_softmax_backward(rows, cols, dtype):
     x, dy = rnd(rows, cols, seed=30, dtype=dtype), rnd(rows, cols, seed=31, dtype=dtype)
