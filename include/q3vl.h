@@ -468,14 +468,19 @@ int q3_transpose(const void* a, void* b, int64_t E, int64_t R, int64_t C, int dt
  * needs_bias_grad) -> [gx, gw, gb] (csrc/matmul_op.cpp:13, .cu:151-233): for
  * y = x . w^T (+ b) with x (M, K), w (N, K), dy (M, N), all contiguous:
  * gx = dy . w (M, K), gw = dy^T . x (N, K), gb = sum over rows of dy (N); any of
- * the three may be null. The operands are transposed into `workspace`
- * (q3_matmul_backward_workspace_bytes) and multiplied by q3_matmul, which may
+ * the three may be null. bf16 operands with N and K multiples of 8, 16-byte
+ * aligned and below 2 GiB each are multiplied as they are; others are transposed
+ * into `workspace` first (q3_matmul_backward_workspace_bytes serves any
+ * operands, q3_matmul_backward_workspace_bytes_for is what the given ones need)
+ * and multiplied by q3_matmul, which may
  * use `gemm_ws` as q3_matmul's workspace (zero-filled before first use, as
  * there; size at least q3_matmul_workspace_bytes of both products;
- * q3_matmul_backward_gemm_workspace_bytes also covers the weight gradient's
- * product over the padded row count it runs at). */
+ * q3_matmul_backward_gemm_workspace_bytes also covers the split form of the
+ * products on untransposed operands and the padded row count of the others). */
 int64_t q3_matmul_backward_workspace_bytes(int64_t M, int64_t N, int64_t K, int dtype);
 int64_t q3_matmul_backward_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int dtype);
+int64_t q3_matmul_backward_workspace_bytes_for(const void* x, const void* w, const void* dy, int64_t M, int64_t N,
+                                               int64_t K, int dtype);
 int q3_matmul_backward(const void* x, const void* w, const void* dy, void* gx, void* gw, void* gb, int64_t M,
                        int64_t N, int64_t K, int dtype, void* workspace, int64_t workspace_bytes, void* gemm_ws,
                        int64_t gemm_ws_bytes, void* stream);

@@ -96,6 +96,7 @@ _SIGS: dict[str, tuple] = {
     "q3_transpose": (c_int, [_V, _V, _I, _I, _I, c_int, _V]),
     "q3_matmul_backward_workspace_bytes": (c_int64, [_I, _I, _I, c_int]),
     "q3_matmul_backward_gemm_workspace_bytes": (c_int64, [_I, _I, _I, c_int]),
+    "q3_matmul_backward_workspace_bytes_for": (c_int64, [_V, _V, _V, _I, _I, _I, c_int]),
     "q3_matmul_backward": (c_int, [_V, _V, _V, _V, _V, _V, _I, _I, _I, c_int, _V, _I, _V, _I, _V]),
     "q3_batched_gemm_backward_workspace_bytes": (c_int64, [_I, _I, _I, _I, c_int]),
     "q3_batched_gemm_backward": (c_int, [_V, _V, _V, _V, _V, _I, _I, _I, _I, c_int, _V, _I, _V]),

@@ -7,6 +7,7 @@
 //  * tiled   : bf16, M > 32     -> 32x32x16 MFMA over a ring of direct-to-LDS tiles
 //  * gemv    : bf16, M <= 32    -> weight-streaming stream-K kernel (gemv.hip)
 //  * generic : fp32, or bf16 whose rows are not 16-byte aligned -> SIMT fp32
+#include "gemm_bwd.h"
 #include "gemm_kernels.h"
 #include "gemv.h"
 
@@ -97,12 +98,13 @@ int launch_generic(const void* x, const void* w, const void* w2, const void* bia
 // =====================================================================
 // Tiled MFMA path.
 // =====================================================================
-template <int BM, int BN, int WM, int WN, int EPI, int NST, int BKT, int NSTW = NST, bool MF16 = false>
+template <int BM, int BN, int WM, int WN, int EPI, int NST, int BKT, int NSTW = NST, bool MF16 = false,
+          bool XT = false, bool WT = false>
 int launch_tiled_cfg(GemmParams p, int64_t batch, hipStream_t st) {
   constexpr int BN_OUT = (EPI == kEpiSwiGLU) ? BN / 2 : BN;
   const int64_t tiles = q3_cdiv(p.M, BM) * q3_cdiv(p.N, BN_OUT);
   p.group_m = 4;  // 4 along M: S=4096 gate/up 587 -> 582 us, o 112 -> 110, S=1024 layer 430.6 -> 425.4 (8 and 16: slower)
-  hipLaunchKernelGGL((gemm_bf16_dma_kernel<BM, BN, WM, WN, EPI, false, NST, BKT, NSTW, MF16>),
+  hipLaunchKernelGGL((gemm_bf16_dma_kernel<BM, BN, WM, WN, EPI, false, NST, BKT, NSTW, MF16, XT, WT>),
                      dim3((unsigned)tiles, 1, (unsigned)batch), dim3(WM * WN * 64), 0, st, p);
   Q3_LAUNCH_CHECK();
   return Q3_OK;
@@ -205,6 +207,9 @@ int launch_tiled(GemmParams p, int64_t batch, hipStream_t st) {
 // workspace's 16 KiB counter region, which they never touch.
 constexpr int64_t kSplitWsOffset = 16 << 10;
 
+// Columns per split: whole 64-wide stages, the last split the rest.
+int64_t split_k_len(int64_t K, int64_t s) { return q3_cdiv(q3_cdiv(K, s), 64) * 64; }
+
 int split_k_plan(int64_t M, int64_t N, int64_t K) {
   if (M <= kGemvMaxRows || K < 2048 || M >= (1 << 20) || N >= (1 << 20)) return 1;
   const int64_t tiles_a = q3_cdiv(M, 256) * q3_cdiv(N, 256);
@@ -213,9 +218,10 @@ int split_k_plan(int64_t M, int64_t N, int64_t K) {
   int best = 1;
   double t_best = t_c;
   for (int s = 2; s <= 8; s *= 2) {
-    if (tiles_a * s > 256 || K % (64 * s) != 0) continue;
+    const int64_t ks = split_k_len(K, s);
+    if (tiles_a * s > 256 || ks * (s - 1) >= K) continue;
     const double bytes = (double)s * M * N * 4 + (double)M * N * 4;  // planes, residual in, C out
-    const double t = 9.8 + 0.0243 * (double)(K / s) + 4.0 + bytes / 5e6 + 4.0;
+    const double t = 9.8 + 0.0243 * (double)ks + 4.0 + bytes / 5e6 + 4.0;
     if (t < t_best) {
       t_best = t;
       best = s;
@@ -277,22 +283,24 @@ __global__ __launch_bounds__(256) void split_k_reduce_kernel(const float* __rest
   }
 }
 
+template <bool XT = false, bool WT = false>
 int launch_split_k(const GemmParams& p0, int S, void* ws, hipStream_t st) {
   GemmParams p = p0;
   float* parts = reinterpret_cast<float*>(static_cast<char*>(ws) + kSplitWsOffset);
-  const int64_t ks = p0.K / S;
+  const int64_t ks = split_k_len(p0.K, S);
   p.C = reinterpret_cast<bf16*>(parts);
   p.K = (int)ks;
+  p.Ktot = p0.K;
   p.ldc = p0.N;
-  p.bsX = ks;
-  p.bsW = ks;
+  p.bsX = XT ? ks * p0.ldx : ks;
+  p.bsW = WT ? ks * p0.ldw : ks;
   p.bsC = (int64_t)p0.M * p0.N;
   p.bias = nullptr;
   p.R = nullptr;
   p.act = 0;
   p.seg.n = 1;
   p.seg.w[0] = p.W;
-  const int rc = launch_tiled_cfg<256, 256, 2, 4, kEpiStoreF32, 2, 64, 3, true>(p, S, st);
+  const int rc = launch_tiled_cfg<256, 256, 2, 4, kEpiStoreF32, 2, 64, 3, true, XT, WT>(p, S, st);
   if (rc != Q3_OK) return rc;
   const bool vec = p0.N % 8 == 0 && p0.ldc % 8 == 0 && q3_aligned(p0.C, 16) &&
                    (!p0.bias || q3_aligned(p0.bias, 16)) && (!p0.R || (q3_aligned(p0.R, 16) && p0.ldr % 8 == 0));
@@ -301,6 +309,23 @@ int launch_split_k(const GemmParams& p0, int S, void* ws, hipStream_t st) {
                      (int64_t)p0.M, (int64_t)p0.N, p0.bias, p0.R, p0.ldr, p0.C, p0.ldc, vec ? 1 : 0);
   Q3_LAUNCH_CHECK();
   return Q3_OK;
+}
+
+// Tiles of the products whose operands have the reduction as rows (XT / WT):
+// the 16x16x32 configurations of launch_tiled by the same estimate, without
+// the 256x192 tiles (24 chunks to a row split no instruction evenly); the
+// 128x128 ring always takes one block per CU.
+template <bool XT, bool WT>
+int launch_tiled_t(const GemmParams& p, int64_t batch, hipStream_t st) {
+  constexpr int kCUs = 256;
+  auto waves = [&](int64_t bm, int64_t bn) { return (double)q3_cdiv(q3_cdiv(p.M, bm) * q3_cdiv(p.N, bn) * batch, kCUs); };
+  const double cost_a = waves(256, 256) * 256.0 * 256.0;
+  const double cost_d = waves(128, 256) * 128.0 * 256.0 / 0.9;
+  const double cost_c = waves(128, 128) * 128.0 * 128.0 / 0.47;
+  if (cost_c < cost_a && cost_c < cost_d)
+    return launch_tiled_cfg<128, 128, 2, 4, kEpiStore, 4, 64, 5, true, XT, WT>(p, batch, st);
+  if (cost_d < cost_a) return launch_tiled_cfg<128, 256, 2, 4, kEpiStore, 2, 64, 4, true, XT, WT>(p, batch, st);
+  return launch_tiled_cfg<256, 256, 2, 4, kEpiStore, 2, 64, 3, true, XT, WT>(p, batch, st);
 }
 
 bool bf16_rows_ok(const void* base, int64_t ld, int64_t K) {
@@ -472,6 +497,64 @@ int rmsnorm_gemv_impl(const void* x, const void* norm_w, float eps, WeightSegmen
 }
 
 }  // namespace
+
+namespace q3 {
+
+// 16-byte loads of rows that are whole chunks, and 32-bit byte offsets.
+bool gemm_t_ok(const void* x, const void* w, int64_t M, int64_t N, int64_t K, bool xt) {
+  return M > 0 && N > 0 && K > 0 && (xt ? M : K) % 8 == 0 && N % 8 == 0 && q3_aligned(x, 16) && q3_aligned(w, 16) &&
+         (K + 64) * N * 2 < (1ll << 31) && ((xt ? K : M) + 256) * (xt ? M : K) * 2 < (1ll << 31);
+}
+
+int64_t gemm_t_workspace_bytes(int64_t M, int64_t N, int64_t K) { return split_k_workspace_bytes(M, N, K); }
+
+template <bool XT>
+static int gemm_t(const void* x, const void* w, void* y, int64_t M, int64_t N, int64_t K, void* ws, int64_t ws_bytes,
+                  hipStream_t st) {
+  GemmParams p{};
+  p.X = static_cast<const bf16*>(x);
+  p.W = static_cast<const bf16*>(w);
+  p.C = static_cast<bf16*>(y);
+  p.M = (int)M;
+  p.N = (int)N;
+  p.K = (int)K;
+  p.ldx = XT ? M : K;
+  p.ldw = N;
+  p.ldc = N;
+  const int S = split_k_plan(M, N, K);
+  if (S > 1 && ws != nullptr && q3_aligned(ws, 16) && ws_bytes >= split_k_workspace_bytes(M, N, K))
+    return launch_split_k<XT, true>(p, S, ws, st);
+  return launch_tiled_t<XT, true>(p, 1, st);
+}
+
+int gemm_nn(const void* x, const void* w, void* y, int64_t M, int64_t N, int64_t K, void* ws, int64_t ws_bytes,
+            hipStream_t st) {
+  return gemm_t<false>(x, w, y, M, N, K, ws, ws_bytes, st);
+}
+
+int gemm_tn(const void* x, const void* w, void* y, int64_t M, int64_t N, int64_t K, void* ws, int64_t ws_bytes,
+            hipStream_t st) {
+  return gemm_t<true>(x, w, y, M, N, K, ws, ws_bytes, st);
+}
+
+int gemm_tn_ranges(const void* x, const void* w, void* y, int64_t M, int64_t N, int64_t rows, const int* k_off,
+                   int64_t nz, hipStream_t st) {
+  GemmParams p{};
+  p.X = static_cast<const bf16*>(x);
+  p.W = static_cast<const bf16*>(w);
+  p.C = static_cast<bf16*>(y);
+  p.M = (int)M;
+  p.N = (int)N;
+  p.K = (int)rows;
+  p.ldx = M;
+  p.ldw = N;
+  p.ldc = N;
+  p.bsC = M * N;
+  p.k_off = k_off;
+  return launch_tiled_cfg<256, 256, 2, 4, kEpiStore, 2, 64, 3, true, true, true>(p, nz, st);
+}
+
+}  // namespace q3
 
 extern "C" {
 

@@ -64,6 +64,11 @@ struct GemmParams {
   const int* group_end;   // per expert: end row (exclusive) in the sorted order
   const int* n_tiles_total;  // device scalar: number of valid m-tiles
   int64_t expert_stride_w;   // elements between consecutive experts' weights
+  // Reduction ranges (z = blockIdx.z): with k_off (XT and WT kernels) problem z
+  // sums rows [k_off[z], k_off[z + 1]) of both operands; with Ktot > 0 split z
+  // sums min(K, Ktot - z K) of them (the last split may be shorter).
+  const int* k_off;
+  int Ktot;
   WeightSegments seg;        // dense (non-grouped, batch 1) store epilogue only
   int act;                   // kEpiStore: 1 = gelu_tanh of (acc + bias), before the residual
 };
@@ -435,6 +440,17 @@ __device__ __forceinline__ int dma_swz(int r) {
   else return (r & 7) ^ ((r >> 3) & 1);
 }
 
+// Swizzle of the stage rows of an operand with the reduction as rows (XT / WT
+// below): even, so that 32-byte column pairs of chunks stay together.
+__device__ __forceinline__ int tr_swz(int r) { return 2 * ((r & 3) | (((r >> 3) & 1) << 2)); }
+
+typedef short tr_short4 __attribute__((ext_vector_type(4)));
+typedef short tr_short8 __attribute__((ext_vector_type(8)));
+__device__ __forceinline__ tr_short4 lds_tr16(uint32_t byte) {
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+      (tr_short4 __attribute__((address_space(3)))*)(uintptr_t)byte);
+}
+
 // The tile GEMM with direct-to-LDS operand loads: stage kt's X and W tiles
 // (BKT-wide in K) go global -> LDS by buffer_load ... lds into a ring of NST
 // slots, issued NST - 1 stages ahead, so neither staging registers nor LDS
@@ -447,13 +463,27 @@ __device__ __forceinline__ int dma_swz(int r) {
 // before its last step's MFMAs (which overlap the first reads of the next
 // stage), so no wave starts a stage waiting on LDS.
 //
+// XT / WT (MF16 only): the operand is stored with the reduction as its rows,
+// X as (K, M) rows of ldx or W as (K, N) rows of ldw elements, as the GEMM
+// backward has them (dX = dY W: WT; dW = dY^T X: both). A stage of such an
+// operand is BKT rows of the tile's columns, and its fragments are read by
+// ds_read_b64_tr_b16, which hands each lane 4 consecutive rows of its column
+// (two per fragment, in the k order of the plain 16-byte reads), so no operand
+// is transposed in memory and the reduction length needs no alignment. Chunk c
+// of row r sits at slot c ^ tr_swz(r): the 8 rows that 32 lanes read 32 bytes
+// of fall into 8 distinct 32-byte bank groups.
+//
 // MF16: the same ring with v_mfma_f32_16x16x32_bf16 instead of 32x32x16. For
 // the same work it moves less data through the register file (operands 4 KB
 // + accumulators 4 KB per 32K flops, against 2 KB + 8 KB): on random data
 // under the power cap a pure MFMA loop sustains ~2.03 PFLOP/s with it against
 // ~1.80 with 32x32x16 (MI355X), and these GEMMs run power-limited.
-template <int BM, int BN, int WM, int WN, int EPI, bool GROUPED, int NST, int BKT, int NSTW = NST, bool MF16 = false>
+template <int BM, int BN, int WM, int WN, int EPI, bool GROUPED, int NST, int BKT, int NSTW = NST, bool MF16 = false,
+          bool XT = false, bool WT = false>
 __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_dma_kernel(const GemmParams p) {
+  static_assert(MF16 || (!XT && !WT), "operands with the reduction as rows: the 16x16x32 loop");
+  static_assert(!WT || EPI != kEpiSwiGLU, "no gate/up pairing of a transposed operand");
+  static_assert(!XT || !GROUPED, "grouped problems gather whole X rows");
   constexpr int NW = WM * WN;
   constexpr int WTM = BM / WM;
   constexpr int WTN = BN / WN;
@@ -490,9 +520,20 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_dma_kernel(const GemmPa
   TileCtx tc;
   if (!tile_ctx<BM, BN_OUT, EPI, GROUPED>(p, tc)) return;
   const int m_begin = tc.m_begin, rows_m = tc.rows_m, n0_out = tc.n0_out, n_lim = tc.n_lim;
-  const int K = p.K;
-  const int nk = (K + BKT - 1) / BKT;
+  int K = p.K;
+  if constexpr (MF16) {
+    if (p.Ktot > 0) K = min(K, p.Ktot - (int)blockIdx.z * K);
+  }
   const int64_t ldx = p.ldx, ldw = p.ldw;
+  if constexpr (XT && WT) {
+    if (p.k_off) {
+      const int k0 = __builtin_amdgcn_readfirstlane(p.k_off[blockIdx.z]);
+      K = __builtin_amdgcn_readfirstlane(p.k_off[blockIdx.z + 1]) - k0;
+      tc.X = uniform_ptr(tc.X + k0 * ldx);
+      tc.W = uniform_ptr(tc.W + k0 * ldw);
+    }
+  }
+  const int nk = (K + BKT - 1) / BKT;
 
   // Lane geometry of instruction i of this wave: tile row, and the global
   // chunk that lands in the lane's LDS slot. The swizzle depends on the row
@@ -501,11 +542,24 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_dma_kernel(const GemmPa
   static_assert((NW * RPI) % 16 == 0, "one swizzle chunk per lane");
   const int lrow = lane / CH, lslot = lane % CH;
   const int dc = lslot ^ dma_swz<BKT>(wave * RPI + lrow);
+  // Operands with the reduction as rows: an instruction fills 64 / (columns / 8)
+  // stage rows; the lane's stage row and column chunk of instruction 0 (the
+  // others' rows are a multiple of 16 further: the same chunk).
+  constexpr int CX = BM / 8, CW = BN / 8;
+  static_assert(!XT || (64 % CX == 0 && (NW * 64 / CX) % 16 == 0 && BM * BKT / 8 == DX * 64), "XT stage");
+  static_assert(!WT || (64 % CW == 0 && (NW * 64 / CW) % 16 == 0 && BN * BKT / 8 == DW * 64), "WT stage");
+  const int xkr = XT ? wave * (64 / CX) + lane / CX : 0, wkr = WT ? wave * (64 / CW) + lane / CW : 0;
+  const int xkc = XT ? (lane % CX) ^ tr_swz(xkr) : 0, wkc = WT ? (lane % CW) ^ tr_swz(wkr) : 0;
   uint32_t xoff[PX], woff[PW];
   const bf16* wsrc[PW];  // weight matrix of each W instruction (its rows share one segment) ...
   int wrows[PW];         // ... and its rows
 #pragma unroll
   for (int i = 0; i < PX; ++i) {
+    if constexpr (XT) {
+      xoff[i] = xkc * 8 < rows_m
+                    ? (uint32_t)(((int64_t)(xkr + NW * (64 / CX) * i) * ldx + m_begin + xkc * 8) * 2) : kOOB;
+      continue;
+    }
     const int r = (wave + NW * i) * RPI + lrow;
     if (r < rows_m) {
       const int lr = m_begin + r;
@@ -517,6 +571,13 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_dma_kernel(const GemmPa
   }
 #pragma unroll
   for (int i = 0; i < PW; ++i) {
+    if constexpr (WT) {
+      wsrc[i] = tc.W;
+      wrows[i] = K;
+      woff[i] = n0_out + wkc * 8 < n_lim
+                    ? (uint32_t)(((int64_t)(wkr + NW * (64 / CW) * i) * ldw + n0_out + wkc * 8) * 2) : kOOB;
+      continue;
+    }
     const int r = (wave + NW * i) * RPI + lrow;
     int n, rbase = 0, rlim;  // global row n; rows of the source matrix: [rbase, rbase + rlim)
     const bf16* wb;
@@ -548,29 +609,43 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_dma_kernel(const GemmPa
     woff[i] = (n - rbase < rlim) ? (uint32_t)((int64_t)(n - rbase) * ldw * 2) : kOOB;
   }
   const __amdgpu_buffer_rsrc_t rx =
+      XT ? make_rsrc(tc.X, (int64_t)K * ldx * 2) :
       make_rsrc(tc.X, p.gather ? (int64_t)p.M_src * ldx * 2 : (int64_t)(m_begin + rows_m) * ldx * 2);
   const uint32_t lbase = lds_addr(smem);
 
   // LDS byte address of stage kt's X / W slot.
   auto xslot = [&](int kt) { return lbase + (uint32_t)((kt % NST) * kStageX * 2); };
   auto wslot = [&](int kt) { return lbase + (uint32_t)((NST * kStageX + (kt % NSTW) * kStageW) * 2); };
-  auto issue_x = [&](int kt) {
+  // Byte offset of instruction i's chunk of stage kt (kOOB past the K range; rows of an XT / WT operand past K
+  // lie past the end of its resource, which loads zeros: a row's last chunk may reach into the next row, never past
+  // the last one, since rows are whole chunks).
+  auto xoff_of = [&](int kt, int i) -> uint32_t {
+    if constexpr (XT) {
+      const bool ok = xoff[i] != kOOB && kt * BKT + xkr + NW * (64 / CX) * i < K;
+      return ok ? xoff[i] + (uint32_t)kt * (uint32_t)(BKT * 2) * (uint32_t)ldx : kOOB;
+    }
     const int k = kt * BKT + dc * 8;
+    return (k < K && xoff[i] != kOOB) ? xoff[i] + (uint32_t)k * 2u : kOOB;
+  };
+  auto woff_of = [&](int kt, int i) -> uint32_t {
+    if constexpr (WT) {
+      const bool ok = woff[i] != kOOB && kt * BKT + wkr + NW * (64 / CW) * i < K;
+      return ok ? woff[i] + (uint32_t)kt * (uint32_t)(BKT * 2) * (uint32_t)ldw : kOOB;
+    }
+    const int k = kt * BKT + dc * 8;
+    return (k < K && woff[i] != kOOB) ? woff[i] + (uint32_t)k * 2u : kOOB;
+  };
+  auto issue_x = [&](int kt) {
     const uint32_t sb = xslot(kt);
 #pragma unroll
-    for (int i = 0; i < PX; ++i) {
-      const uint32_t off = (k < K && xoff[i] != kOOB) ? xoff[i] + (uint32_t)k * 2u : kOOB;
-      dma16(rx, off, sb + (uint32_t)((wave + NW * i) * 1024));
-    }
+    for (int i = 0; i < PX; ++i) dma16(rx, xoff_of(kt, i), sb + (uint32_t)((wave + NW * i) * 1024));
   };
   auto issue_w = [&](int kt) {
-    const int k = kt * BKT + dc * 8;
     const uint32_t sb = wslot(kt);
 #pragma unroll
-    for (int i = 0; i < PW; ++i) {
-      const uint32_t off = (k < K && woff[i] != kOOB) ? woff[i] + (uint32_t)k * 2u : kOOB;
-      dma16(make_rsrc(wsrc[i], (int64_t)wrows[i] * ldw * 2), off, sb + (uint32_t)((wave + NW * i) * 1024));
-    }
+    for (int i = 0; i < PW; ++i)
+      dma16(make_rsrc(wsrc[i], (int64_t)wrows[i] * ldw * 2), woff_of(kt, i),
+            sb + (uint32_t)((wave + NW * i) * 1024));
   };
   // The DMAs are issued in groups, one per stage: the group issued at the end
   // of stage j is X(j + NST) then W(j + NSTW) (each into the slot stage j has
@@ -607,12 +682,37 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_dma_kernel(const GemmPa
     bf16x8 fw[2][T16N], fx[T16M];
     const int l16 = lane & 15, q4 = lane >> 4;
     const int rn = wn * WTN, rm = wm * WTM;
+    // Transposed fragment reads: lane (q4, rr, qq) addresses row 32 ks + 8 q4 + rr (+ 4), columns 16 i + 4 qq of
+    // the wave's range; tr_swz depends on rr and q4 alone, and the wave's first chunk and 2 i share no bits, so
+    // tile i's address is tile 0's with bits flipped.
+    const int rr = (lane & 15) >> 2, qq = lane & 3, trow = 8 * q4 + rr;
+    auto tr0 = [&](int ld, int col0) {
+      return (uint32_t)((trow * ld + (((col0 >> 3) + (qq >> 1)) ^ tr_swz(trow)) * 8 + 4 * (qq & 1)) * 2);
+    };
+    const uint32_t xt0 = XT ? tr0(BM, rm) : 0, wt0 = WT ? tr0(BN, rn) : 0;
+    static_assert(!XT || WTM % 128 == 0 || (T16M <= 4 && WTM % 64 == 0), "XT: disjoint chunk bits");
+    static_assert(!WT || (T16N <= 4 && WTN % 64 == 0) || (T16N <= 2 && WTN % 32 == 0), "WT: disjoint chunk bits");
+    auto rd_tr = [&](uint32_t slot, uint32_t a0, int ld, int ks, int i) {
+      const uint32_t a = (slot + a0) ^ (uint32_t)(i << 5);
+      const tr_short4 lo = lds_tr16(a + (uint32_t)(32 * ks * ld * 2));
+      const tr_short4 hi = lds_tr16(a + (uint32_t)((32 * ks + 4) * ld * 2));
+      const tr_short8 v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      return __builtin_bit_cast(bf16x8, v);
+    };
     auto rd_w = [&](int buf, int kt, int ks, int i) {
+      if constexpr (WT) {
+        fw[buf][i] = rd_tr(wslot(kt), wt0, BN, ks, i);
+        return;
+      }
       const bf16* sw = smem + NST * kStageX + (kt % NSTW) * kStageW;
       const int r = rn + i * 16 + l16, c = ks * 4 + q4;
       fw[buf][i] = *reinterpret_cast<const bf16x8*>(sw + r * BKT + ((c ^ dma_swz<BKT>(r)) << 3));
     };
     auto rd_x = [&](int kt, int ks, int j) {
+      if constexpr (XT) {
+        fx[j] = rd_tr(xslot(kt), xt0, BM, ks, j);
+        return;
+      }
       const bf16* sx = smem + (kt % NST) * kStageX;
       const int r = rm + j * 16 + l16, c = ks * 4 + q4;
       fx[j] = *reinterpret_cast<const bf16x8*>(sx + r * BKT + ((c ^ dma_swz<BKT>(r)) << 3));
@@ -626,14 +726,10 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_dma_kernel(const GemmPa
       return in;
     };
     auto dma_x = [&](int kx_stage, int d) {
-      const int k = kx_stage * BKT + dc * 8;
-      const uint32_t off = (k < K && xoff[d] != kOOB) ? xoff[d] + (uint32_t)k * 2u : kOOB;
-      dma16(rx, off, xslot(kx_stage) + (uint32_t)((wave + NW * d) * 1024));
+      dma16(rx, xoff_of(kx_stage, d), xslot(kx_stage) + (uint32_t)((wave + NW * d) * 1024));
     };
     auto dma_w16 = [&](int kw, int i) {
-      const int k = kw * BKT + dc * 8;
-      const uint32_t off = (k < K && woff[i] != kOOB) ? woff[i] + (uint32_t)k * 2u : kOOB;
-      dma16(make_rsrc(wsrc[i], (int64_t)wrows[i] * ldw * 2), off, wslot(kw) + (uint32_t)((wave + NW * i) * 1024));
+      dma16(make_rsrc(wsrc[i], (int64_t)wrows[i] * ldw * 2), woff_of(kw, i), wslot(kw) + (uint32_t)((wave + NW * i) * 1024));
     };
 
 #pragma unroll

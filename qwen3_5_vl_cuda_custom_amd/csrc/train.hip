@@ -7,15 +7,16 @@
 //  * backward: sigmoid_mul, swiglu, gelu_tanh (elementwise); softmax (row);
 //    rmsnorm and layernorm (row pass for the input gradient, fixed-order
 //    reductions for the weight / bias gradients); cross_entropy; top-k (a
-//    scatter of the value gradients); matmul and the batched GEMM (operands
-//    transposed into a workspace, then the MFMA GEMM of gemm.hip, and the
-//    bias gradient as a fixed-order column sum).
+//    scatter of the value gradients); matmul (the MFMA GEMMs of gemm.hip on
+//    the operands as they are, or, like the batched GEMM, on operands
+//    transposed into a workspace; the bias gradient as a fixed-order column sum).
 //
 // Everything computes in fp32 and rounds once to the tensor dtype. No
 // reduction uses atomics: every sum runs in a fixed order, so results are
 // bitwise reproducible run to run.
 #include <type_traits>
 
+#include "gemm_bwd.h"
 #include "q3_common.h"
 
 namespace {
@@ -905,6 +906,17 @@ MmBwdLayout mm_bwd_layout(int64_t M, int64_t N, int64_t K, int dtype) {
   return l;
 }
 
+// The products on the operands as they are (no transposes): bf16 rows of whole
+// 16-byte pieces and byte offsets below 2 GiB (gemm_bwd.h). The 21 transposes
+// of a dense layer's backward at S=2048 took 311 us of its 3143, the three of
+// a 151936 x 4096 head's 641 of 4289.
+bool mm_bwd_direct_x(const void* w, const void* dy, int64_t M, int64_t N, int64_t K, int dtype) {
+  return dtype == Q3_BF16 && q3::gemm_t_ok(dy, w, M, K, N, false);
+}
+bool mm_bwd_direct_w(const void* x, const void* dy, int64_t M, int64_t N, int64_t K, int dtype) {
+  return dtype == Q3_BF16 && q3::gemm_t_ok(dy, x, N, K, M, true);
+}
+
 }  // namespace
 
 extern "C" {
@@ -1061,8 +1073,18 @@ int64_t q3_matmul_backward_workspace_bytes(int64_t M, int64_t N, int64_t K, int 
 
 int64_t q3_matmul_backward_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int dtype) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
-  return std::max(q3_matmul_workspace_bytes(M, K, N, dtype, 0),
-                  q3_matmul_workspace_bytes(N, K, padded_rows(M, dtype), dtype, 0));
+  int64_t need = std::max(q3_matmul_workspace_bytes(M, K, N, dtype, 0),
+                          q3_matmul_workspace_bytes(N, K, padded_rows(M, dtype), dtype, 0));
+  if (dtype == Q3_BF16)
+    need = std::max({need, q3::gemm_t_workspace_bytes(M, K, N), q3::gemm_t_workspace_bytes(N, K, M)});
+  return need;
+}
+
+int64_t q3_matmul_backward_workspace_bytes_for(const void* x, const void* w, const void* dy, int64_t M, int64_t N,
+                                               int64_t K, int dtype) {
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  const bool direct = mm_bwd_direct_x(w, dy, M, N, K, dtype) && mm_bwd_direct_w(x, dy, M, N, K, dtype);
+  return direct ? align256(colsum_parts(M) * N * 4) : mm_bwd_layout(M, N, K, dtype).total;
 }
 
 int q3_matmul_backward(const void* x, const void* w, const void* dy, void* gx, void* gw, void* gb, int64_t M,
@@ -1072,31 +1094,44 @@ int q3_matmul_backward(const void* x, const void* w, const void* dy, void* gx, v
   Q3_REQUIRE(M >= 0 && N >= 0 && K >= 0 && M < (1ll << 31) && N < (1ll << 31) && K < (1ll << 31), Q3_ERR_SHAPE);
   Q3_REQUIRE(dtype == Q3_BF16 || dtype == Q3_F32, Q3_ERR_DTYPE);
   if (M == 0 || N == 0 || K == 0) return Q3_OK;
-  const MmBwdLayout l = mm_bwd_layout(M, N, K, dtype);
+  const bool dir_x = mm_bwd_direct_x(w, dy, M, N, K, dtype), dir_w = mm_bwd_direct_w(x, dy, M, N, K, dtype);
+  MmBwdLayout l = mm_bwd_layout(M, N, K, dtype);
+  if (dir_x && dir_w) {  // no operand is transposed: the workspace holds the bias gradient's partial sums alone
+    l.part = 0;
+    l.total = align256(colsum_parts(M) * N * 4);
+  }
   Q3_REQUIRE(workspace && workspace_bytes >= l.total, Q3_ERR_WORKSPACE);
   Q3_REQUIRE(q3_aligned(workspace, 256), Q3_ERR_ALIGN);
   char* ws = static_cast<char*>(workspace);
   hipStream_t st = static_cast<hipStream_t>(stream);
   int rc;
-  if (gx) {  // gx (M, K) = dY (M, N) . W (N, K) = dY . (W^T)^T with W^T (K, N) as the GEMM's weight
-    const int64_t need = q3_matmul_workspace_bytes(M, K, N, dtype, 0);
-    Q3_REQUIRE(need <= 0 || (gemm_ws && gemm_ws_bytes >= need), Q3_ERR_WORKSPACE);
-    if ((rc = transpose(w, ws + l.wt, 1, N, K, N, dtype, st)) != Q3_OK) return rc;
-    if ((rc = q3_matmul(dy, ws + l.wt, nullptr, nullptr, gx, M, K, N, N, N, 0, K, dtype, gemm_ws, gemm_ws_bytes,
-                        stream)) != Q3_OK)
-      return rc;
+  if (gx) {  // gx (M, K) = dY (M, N) . W (N, K)
+    if (dir_x) {
+      if ((rc = q3::gemm_nn(dy, w, gx, M, K, N, gemm_ws, gemm_ws_bytes, st)) != Q3_OK) return rc;
+    } else {  // dY . (W^T)^T with W^T (K, N) as the GEMM's weight
+      const int64_t need = q3_matmul_workspace_bytes(M, K, N, dtype, 0);
+      Q3_REQUIRE(need <= 0 || (gemm_ws && gemm_ws_bytes >= need), Q3_ERR_WORKSPACE);
+      if ((rc = transpose(w, ws + l.wt, 1, N, K, N, dtype, st)) != Q3_OK) return rc;
+      if ((rc = q3_matmul(dy, ws + l.wt, nullptr, nullptr, gx, M, K, N, N, N, 0, K, dtype, gemm_ws, gemm_ws_bytes,
+                          stream)) != Q3_OK)
+        return rc;
+    }
   }
-  if (gw) {  // gw (N, K) = dY^T (N, M) . X (M, K) = dY^T . (X^T)^T with X^T (K, M) as the weight
-    const int64_t need = q3_matmul_workspace_bytes(N, K, M, dtype, 0);
-    Q3_REQUIRE(need <= 0 || (gemm_ws && gemm_ws_bytes >= need), Q3_ERR_WORKSPACE);
-    // A tiled GEMM whose workspace covers only the unpadded length runs unsplit; the GEMV (N <= 32) needs all of it.
-    int64_t Mp = padded_rows(M, dtype);
-    if (N <= 32 && gemm_ws_bytes < q3_matmul_workspace_bytes(N, K, Mp, dtype, 0)) Mp = M;
-    if ((rc = transpose(dy, ws + l.dyt, 1, M, N, Mp, dtype, st)) != Q3_OK) return rc;
-    if ((rc = transpose(x, ws + l.xt, 1, M, K, Mp, dtype, st)) != Q3_OK) return rc;
-    if ((rc = q3_matmul(ws + l.dyt, ws + l.xt, nullptr, nullptr, gw, N, K, Mp, Mp, Mp, 0, K, dtype, gemm_ws,
-                        gemm_ws_bytes, stream)) != Q3_OK)
-      return rc;
+  if (gw) {  // gw (N, K) = dY^T (N, M) . X (M, K)
+    if (dir_w) {
+      if ((rc = q3::gemm_tn(dy, x, gw, N, K, M, gemm_ws, gemm_ws_bytes, st)) != Q3_OK) return rc;
+    } else {  // dY^T . (X^T)^T with X^T (K, M) as the weight
+      const int64_t need = q3_matmul_workspace_bytes(N, K, M, dtype, 0);
+      Q3_REQUIRE(need <= 0 || (gemm_ws && gemm_ws_bytes >= need), Q3_ERR_WORKSPACE);
+      // A tiled GEMM whose workspace covers only the unpadded length runs unsplit; the GEMV (N <= 32) needs all of it.
+      int64_t Mp = padded_rows(M, dtype);
+      if (N <= 32 && gemm_ws_bytes < q3_matmul_workspace_bytes(N, K, Mp, dtype, 0)) Mp = M;
+      if ((rc = transpose(dy, ws + l.dyt, 1, M, N, Mp, dtype, st)) != Q3_OK) return rc;
+      if ((rc = transpose(x, ws + l.xt, 1, M, K, Mp, dtype, st)) != Q3_OK) return rc;
+      if ((rc = q3_matmul(ws + l.dyt, ws + l.xt, nullptr, nullptr, gw, N, K, Mp, Mp, Mp, 0, K, dtype, gemm_ws,
+                          gemm_ws_bytes, stream)) != Q3_OK)
+        return rc;
+    }
   }
   if (gb) {  // gb (N) = sum over the M rows of dY, in row order
     float* part = reinterpret_cast<float*>(ws + l.part);

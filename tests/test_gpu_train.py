@@ -270,6 +270,36 @@ def test_matmul_backward_odd_rows_bf16(M, N, K_):
         assert_grad_close(a, r, f"matmul {n} bf16 {(M, N, K_)}")
 
 
+@pytest.mark.parametrize("M,N,K_", [(1, 8, 8), (63, 136, 264), (64, 264, 136), (65, 520, 248), (129, 1032, 776),
+                                    (300, 4096, 1160), (40, 8192, 512), (1000, 512, 2056), (33, 40, 16456)])
+def test_matmul_backward_untransposed_against_transposed(M, N, K_):
+    """dX and dW on the operands as they are (tile edges in every dimension, the three tile shapes, splits over K with
+    a shorter last split) against q3_matmul on transposed copies, which sums each element's products in fp32 too: the
+    two may differ by one bf16 rounding of the element (2^-7) and the fp32 sums' order (2^-16 of the largest)."""
+    x, w, dy = (rnd(M, K_, seed=44).bfloat16().to(DEV), rnd(N, K_, seed=45, std=0.1).bfloat16().to(DEV),
+                rnd(M, N, seed=47).bfloat16().to(DEV))
+    _, (gx, gw) = run_grads(K.matmul, [x, w], dy)
+    pad = (-M) % 8
+    zeros = lambda t: torch.cat([t, torch.zeros(pad, t.shape[1], dtype=t.dtype, device=t.device)])  # noqa: E731
+    rx = K.matmul(dy, w.t().contiguous())
+    rw = K.matmul(zeros(dy).t().contiguous(), zeros(x).t().contiguous())
+    for a, b, n in ((gx, rx, "dx"), (gw, rw, "dw")):
+        a, b = a.float(), b.float()
+        over = float(((a - b).abs() - 2.0 ** -7 * b.abs() - 2.0 ** -16 * b.abs().max()).max())
+        assert over <= 0, f"{n} {(M, N, K_)}: {over:.3e} over"
+
+
+@pytest.mark.parametrize("M,N,K_", [(1024, 4096, 12352), (512, 2048, 8256)])
+def test_matmul_split_with_shorter_last_split(M, N, K_):
+    """A K that no split count divides into whole 64-wide stages: the last split is shorter. Outputs reach |11|, where
+    half a bf16 step is 0.031: the bound is one rounding of each value (2^-8 of it) plus the fp32 sums' order (2^-16 of
+    the largest), not the fixed 0.02 of unit-sized outputs."""
+    x, w = rnd(M, K_, seed=44).bfloat16(), rnd(N, K_, seed=45, std=0.02).bfloat16()
+    got, ref = K.matmul(x.to(DEV), w.to(DEV)).float().cpu(), O.linear(x.float(), w.float())
+    over = float(((got - ref).abs() - 2.0 ** -8 * ref.abs() - 2.0 ** -16 * ref.abs().max()).max())
+    assert over <= 0, f"split {M} {N} {K_}: {over:.3e} over"
+
+
 @pytest.mark.parametrize("R,C", [(64, 64), (8, 200), (200, 8), (72, 136), (65, 64), (64, 65), (1, 7)])
 def test_transpose_is_exact(R, C):
     """q3_transpose, whole 16-byte rows (the vector kernel) and not: bit-exact."""
