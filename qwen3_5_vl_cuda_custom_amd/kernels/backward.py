@@ -365,6 +365,46 @@ class TopKFunction(torch.autograd.Function):
         return gx, None
 
 
+class MoEExpertsFunction(torch.autograd.Function):
+    """The routed experts' SwiGLU MLPs and their combine, differentiable in the tokens, both expert weights and the
+    routing weights (reference modules/moe.py:70-83, there through autograd over a loop of the experts)."""
+
+    @staticmethod
+    def forward(ctx, x, gate_up, down, top_idx, top_w):
+        x, gate_up, down, top_w = _c(x), _c(gate_up), _c(down), _c(top_w)
+        T, H = x.shape
+        E, I, k = gate_up.shape[0], down.shape[2], top_idx.shape[1]
+        lib = _lib.lib()
+        state, nstate = _lib.workspace(lib.q3_moe_train_state_bytes(T, H, I, E, k), x.device)
+        ws, nws = _lib.workspace(lib.q3_moe_train_workspace_bytes(T, H, I, E, k, 0), x.device)
+        out = torch.empty_like(x)
+        _lib.call("q3_moe_train_forward", x.data_ptr(), gate_up.data_ptr(), down.data_ptr(), _c(top_idx).data_ptr(),
+                  top_w.data_ptr(), out.data_ptr(), T, H, I, E, k, _lib.ptr(state), nstate, _lib.ptr(ws), nws,
+                  _lib.stream())
+        ctx.save_for_backward(x, gate_up, down, state)
+        ctx.k = k
+        return out
+
+    @staticmethod
+    def backward(ctx, dy):
+        x, gate_up, down, state = ctx.saved_tensors
+        T, H = x.shape
+        E, I, k = gate_up.shape[0], down.shape[2], ctx.k
+        need = ctx.needs_input_grad
+        gx = torch.empty_like(x) if need[0] else None
+        ggu = torch.empty_like(gate_up) if need[1] else None
+        gdn = torch.empty_like(down) if need[2] else None
+        gw = torch.empty((T, k), dtype=x.dtype, device=x.device) if need[4] else None
+        dyc = _c(dy).to(x.dtype)
+        if dyc.data_ptr() % 16:
+            dyc = dyc.clone()
+        ws, nws = _lib.workspace(_lib.lib().q3_moe_train_workspace_bytes(T, H, I, E, k, 1), x.device)
+        _lib.call("q3_moe_train_backward", x.data_ptr(), gate_up.data_ptr(), down.data_ptr(), dyc.data_ptr(),
+                  _lib.ptr(gx), _lib.ptr(ggu), _lib.ptr(gdn), _lib.ptr(gw), T, H, I, E, k, state.data_ptr(),
+                  state.numel(), _lib.ptr(ws), nws, _lib.stream())
+        return gx, ggu, gdn, None, gw
+
+
 class IndexAddFunction(torch.autograd.Function):
     """Reference: kernels/moe_routing.py:72-100: under autograd the op returns a new tensor
     (target + the scattered sources); d target = dy, d source = dy[index]."""

@@ -6,7 +6,7 @@ import torch
 
 from .. import _lib
 from ._common import check, mfma_operand, note_slow_path
-from .backward import BatchedGemmFunction, IndexAddFunction, TopKFunction, needs_grad
+from .backward import MoEExpertsFunction, BatchedGemmFunction, IndexAddFunction, TopKFunction, needs_grad
 
 
 def cuda_topk(x: torch.Tensor, k: int) -> tuple[torch.Tensor, torch.Tensor]:
@@ -163,6 +163,23 @@ def moe_experts(x: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, top_
               top_idx.contiguous().data_ptr(), top_w.contiguous().data_ptr(), _lib.ptr(r), out.data_ptr(), T, H, I,
               E, k, _lib.ptr(ws), nws, _lib.stream())
     return out
+
+
+def moe_experts_train(x: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, top_idx: torch.Tensor,
+                      top_w: torch.Tensor) -> torch.Tensor | None:
+    """moe_experts with a backward (x, gate_up, down and top_w), every expert in a few grouped launches; None where it
+    does not cover the operands (fp32, widths that are no multiple of 8, unaligned views, 2 GiB and more): the caller
+    then runs the experts one by one on the single ops. top_idx (T, k), distinct experts in [0, E) per token."""
+    ts = (x, gate_up, down, top_w)
+    T, H = x.shape
+    E, I2, _ = gate_up.shape
+    k = top_idx.shape[1]
+    if (not all(t.is_cuda and t.dtype == torch.bfloat16 for t in ts) or gate_up.shape[2] != H or I2 % 2
+            or tuple(down.shape) != (E, H, I2 // 2) or tuple(top_w.shape) != (T, k)
+            or any(t.data_ptr() % 16 for t in ts[:3])
+            or _lib.lib().q3_moe_train_state_bytes(T, H, I2 // 2, E, k) == 0):
+        return None
+    return MoEExpertsFunction.apply(x, gate_up, down, top_idx.to(torch.int32), top_w)
 
 
 def moe_permute(top_idx: torch.Tensor, top_w: torch.Tensor, num_experts: int):

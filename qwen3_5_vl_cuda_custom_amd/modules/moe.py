@@ -4,7 +4,7 @@ from __future__ import annotations
 import torch
 from torch import nn
 
-from ..kernels import (cuda_index_add, cuda_topk, matmul, moe_experts, moe_route, moe_router, residual_add, softmax,
+from ..kernels import (cuda_index_add, cuda_topk, matmul, moe_experts, moe_experts_train, moe_route, moe_router, residual_add, softmax,
                        swiglu)
 from ..kernels.backward import needs_grad
 
@@ -78,9 +78,9 @@ class CudaSparseMoE(nn.Module):
 
     def _forward_autograd(self, x: torch.Tensor, residual: torch.Tensor | None):
         """Training: the reference's forward (modules/moe.py:54-85) on the differentiable ops: router
-        GEMM, softmax of the fp32 logits, top-k, renormalise and cast, then per expert its tokens'
-        gate_up GEMM, swiglu, down GEMM, the routing-weight product and the autograd form of
-        index_add (a new tensor per expert)."""
+        GEMM, softmax of the fp32 logits, top-k, renormalise and cast, then the experts: in bf16 all
+        at once (moe_experts_train), else per expert its tokens' gate_up GEMM, swiglu, down GEMM, the
+        routing-weight product and the autograd form of index_add (a new tensor per expert)."""
         B, S, H = x.shape
         x_flat = x.reshape(-1, H)
         logits = matmul(x_flat, self.gate_weight)
@@ -88,6 +88,14 @@ class CudaSparseMoE(nn.Module):
         if self.norm_topk_prob:
             vals = vals / vals.sum(dim=-1, keepdim=True)
         vals = vals.to(x.dtype)
+        final = moe_experts_train(x_flat, self.gate_up_proj, self.down_proj, idx, vals)
+        if final is None:
+            final = self._experts_one_by_one(x_flat, idx, vals)
+        if residual is not None:
+            final = residual_add(final, residual.reshape(-1, H))
+        return final.view(B, S, H), logits
+
+    def _experts_one_by_one(self, x_flat: torch.Tensor, idx: torch.Tensor, vals: torch.Tensor) -> torch.Tensor:
         final = torch.zeros_like(x_flat)
         I = self.moe_intermediate_size
         for e in range(self.num_experts):
@@ -96,7 +104,5 @@ class CudaSparseMoE(nn.Module):
                 continue
             gu = matmul(x_flat[token_idx], self.gate_up_proj[e])
             eo = matmul(swiglu(gu[:, :I], gu[:, I:]), self.down_proj[e])
-            final = cuda_index_add(final, (eo * vals[token_idx, slot_idx, None]).to(x.dtype), token_idx)
-        if residual is not None:
-            final = residual_add(final, residual.reshape(-1, H))
-        return final.view(B, S, H), logits
+            final = cuda_index_add(final, (eo * vals[token_idx, slot_idx, None]).to(x_flat.dtype), token_idx)
+        return final

@@ -532,6 +532,55 @@ def test_moe_layer_trains_like_the_oracle():
     _check_grads(got, ref, "moe layer", torch.float32)
 
 
+@pytest.mark.parametrize("T,H,I,E,k", [(1, 64, 24, 4, 1), (64, 128, 48, 8, 2), (300, 264, 136, 16, 4),
+                                       (600, 256, 128, 3, 2), (520, 512, 192, 128, 8)])
+def test_moe_block_trains_in_bf16_like_the_oracle(T, H, I, E, k):
+    """The grouped bf16 training path (experts with no rows, a few, and more than one 256-row tile) against the fp32
+    oracle on the same routing: the block's ~6 bf16 intermediates each round once (the bounds of a layer)."""
+    from oracle import layers as L
+    from qwen3_5_vl_cuda_custom_amd.modules import CudaSparseMoE
+    moe = CudaSparseMoE(hidden_size=H, moe_intermediate_size=I, num_experts=E, top_k=k).to(DEV).bfloat16()
+    g = torch.Generator(device=DEV).manual_seed(9)
+    with torch.no_grad():
+        for p in moe.parameters():
+            p.normal_(0, 0.1, generator=g)
+    x, dy = rnd(1, T, H, seed=91).bfloat16(), rnd(1, T, H, seed=92).bfloat16()
+    # the oracle routes on fp32 logits, the block on bf16 ones: keep the tokens whose k-th and next logit lie further
+    # apart than the bf16 rounding of both (2^-8 of each)
+    with torch.no_grad():
+        ref = (x.float().view(T, H) @ moe.gate_weight.float().cpu().t()).sort(-1, descending=True).values
+        same = (ref[:, k - 1] - ref[:, k] > 2.0 ** -7 * ref.abs().amax(-1)) if k < E else torch.ones(T, dtype=bool)
+        same[0] = True
+    x, dy = x[:, same], dy[:, same]
+    got = _module_grads(moe, lambda m, t: m(t)[0], x, dy)
+    ref = _oracle_grads(lambda t, p: L.sparse_moe(t, p, top_k=k)[0], dict(moe.named_parameters()), x, dy)
+    _check_grads(got, ref, f"moe bf16 {(T, H, I, E, k)}", torch.bfloat16)
+    moe.requires_grad_(False)
+    fwd = moe(x.to(DEV))[0].float().cpu()  # the inference path on the same routing
+    assert_grad_close(got[0], fwd, "train forward vs inference", max_rel=2e-2, mean_rel=5e-3)
+
+
+def test_moe_training_gradients_are_reproducible_and_partial():
+    """Twice the same bits, and the same bits with some gradients left out (a frozen weight, no input gradient)."""
+    from qwen3_5_vl_cuda_custom_amd.kernels.moe_routing import moe_experts_train
+    T, H, I, E, k = 200, 128, 64, 8, 2
+    x, gu, dn = (rnd(*s, seed=i, std=0.1).bfloat16().to(DEV) for i, s in
+                 enumerate([(T, H), (E, 2 * I, H), (E, H, I)]))
+    idx = torch.stack([torch.randperm(E, generator=torch.Generator().manual_seed(t))[:k] for t in range(T)]).to(DEV)
+    w, dy = torch.rand(T, k, device=DEV).bfloat16(), rnd(T, H, seed=5).bfloat16().to(DEV)
+
+    def grads(which):
+        ts = [t.clone().requires_grad_(i in which) for i, t in enumerate((x, gu, dn, w))]
+        with torch.enable_grad():
+            moe_experts_train(ts[0], ts[1], ts[2], idx, ts[3]).backward(dy)
+        return [t.grad for t in ts]
+
+    full = grads({0, 1, 2, 3})
+    for which in ({0, 1, 2, 3}, {0}, {1}, {2}, {3}, {0, 3}):
+        for i, (a, b) in enumerate(zip(grads(which), full)):
+            assert torch.equal(a, b) if i in which else a is None
+
+
 def test_vision_block_trains_like_the_oracle():
     from oracle import layers as L
     from qwen3_5_vl_cuda_custom_amd.modules import CudaVisionBlock
