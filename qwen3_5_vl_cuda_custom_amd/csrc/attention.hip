@@ -1200,54 +1200,140 @@ __global__ __launch_bounds__(512) void flash_fwd_pipe_kernel(const AttnParams p)
   }
 }
 
-template <typename T>
-__global__ __launch_bounds__(128) void flash_generic_kernel(const AttnParams p, int D, const int* kv_lens) {
-  const int64_t row = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  const int64_t total = (int64_t)p.B * p.Hq * p.Sq;
-  if (row >= total) return;
-  const int i = (int)(row % p.Sq);
-  const int hq = (int)((row / p.Sq) % p.Hq);
-  const int b = (int)(row / ((int64_t)p.Sq * p.Hq));
+// Any type, strides and head dim up to 256 in fp32: fp32 tensors, other head
+// dims, unaligned views; prefill (also packed or into a cache) and decode over
+// kv_lens. A block takes 16 queries of one head, 16 lanes per query: K and V
+// tiles of 32 keys go to LDS as fp32, lane kl of a query forms the scores of
+// keys kl and kl + 16 (whole dot products, 16-byte LDS reads; rows DMAX + 4
+// apart so 16 consecutive rows are conflict-free), the softmax is a 16-lane
+// exchange, and each lane sums dims 4 kl + 64 i .. + 3 of P V. One thread per
+// query with its row in scratch took 1741 us for 4 x 128 queries of 64 dims,
+// causal; this takes 23 us.
+template <typename T, int DMAX>
+__global__ __launch_bounds__(256) void flash_generic_kernel(const AttnParams p, int D, const int* kv_lens) {
+  constexpr int kQB = 16, kKB = 32, LD = DMAX + 4, NV = DMAX / 64 > 0 ? DMAX / 64 : 1;
+  __shared__ __attribute__((aligned(16))) float s_q[kQB * LD], s_k[kKB * LD], s_v[kKB * LD];
+  __shared__ float s_p[kQB][kKB + 1];
+  const int tid = threadIdx.x, qi = tid >> 4, kl = tid & 15;
+  const int n_qt = (p.Sq + kQB - 1) / kQB;
+  const int qt = p.causal ? n_qt - 1 - (int)(blockIdx.x % n_qt) : (int)(blockIdx.x % n_qt);  // heaviest first
+  const int bh = blockIdx.x / n_qt;
+  const int hq = bh % p.Hq, b = bh / p.Hq;
   const int kvh = hq / p.groups;
   int64_t qb_off = (int64_t)b * p.qb, kb_off = (int64_t)b * p.kb, vb_off = (int64_t)b * p.vb,
           ob_off = (int64_t)b * p.ob;
-  int Sk = p.Sk;
+  int Sq = p.Sq, Sk = p.Sk;
   if (p.cu_seqlens) {  // packed sequences: row i of sequence b is packed row cu_seqlens[b] + i
     const int row0 = p.cu_seqlens[b];
-    Sk = p.cu_seqlens[b + 1] - row0;
-    if (i >= Sk) return;
+    Sq = Sk = p.cu_seqlens[b + 1] - row0;
     qb_off = (int64_t)row0 * p.qs;
     kb_off = (int64_t)row0 * p.ks;
     vb_off = (int64_t)row0 * p.vs;
     ob_off = (int64_t)row0 * p.os;
   }
-  const T* q = reinterpret_cast<const T*>(p.q) + qb_off + (int64_t)hq * p.qh + (int64_t)i * p.qs;
+  const int q0 = qt * kQB;
+  if (q0 >= Sq) return;  // uniform over the block
+  const int i = q0 + qi;
+  const T* qb = reinterpret_cast<const T*>(p.q) + qb_off + (int64_t)hq * p.qh;
   const T* kb = reinterpret_cast<const T*>(p.k) + kb_off + (int64_t)kvh * p.kh;
   const T* vb = reinterpret_cast<const T*>(p.v) + vb_off + (int64_t)kvh * p.vh;
   const int off = p.q_off ? max(p.q_off[b], 0) : 0;
-  int nk = kv_lens ? min(kv_lens[b] + p.len_add, Sk) : (p.q_off ? min(Sk, off + p.Sq) : Sk);
-  if (p.causal) nk = min(nk, i + off + 1);
-  float acc[256];
-  for (int d = 0; d < D; ++d) acc[d] = 0.f;
-  float m = -INFINITY, l = 0.f;
+  const int nk = kv_lens ? min(kv_lens[b] + p.len_add, Sk) : (p.q_off ? min(Sk, off + p.Sq) : Sk);
+  const int nki = p.causal ? min(nk, i + off + 1) : nk;                              // this query's keys
+  const int nkb = p.causal ? min(nk, min(q0 + kQB, Sq) + off) : nk;                  // the block's
+  const int D4 = (D + 3) / 4;
   const float scale = p.scale_log2 / kLog2e;
-  for (int j = 0; j < nk; ++j) {
-    const T* kr = kb + (int64_t)j * p.ks;
-    float s = 0.f;
-    for (int d = 0; d < D; ++d) s += to_f<T>(q[d]) * to_f<T>(kr[d]);
-    s *= scale;
-    const float mn = fmaxf(m, s);
-    const float a = expf(m - mn);
-    const float e = expf(s - mn);
-    l = l * a + e;
-    const T* vr = vb + (int64_t)j * p.vs;
-    for (int d = 0; d < D; ++d) acc[d] = acc[d] * a + e * to_f<T>(vr[d]);
+  for (int e = kl; e < D4 * 4; e += 16) s_q[qi * LD + e] = i < Sq && e < D ? to_f<T>(qb[(int64_t)i * p.qs + e]) : 0.f;
+  floatx4 acc[NV];
+#pragma unroll
+  for (int n = 0; n < NV; ++n) acc[n] = floatx4{0.f, 0.f, 0.f, 0.f};
+  float m = -INFINITY, l = 0.f;
+  const int lr = tid >> 3, lc = tid & 7;  // K / V loads: row of the tile, first element
+  for (int j0 = 0; j0 < nkb; j0 += kKB) {
+    __syncthreads();  // the previous tile's readers are done
+    {
+      const int j = j0 + lr;
+      const T* kr = kb + (int64_t)j * p.ks;
+      const T* vr = vb + (int64_t)j * p.vs;
+#pragma unroll 4
+      for (int e = lc; e < D4 * 4; e += 8) {
+        const bool ok = j < nkb && e < D;
+        s_k[lr * LD + e] = ok ? to_f<T>(kr[e]) : 0.f;
+        s_v[lr * LD + e] = ok ? to_f<T>(vr[e]) : 0.f;
+      }
+    }
+    __syncthreads();
+    float s0 = 0.f, s1 = 0.f;
+#pragma unroll 4
+    for (int d = 0; d < D4; ++d) {
+      const floatx4 q = *reinterpret_cast<const floatx4*>(s_q + qi * LD + 4 * d);
+      const floatx4 a = *reinterpret_cast<const floatx4*>(s_k + kl * LD + 4 * d);
+      const floatx4 c = *reinterpret_cast<const floatx4*>(s_k + (kl + 16) * LD + 4 * d);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        s0 = fmaf(q[e], a[e], s0);
+        s1 = fmaf(q[e], c[e], s1);
+      }
+    }
+    s0 = j0 + kl < nki ? s0 * scale : -INFINITY;
+    s1 = j0 + kl + 16 < nki ? s1 * scale : -INFINITY;
+    const float mn = fmaxf(m, group_max<16>(fmaxf(s0, s1)));
+    // nothing but masked keys so far: the sums stay empty
+    const float alpha = mn == -INFINITY ? 1.f : expf(m - mn);
+    const float e0 = mn == -INFINITY && s0 == -INFINITY ? 0.f : expf(s0 - mn);
+    const float e1 = mn == -INFINITY && s1 == -INFINITY ? 0.f : expf(s1 - mn);
+    l = l * alpha + group_sum<16>(e0 + e1);
     m = mn;
+    s_p[qi][kl] = e0;
+    s_p[qi][kl + 16] = e1;
+    __syncthreads();
+#pragma unroll
+    for (int n = 0; n < NV; ++n) acc[n] *= alpha;
+    const int jn = min(kKB, nkb - j0);
+    for (int j = 0; j < jn; ++j) {
+      const float pr = s_p[qi][j];
+#pragma unroll
+      for (int n = 0; n < NV; ++n)
+        if (4 * kl + 64 * n < D4 * 4) {
+          const floatx4 v = *reinterpret_cast<const floatx4*>(s_v + j * LD + 4 * kl + 64 * n);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[n][e] = fmaf(pr, v[e], acc[n][e]);
+        }
+    }
   }
+  if (i >= Sq) return;
   T* o = reinterpret_cast<T*>(p.o) + ob_off + (int64_t)hq * p.oh + (int64_t)i * p.os;
   const float inv = l > 0.f ? 1.0f / l : 0.f;
-  for (int d = 0; d < D; ++d) o[d] = from_f<T>(acc[d] * inv);
-  if (p.lse) p.lse[((int64_t)b * p.Hq + hq) * p.Sq + i] = m + logf(l);
+#pragma unroll
+  for (int n = 0; n < NV; ++n)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int d = 4 * kl + 64 * n + e;
+      if (d < D) o[d] = from_f<T>(acc[n][e] * inv);
+    }
+  if (p.lse && kl == 0) p.lse[((int64_t)b * p.Hq + hq) * p.Sq + i] = m + logf(l);
+}
+
+template <typename T>
+int launch_generic_t(const AttnParams& p, int D, const int* kv_lens, hipStream_t st) {
+  const int64_t blocks = q3_cdiv(p.Sq, 16) * p.B * p.Hq;
+  Q3_REQUIRE(blocks < (1ll << 31), Q3_ERR_UNSUPPORTED);
+  if (blocks == 0) return Q3_OK;
+  const dim3 grid((unsigned)blocks);
+  if (D <= 64)
+    hipLaunchKernelGGL((flash_generic_kernel<T, 64>), grid, dim3(256), 0, st, p, D, kv_lens);
+  else if (D <= 128)
+    hipLaunchKernelGGL((flash_generic_kernel<T, 128>), grid, dim3(256), 0, st, p, D, kv_lens);
+  else
+    hipLaunchKernelGGL((flash_generic_kernel<T, 256>), grid, dim3(256), 0, st, p, D, kv_lens);
+  Q3_LAUNCH_CHECK();
+  return Q3_OK;
+}
+
+int launch_generic(const AttnParams& p, int D, const int* kv_lens, int dtype, hipStream_t st) {
+  if (dtype == Q3_F32) return launch_generic_t<float>(p, D, kv_lens, st);
+  if (dtype == Q3_BF16) return launch_generic_t<bf16>(p, D, kv_lens, st);
+  return Q3_ERR_DTYPE;
 }
 
 bool mfma_head_dim(int64_t D) { return D == 64 || D == 72 || D == 80 || D == 96 || D == 128; }
@@ -1413,16 +1499,7 @@ int fwd_impl(const void* q, const void* k, const void* v, void* o, float* lse, i
         rc = pipe ? launch_fwd_pipe<128>(p, st) : launch_fwd<128>(p, st);
     }
   } else {
-    const int64_t rows = B * Hq * Sq;
-    if (dtype == Q3_F32)
-      hipLaunchKernelGGL(flash_generic_kernel<float>, dim3((unsigned)q3_cdiv(rows, 128)), dim3(128), 0, st, p,
-                         (int)D, nullptr);
-    else if (dtype == Q3_BF16)
-      hipLaunchKernelGGL(flash_generic_kernel<bf16>, dim3((unsigned)q3_cdiv(rows, 128)), dim3(128), 0, st, p,
-                         (int)D, nullptr);
-    else
-      return Q3_ERR_DTYPE;
-    Q3_LAUNCH_CHECK();
+    rc = launch_generic(p, (int)D, nullptr, dtype, st);
   }
   if (rc != Q3_OK) return rc;
   if (lens_add) {
@@ -1642,16 +1719,8 @@ int decode_impl(const void* q, const void* k_cache, const void* v_cache, const i
     Q3_LAUNCH_CHECK();
     return Q3_OK;
   }
-  const int64_t rows = B * Hq;
-  if (dtype == Q3_F32)
-    hipLaunchKernelGGL(flash_generic_kernel<float>, dim3((unsigned)q3_cdiv(rows, 128)), dim3(128), 0, st, p, (int)D,
-                       kv_lens);
-  else if (dtype == Q3_BF16)
-    hipLaunchKernelGGL(flash_generic_kernel<bf16>, dim3((unsigned)q3_cdiv(rows, 128)), dim3(128), 0, st, p, (int)D,
-                       kv_lens);
-  else
-    return Q3_ERR_DTYPE;
-  Q3_LAUNCH_CHECK();
+  const int rc = launch_generic(p, (int)D, kv_lens, dtype, st);
+  if (rc != Q3_OK) return rc;
   if (lens_inc) {
     hipLaunchKernelGGL(lens_inc_kernel, dim3((unsigned)q3_cdiv(B, 256)), dim3(256), 0, st, lens_inc, (int)B, 1);
     Q3_LAUNCH_CHECK();

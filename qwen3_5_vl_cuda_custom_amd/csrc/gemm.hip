@@ -3,10 +3,13 @@
 //
 //   Y[m, n] = sum_k X[m, k] * W[n, k] (+ bias[n]) (+ R[m, n])   (nn.Linear layout)
 //
-// Three device paths, chosen on the host from the shape:
+// Four device paths, chosen on the host from the shape:
 //  * tiled   : bf16, M > 32     -> 32x32x16 MFMA over a ring of direct-to-LDS tiles
 //  * gemv    : bf16, M <= 32    -> weight-streaming stream-K kernel (gemv.hip)
-//  * generic : fp32, or bf16 whose rows are not 16-byte aligned -> SIMT fp32
+//  * fp32    : fp32 rows of whole 16-byte pieces -> 16x16x4 fp32 MFMA
+//  * generic : other fp32, or bf16 whose rows are not 16-byte aligned -> SIMT fp32
+#include <type_traits>
+
 #include "gemm_bwd.h"
 #include "gemm_kernels.h"
 #include "gemv.h"
@@ -94,6 +97,158 @@ int launch_generic(const void* x, const void* w, const void* w2, const void* bia
   Q3_LAUNCH_CHECK();
   return Q3_OK;
 }
+
+// =====================================================================
+// fp32 operands on the matrix cores (v_mfma_f32_16x16x4_f32: fp32 products and
+// sums). Y[m, n] = sum_k X[m, k] W[n, k], or with XT / WT an operand stored
+// with k as its rows (the GEMM backward's layouts, so nothing is transposed).
+// A wave owns 32 x 32 outputs and reads its fragments straight from memory:
+// per 16 k a lane takes 4 consecutive k of its row, the same 4 for both
+// operands, which is a k permutation common to both. KSPLIT: the block's 4
+// waves take 32-wide K chunks of one 32 x 32 tile in turn and are summed in
+// wave order (small problems, where tiles are few and a block's K loop is a
+// chain of load latencies); otherwise each wave has a tile of its own (64 x 64
+// per block). Against the SIMT kernel above (64 x 64 tiles: 8 blocks for 128 x
+// 256 outputs): the 21 products of a training step of a 256-wide layer at 128
+// tokens 1459 -> 203 us, without the 127 us of transposes.
+// =====================================================================
+__device__ __forceinline__ floatx4 mfma16x16x4f32(float a, float b, floatx4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+struct F32Params {
+  const float *X, *W, *bias, *R;
+  float* C;
+  int M, N, K;
+  int64_t ldx, ldw, ldr, ldc, bsX, bsW, bsC;
+  int act;
+};
+
+template <bool KSPLIT, bool XT, bool WT>
+__global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const F32Params p) {
+  __shared__ float s_red[KSPLIT ? 3 * 32 * 33 : 1];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l16 = lane & 15, g = lane >> 4;
+  const int64_t z = blockIdx.z;
+  const float* X = p.X + z * p.bsX;
+  const float* W = p.W + z * p.bsW;
+  const int m0 = KSPLIT ? blockIdx.y * 32 : blockIdx.y * 64 + 32 * (wave >> 1);
+  const int n0 = KSPLIT ? blockIdx.x * 32 : blockIdx.x * 64 + 32 * (wave & 1);
+  const int M = p.M, N = p.N, K = p.K;
+  constexpr int kStep = 32, kHalf = kStep / 16;  // k per chunk; 16-wide groups of it
+  // 4 k values (kb .. kb + 3) of row `r` of an operand; zeros outside it. K is a multiple of 4 where the k run along
+  // a row (one 16-byte load); with k as rows each is a load of its own and the row a column.
+  auto load = [&](const float* a, int64_t ld, int r, int rows, int kb, auto t) -> floatx4 {
+    floatx4 v = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (decltype(t)::value) {
+      if (r < rows) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (kb + e < K) v[e] = a[(int64_t)(kb + e) * ld + r];
+      }
+    } else {
+      if (r < rows && kb < K) v = *reinterpret_cast<const floatx4*>(a + (int64_t)r * ld + kb);
+    }
+    return v;
+  };
+  floatx4 acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  floatx4 xa[2][kHalf], wa[2][kHalf], xb[2][kHalf], wb[2][kHalf];
+  auto fetch = [&](floatx4 (&x)[2][kHalf], floatx4 (&w)[2][kHalf], int k0) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int h = 0; h < kHalf; ++h) {
+        x[i][h] = load(X, p.ldx, m0 + 16 * i + l16, M, k0 + 16 * h + 4 * g, std::integral_constant<bool, XT>{});
+        w[i][h] = load(W, p.ldw, n0 + 16 * i + l16, N, k0 + 16 * h + 4 * g, std::integral_constant<bool, WT>{});
+      }
+  };
+  auto mma = [&](const floatx4 (&x)[2][kHalf], const floatx4 (&w)[2][kHalf]) {
+#pragma unroll
+    for (int h = 0; h < kHalf; ++h)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) acc[i][j] = mfma16x16x4f32(x[i][h][e], w[j][h][e], acc[i][j]);
+  };
+  const int step = KSPLIT ? 4 * kStep : kStep;
+  int k0 = KSPLIT ? wave * kStep : 0;
+  fetch(xa, wa, k0);
+  for (; k0 < K; k0 += 2 * step) {  // two register sets in turn, one chunk ahead
+    fetch(xb, wb, k0 + step);
+    mma(xa, wa);
+    fetch(xa, wa, k0 + 2 * step);
+    mma(xb, wb);
+  }
+  // register r of lane (g, l16): row 4 g + r, column l16 of each 16 x 16 tile
+  if constexpr (KSPLIT) {
+    if (wave > 0) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            s_red[((wave - 1) * 32 + 16 * i + 4 * g + r) * 33 + 16 * j + l16] = acc[i][j][r];
+    }
+    __syncthreads();
+    if (wave > 0) return;
+#pragma unroll
+    for (int u = 0; u < 3; ++u)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            acc[i][j][r] += s_red[(u * 32 + 16 * i + 4 * g + r) * 33 + 16 * j + l16];
+  }
+  float* C = p.C + z * p.bsC;
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int n = n0 + 16 * j + l16;
+    if (n >= N) continue;
+    const float b = p.bias ? p.bias[n] : 0.f;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int m = m0 + 16 * i + 4 * g + r;
+        if (m >= M) continue;
+        float v = acc[i][j][r];
+        if (p.bias) v += b;
+        if (p.act) v = gelu_tanh_f(v);
+        if (p.R) v += p.R[(int64_t)m * p.ldr + n];
+        C[(int64_t)m * p.ldc + n] = v;
+      }
+  }
+}
+
+// 64 x 64 blocks once they give every CU two; below that 32 x 32 tiles with K
+// over the block's waves (four times the blocks and a quarter of the chain).
+template <bool XT, bool WT>
+int launch_f32(const F32Params& p, int64_t batch, hipStream_t st) {
+  if (q3_cdiv(p.M, 64) * q3_cdiv(p.N, 64) * batch >= 512) {
+    const dim3 grid((unsigned)q3_cdiv(p.N, 64), (unsigned)q3_cdiv(p.M, 64), (unsigned)batch);
+    hipLaunchKernelGGL((gemm_f32_mfma_kernel<false, XT, WT>), grid, dim3(256), 0, st, p);
+  } else {
+    const dim3 grid((unsigned)q3_cdiv(p.N, 32), (unsigned)q3_cdiv(p.M, 32), (unsigned)batch);
+    hipLaunchKernelGGL((gemm_f32_mfma_kernel<true, XT, WT>), grid, dim3(256), 0, st, p);
+  }
+  Q3_LAUNCH_CHECK();
+  return Q3_OK;
+}
+
+// A plain operand's rows as 16-byte pieces of 4.
+bool f32_rows_ok(const void* base, int64_t ld, int64_t K, int64_t bs) {
+  return q3_aligned(base, 16) && ld % 4 == 0 && K % 4 == 0 && bs % 4 == 0;
+}
+bool f32_grid_ok(int64_t M) { return q3_cdiv(M, 32) <= 65535; }
 
 // =====================================================================
 // Tiled MFMA path.
@@ -344,6 +499,13 @@ int matmul_impl(const void* x, const void* w, const void* w2, const void* bias, 
   Q3_REQUIRE(dtype == Q3_F32 || dtype == Q3_BF16, Q3_ERR_DTYPE);
   Q3_REQUIRE(!(swiglu && (bias || residual)), Q3_ERR_UNSUPPORTED);
   if (M == 0 || N == 0) return Q3_OK;
+  if (dtype == Q3_F32 && !swiglu && K > 0 && f32_rows_ok(x, ldx, K, bsX) && f32_rows_ok(w, ldw, K, bsW) &&
+      f32_grid_ok(M) && batch < 65536) {
+    F32Params f{static_cast<const float*>(x), static_cast<const float*>(w), static_cast<const float*>(bias),
+                static_cast<const float*>(residual), static_cast<float*>(y), (int)M, (int)N, (int)K, ldx, ldw, ldr,
+                ldc, bsX, bsW, bsC, act};
+    return launch_f32<false, false>(f, batch, st);
+  }
   if (dtype == Q3_F32)
     return launch_generic<float>(x, w, w2, bias, residual, y, M, N, K, batch, ldx, ldw, ldr, ldc, bsX, bsW, bsC,
                                  swiglu, st, act);
@@ -535,6 +697,16 @@ int gemm_nn(const void* x, const void* w, void* y, int64_t M, int64_t N, int64_t
 int gemm_tn(const void* x, const void* w, void* y, int64_t M, int64_t N, int64_t K, void* ws, int64_t ws_bytes,
             hipStream_t st) {
   return gemm_t<true>(x, w, y, M, N, K, ws, ws_bytes, st);
+}
+
+int gemm_f32_t(const void* x, const void* w, void* y, int64_t M, int64_t N, int64_t K, bool xt, hipStream_t st) {
+  F32Params f{static_cast<const float*>(x), static_cast<const float*>(w), nullptr, nullptr, static_cast<float*>(y),
+              (int)M, (int)N, (int)K, xt ? M : K, N, 0, N, 0, 0, 0, 0};
+  return xt ? launch_f32<true, true>(f, 1, st) : launch_f32<false, true>(f, 1, st);
+}
+
+bool gemm_f32_t_ok(const void* x, int64_t M, int64_t K, bool xt) {
+  return M > 0 && K > 0 && f32_grid_ok(M) && (xt || f32_rows_ok(x, K, K, 0));
 }
 
 int gemm_tn_ranges(const void* x, const void* w, void* y, int64_t M, int64_t N, int64_t rows, const int* k_off,

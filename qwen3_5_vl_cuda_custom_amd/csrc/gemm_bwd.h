@@ -22,4 +22,9 @@ int gemm_tn(const void* x, const void* w, void* y, int64_t M, int64_t N, int64_t
 int gemm_tn_ranges(const void* x, const void* w, void* y, int64_t M, int64_t N, int64_t rows, const int* k_off,
                    int64_t nz, hipStream_t st);
 
+// fp32: y (M, N) = x . w (K, N) with x (M, K), or with xt x (K, M) transposed. The
+// plain x needs 16-byte rows of whole pieces; w and a transposed x any layout.
+bool gemm_f32_t_ok(const void* x, int64_t M, int64_t K, bool xt);
+int gemm_f32_t(const void* x, const void* w, void* y, int64_t M, int64_t N, int64_t K, bool xt, hipStream_t st);
+
 }  // namespace q3

@@ -907,14 +907,14 @@ MmBwdLayout mm_bwd_layout(int64_t M, int64_t N, int64_t K, int dtype) {
 }
 
 // The products on the operands as they are (no transposes): bf16 rows of whole
-// 16-byte pieces and byte offsets below 2 GiB (gemm_bwd.h). The 21 transposes
+// 16-byte pieces and byte offsets below 2 GiB, or fp32 (gemm_bwd.h). The 21 transposes
 // of a dense layer's backward at S=2048 took 311 us of its 3143, the three of
 // a 151936 x 4096 head's 641 of 4289.
 bool mm_bwd_direct_x(const void* w, const void* dy, int64_t M, int64_t N, int64_t K, int dtype) {
-  return dtype == Q3_BF16 && q3::gemm_t_ok(dy, w, M, K, N, false);
+  return dtype == Q3_BF16 ? q3::gemm_t_ok(dy, w, M, K, N, false) : q3::gemm_f32_t_ok(dy, M, N, false);
 }
 bool mm_bwd_direct_w(const void* x, const void* dy, int64_t M, int64_t N, int64_t K, int dtype) {
-  return dtype == Q3_BF16 && q3::gemm_t_ok(dy, x, N, K, M, true);
+  return dtype == Q3_BF16 ? q3::gemm_t_ok(dy, x, N, K, M, true) : q3::gemm_f32_t_ok(dy, N, M, true);
 }
 
 }  // namespace
@@ -1107,7 +1107,9 @@ int q3_matmul_backward(const void* x, const void* w, const void* dy, void* gx, v
   int rc;
   if (gx) {  // gx (M, K) = dY (M, N) . W (N, K)
     if (dir_x) {
-      if ((rc = q3::gemm_nn(dy, w, gx, M, K, N, gemm_ws, gemm_ws_bytes, st)) != Q3_OK) return rc;
+      rc = dtype == Q3_BF16 ? q3::gemm_nn(dy, w, gx, M, K, N, gemm_ws, gemm_ws_bytes, st)
+                            : q3::gemm_f32_t(dy, w, gx, M, K, N, false, st);
+      if (rc != Q3_OK) return rc;
     } else {  // dY . (W^T)^T with W^T (K, N) as the GEMM's weight
       const int64_t need = q3_matmul_workspace_bytes(M, K, N, dtype, 0);
       Q3_REQUIRE(need <= 0 || (gemm_ws && gemm_ws_bytes >= need), Q3_ERR_WORKSPACE);
@@ -1119,7 +1121,9 @@ int q3_matmul_backward(const void* x, const void* w, const void* dy, void* gx, v
   }
   if (gw) {  // gw (N, K) = dY^T (N, M) . X (M, K)
     if (dir_w) {
-      if ((rc = q3::gemm_tn(dy, x, gw, N, K, M, gemm_ws, gemm_ws_bytes, st)) != Q3_OK) return rc;
+      rc = dtype == Q3_BF16 ? q3::gemm_tn(dy, x, gw, N, K, M, gemm_ws, gemm_ws_bytes, st)
+                            : q3::gemm_f32_t(dy, x, gw, N, K, M, true, st);
+      if (rc != Q3_OK) return rc;
     } else {  // dY^T . (X^T)^T with X^T (K, M) as the weight
       const int64_t need = q3_matmul_workspace_bytes(N, K, M, dtype, 0);
       Q3_REQUIRE(need <= 0 || (gemm_ws && gemm_ws_bytes >= need), Q3_ERR_WORKSPACE);

@@ -410,6 +410,45 @@ def test_flash_attention_backward_mfma_against_simt(B, Hq, Hkv, Sq, Sk, D, causa
             assert_grad_close(a, r, f"flash {n} D={D}")
 
 
+@pytest.mark.parametrize("M,N,K_", [(1, 4, 4), (31, 33, 36), (33, 31, 132), (128, 256, 688), (130, 66, 260),
+                                    (2050, 1030, 100), (65, 20, 30)])
+def test_matmul_and_backward_fp32_tiles(M, N, K_):
+    """fp32 GEMM, its gradients and the epilogue at the edges of the 32 x 32 and 64 x 64 tiles, of the K chunks and
+    (the last: rows that are no whole pieces) on the SIMT kernel. fp32 products and sums: at most (K + 2) 2^-24 of
+    the sum of absolute products."""
+    x, w, b, r, dy = (rnd(*sh, seed=40 + i) for i, sh in enumerate([(M, K_), (N, K_), (N,), (M, N), (M, N)]))
+    out, (gx, gw, gb, gr) = run_grads(lambda a, c, d, e: K.matmul(a, c, d, residual=e), [x, w, b, r], dy)
+    xd, wd, dd = x.double(), w.double(), dy.double()
+    for got, ref, mag, n in ((out, xd @ wd.t() + b.double() + r.double(), x.abs() @ w.abs().t() + b.abs() + r.abs(), K_),
+                             (gx, dd @ wd, dy.abs() @ w.abs(), N), (gw, dd.t() @ xd, dy.abs().t() @ x.abs(), M)):
+        over = float(((got.cpu().double() - ref).abs() - (n + 4) * 2.0 ** -24 * mag.double()).max())
+        assert over <= 0, over
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,D,causal,dtype", [
+    (1, 2, 1, 1, 1, 8, True, torch.float32), (2, 4, 2, 15, 33, 64, False, torch.float32),
+    (1, 4, 2, 128, 128, 64, True, torch.float32), (1, 3, 3, 17, 70, 65, False, torch.float32),
+    (1, 2, 2, 40, 40, 256, True, torch.float32), (2, 2, 1, 33, 31, 130, False, torch.float32),
+    (1, 4, 1, 50, 50, 32, True, torch.bfloat16), (1, 2, 2, 20, 64, 7, False, torch.bfloat16),
+])
+def test_flash_attention_generic_forward(B, Hq, Hkv, Sq, Sk, D, causal, dtype):
+    """The generic forward (fp32, other head dims) and its log-sum-exp at the edges of its 16-query and 32-key tiles."""
+    from qwen3_5_vl_cuda_custom_amd.kernels.flash_attention import flash_attention_lse
+    q, k, v = (rnd(B, h, s_, D, seed=60 + i, dtype=dtype) for i, (h, s_) in
+               enumerate([(Hq, Sq), (Hkv, Sk), (Hkv, Sk)]))
+    sc = D ** -0.5
+    o, lse = flash_attention_lse(q.to(DEV), k.to(DEV), v.to(DEV), sc, causal, Hq // Hkv)
+    ref = O.flash_attention(q.float(), k.float(), v.float(), sc, causal, Hq // Hkv)
+    if dtype == torch.float32:
+        assert_close(o, ref, atol=2e-5, what="o")  # sums of up to 70 fp32 terms of magnitude ~1
+    else:
+        assert_bf16_close(o, ref, what="o bf16")
+    scores = (q.float() @ k.float().repeat_interleave(Hq // Hkv, dim=1).transpose(-1, -2)) * sc
+    if causal:
+        scores = scores.masked_fill(torch.ones(Sq, Sk).triu(1).bool(), float("-inf"))
+    assert_close(lse, scores.logsumexp(-1), atol=2e-5, what="lse")
+
+
 # ------------------------------------------------------------------ embedding, rotary, routing
 @pytest.mark.parametrize("dtype,padding_idx", [(torch.float32, None), (torch.bfloat16, 3)])
 def test_embedding_backward(dtype, padding_idx):
