@@ -18,12 +18,15 @@
 //                                   rounding after each add (the order and
 //                                   rounding of a per-expert bf16 index_add),
 //                                   optionally plus a residual
+//                   At most 32 tokens (a decode step): one-block dispatch and
+//                   weight-streaming kernels instead of 1 to 5.
 //  q3_index_add     deterministic target[idx[i]] += src[i]: bucket the sources
 //                   by target, then each target adds its sources in ascending
 //                   source order in fp32 and rounds once.
 #include <algorithm>
 
 #include <climits>
+#include <type_traits>
 
 #include "gemm_bwd.h"
 #include "gemm_kernels.h"
@@ -177,6 +180,8 @@ struct MoeWs {
   int* pos_of;
   bf16* act;     // (P, I)
   bf16* y_perm;  // (P, H)
+  int* chunk_table;  // decode (moe_gemv_kernel): 16-row chunks of the experts' rows
+  int* n_chunks;
 };
 
 constexpr int kMoeChunk = 64;  // tokens per dispatch chunk (one wave)
@@ -484,6 +489,220 @@ __global__ __launch_bounds__(1024) void moe_combine_wide_kernel(const int* __res
   reinterpret_cast<bf16x8*>(out + (int64_t)t * H)[j] = o;
 }
 
+// ------------------------------------------------------------------ decode
+// A decode step routes at most 32 tokens, so an expert gets a few rows and its
+// products are a stream of its weights. The tile GEMMs (256-row tiles) leave
+// the last wave of tiles nearly empty there (82 experts x 8 down tiles: 2.6
+// waves) and stage and multiply 256 rows for one or two; moe_gemv_kernel
+// instead deals (16-row chunk of an expert, 32 weight rows) units evenly over
+// 256 blocks, and the dispatch of at most 1024 entries is one block's work.
+constexpr int kSmallT = 32, kSmallP = 1024, kSmallK = 2048;
+bool moe_small(int64_t T, int64_t H, int64_t I, int64_t k) {
+  return T <= kSmallT && T * k <= kSmallP && H <= kSmallK && I <= kSmallK;
+}
+
+// One block: counts, offsets, every entry's row (ascending (token, slot) per
+// expert: the entries before it with the same expert, counted by a scan of the
+// list in LDS) and the 16-row chunks (expert << 20 | first row), expert-major.
+__global__ __launch_bounds__(kSmallP) void moe_dispatch_small_kernel(const int* __restrict__ top_idx,
+                                                                     const bf16* __restrict__ top_w, int P, int k,
+                                                                     int E, MoeWs w) {
+  __shared__ __attribute__((aligned(16))) int s_e[kSmallP];
+  extern __shared__ int s_int[];  // counts -> offsets (E + 1), chunk counts -> offsets (E + 1)
+  int* s_off = s_int;
+  int* s_ch = s_int + E + 1;
+  const int i = threadIdx.x;
+  for (int e = i; e <= E; e += kSmallP) s_off[e] = s_ch[e] = 0;
+  int e = -1;
+  if (i < P) {
+    e = top_idx[i];
+    if (e < 0 || e >= E) e = -1;  // never dispatched
+  }
+  s_e[i] = e;
+  __syncthreads();
+  if (e >= 0) atomicAdd(&s_off[e], 1);
+  __syncthreads();
+  for (int x = i; x < E; x += kSmallP) s_ch[x] = (s_off[x] + 15) / 16;
+  __syncthreads();
+  if (i < 64) wave_excl_scan(s_off, E + 1);
+  else if (i < 128) wave_excl_scan(s_ch, E + 1);
+  int rank = 0;
+  const int4* e4 = reinterpret_cast<const int4*>(s_e);
+#pragma unroll 8
+  for (int j = 0; j < (P + 3) / 4; ++j) {
+    const int4 v = e4[j];
+    rank += (4 * j < i && v.x == e) + (4 * j + 1 < i && v.y == e) + (4 * j + 2 < i && v.z == e) +
+            (4 * j + 3 < i && v.w == e);
+  }
+  __syncthreads();
+  if (i < P) {
+    const int pos = e >= 0 ? s_off[e] + rank : -1;
+    w.pos_of[i] = pos;
+    if (pos >= 0) {
+      w.sorted_token[pos] = i / k;
+      w.sorted_w[pos] = top_w[i];
+    }
+  }
+  for (int x = i; x <= E; x += kSmallP) {
+    w.offsets[x] = s_off[x];
+    if (x < E)
+      for (int c = s_ch[x]; c < s_ch[x + 1]; ++c) w.chunk_table[c] = (x << 20) | (s_off[x] + 16 * (c - s_ch[x]));
+  }
+  if (i == 0) *w.n_chunks = s_ch[E];
+}
+
+struct MoeGemvP {
+  const bf16 *X, *W, *rowscale;  // X rows (through `gather` when set), W (E, rows, K)
+  bf16* C;                       // (P, N)
+  const int *gather, *chunk_table, *n_chunks, *offsets;
+  int N, K, ldx, x_rows;         // N: output columns (SWIGLU: I, W has 2 I rows)
+};
+
+// C[row] = X[row] . W[e]^T of at most 16 rows per chunk. A unit is 32 weight
+// rows (SWIGLU: 16 gate rows and the 16 up rows of the same columns, else 32
+// consecutive ones): waves 0, 1 take the first 16 rows, waves 2, 3 the other
+// 16, each wave one half of K, so its X fragments stay in registers while the
+// expert lasts (NST stages of 128 k, 4 fragments each). A wave streams its
+// weights through a private LDS ring of kRing stages (16 rows x 128 k, 4 KB) by
+// non-temporal direct-to-LDS loads that run on across units, no barrier in
+// between; the halves (and gate and up) meet in LDS once per unit, two buffers
+// in turn. Chunk c of a stage row r sits at slot c ^ r (conflict-free fragment
+// reads). SPLIT false (K <= 1024, plain): a unit is 64 rows, each wave takes 16
+// of them over all of K and stores them alone, with no exchange or barrier.
+// Bound by the weight stream: 16
+// tokens, top-8 of 128 experts, H = 2048, I = 768 (about 82 experts, 775 MB):
+// gate/up 110 -> 83 us (6.2 TB/s), down 59 -> 47 us against the tile GEMMs.
+template <bool SWIGLU, int NST, bool SPLIT>
+__global__ __launch_bounds__(256) void moe_gemv_kernel(const MoeGemvP p) {
+  constexpr int kRing = 8, kStage = 16 * 128;
+  __shared__ __attribute__((aligned(1024))) bf16 ring[4 * kRing * kStage];
+  __shared__ __attribute__((aligned(16))) floatx4 s_part[2][SPLIT ? 4 : 1][64];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  static_assert(SPLIT || !SWIGLU, "gate and up meet in the exchange");
+  constexpr int kUnit = SPLIT ? 32 : 64;  // weight rows per unit (SWIGLU: 16 of each matrix)
+  const int grp = SPLIT ? wave >> 1 : wave, kh = SPLIT ? wave & 1 : 0, l16 = lane & 15, q4 = lane >> 4;
+  const int N = p.N, K = p.K;
+  const int NG = SWIGLU ? (N + 15) / 16 : (N + kUnit - 1) / kUnit;
+  const int wrows = SWIGLU ? 2 * N : N;
+  const int64_t U = (int64_t)*p.n_chunks * NG;
+  const int u0 = (int)(U * blockIdx.x / gridDim.x), u1 = (int)(U * (blockIdx.x + 1) / gridDim.x);
+  if (u0 >= u1) return;
+  const int kbeg = kh * NST * 128;
+  const uint32_t lring = q3::lds_addr(ring + wave * kRing * kStage);
+
+  // Issue cursor: stage `is` of unit `iu` (chunk ic, group ig).
+  int iu = u0, is = 0, ic = u0 / NG, ig = u0 - ic * NG, slot_i = 0;
+  int ie = __builtin_amdgcn_readfirstlane(p.chunk_table[ic]) >> 20;
+  const int lrow = lane >> 4;
+  auto issue = [&]() {
+    const bool live = iu < u1;
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(p.W + (int64_t)ie * wrows * K, (int64_t)wrows * K * 2);
+    const int r0 = SWIGLU ? (grp ? N : 0) + 16 * ig : kUnit * ig + 16 * grp;
+    const int rlim = (SWIGLU ? 16 * ig : r0) + 16 <= N ? 16 : N - (SWIGLU ? 16 * ig : r0);  // live rows (may be <= 0)
+    const uint32_t dst = lring + (uint32_t)(slot_i * kStage * 2);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = 4 * i + lrow, k = kbeg + is * 128 + ((l16 ^ r) << 3);
+      const bool ok = live && r < rlim && k < K;
+      dma16_nt(rs, ok ? (uint32_t)(((r0 + r) * K + k) * 2) : kOOB, dst + (uint32_t)(i * 1024));
+    }
+    slot_i = slot_i + 1 == kRing ? 0 : slot_i + 1;
+    if (++is == NST) {
+      is = 0;
+      ++iu;
+      if (++ig == NG && iu < u1) {
+        ig = 0;
+        ie = __builtin_amdgcn_readfirstlane(p.chunk_table[++ic]) >> 20;
+      }
+    }
+  };
+#pragma unroll
+  for (int j = 0; j < kRing - 1; ++j) issue();
+
+  const __amdgpu_buffer_rsrc_t xrs = make_rsrc(p.X, (int64_t)p.x_rows * p.ldx * 2);
+  bf16x8 xf[NST * 4];
+  float rs = 1.f;  // this lane's row scale (loaded with the rows: a load in the epilogue would drain the ring)
+  int cc = -1, row0 = 0, rows = 0, slot_c = 0;
+  for (int u = u0; u < u1; ++u) {
+    const int c = u / NG, g = u - c * NG;
+    if (c != cc) {  // this chunk's rows as B fragments: lane l holds row l % 16, k 8 (l / 16) .. + 7 of each 32
+      cc = c;
+      const int entry = __builtin_amdgcn_readfirstlane(p.chunk_table[c]);
+      row0 = entry & 0xFFFFF;
+      rows = min(16, __builtin_amdgcn_readfirstlane(p.offsets[(entry >> 20) + 1]) - row0);
+      const bool live = l16 < rows;
+      const int src = live ? (p.gather ? p.gather[row0 + l16] : row0 + l16) : 0;
+      if constexpr (!SWIGLU) rs = live ? bf2f(p.rowscale[row0 + l16]) : 0.f;
+      const uint32_t x0 = live ? (uint32_t)(src * p.ldx * 2) : kOOB;
+#pragma unroll
+      for (int s = 0; s < NST * 4; ++s) {
+        const int k = kbeg + s * 32 + 8 * q4;
+        xf[s] = buffer_load16(xrs, k < K ? x0 + (uint32_t)(k * 2) : kOOB);
+      }
+    }
+    floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < NST; ++s) {
+      issue();
+      vm_wait<(kRing - 1) * 4>();  // the oldest stage has landed
+      const bf16* st = ring + (wave * kRing + slot_c) * kStage + l16 * 128;
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) {
+        const bf16x8 a = *reinterpret_cast<const bf16x8*>(st + (((4 * ks + q4) ^ l16) << 3));
+        acc = mfma16x16x32(a, xf[4 * s + ks], acc);
+      }
+      slot_c = slot_c + 1 == kRing ? 0 : slot_c + 1;
+    }
+    // register r of lane (q4, l16): weight row 4 q4 + r, token row l16
+    const int buf = u & 1;
+    if constexpr (SPLIT) {
+      s_part[buf][wave][lane] = acc;
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    }
+    if (kh == 0 && (!SWIGLU || grp == 0) && l16 < rows) {
+      floatx4 a = acc;
+      if constexpr (SPLIT) a += s_part[buf][wave + 1][lane];
+      const int n = SWIGLU ? 16 * g + 4 * q4 : kUnit * g + 16 * grp + 4 * q4;
+      bf16x4 o;
+      if constexpr (SWIGLU) {
+        const floatx4 b = s_part[buf][2][lane] + s_part[buf][3][lane];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = f2bf(silu_mul(a[e], b[e]));
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = f2bf(bf2f(f2bf(a[e])) * rs);
+      }
+      if (n < N) *reinterpret_cast<bf16x4*>(p.C + (int64_t)(row0 + l16) * N + n) = o;  // N is a multiple of 8
+    }
+  }
+  vm_wait<0>();  // no load may still target this block's LDS when the wave retires
+}
+
+template <bool SWIGLU, bool SPLIT>
+int launch_moe_gemv_t(const MoeGemvP& p, hipStream_t st) {
+  const int n = (int)q3_cdiv(p.K, SPLIT ? 256 : 128);  // stages of 128 k per wave
+  auto run = [&](auto stages) {
+    hipLaunchKernelGGL((moe_gemv_kernel<SWIGLU, decltype(stages)::value, SPLIT>), dim3(256), dim3(256), 0, st, p);
+  };
+  if constexpr (SWIGLU || !SPLIT) {  // (the plain split form starts at K > 1024)
+    if (n == 1) run(std::integral_constant<int, 1>{});
+    if (n == 2) run(std::integral_constant<int, 2>{});
+    if (n == 3) run(std::integral_constant<int, 3>{});
+    if (n == 4) run(std::integral_constant<int, 4>{});
+  }
+  if (n == 5 || n == 6) run(std::integral_constant<int, 6>{});
+  if (n > 6) run(std::integral_constant<int, 8>{});
+  Q3_LAUNCH_CHECK();
+  return Q3_OK;
+}
+template <bool SWIGLU>
+int launch_moe_gemv(const MoeGemvP& p, hipStream_t st) {
+  if constexpr (!SWIGLU) {
+    if (p.K <= 1024) return launch_moe_gemv_t<SWIGLU, false>(p, st);
+  }
+  return launch_moe_gemv_t<SWIGLU, true>(p, st);
+}
+
 int64_t align256(int64_t x) { return (x + 255) / 256 * 256; }
 
 int64_t moe_ws_layout(int64_t T, int64_t H, int64_t I, int64_t E, int64_t k, MoeWs* ws, char* base) {
@@ -508,6 +727,10 @@ int64_t moe_ws_layout(int64_t T, int64_t H, int64_t I, int64_t E, int64_t k, Moe
   w.pos_of = reinterpret_cast<int*>(take(P * 4));
   w.act = reinterpret_cast<bf16*>(take(P * I * 2));
   w.y_perm = reinterpret_cast<bf16*>(take(P * H * 2));
+  if (moe_small(T, H, I, k)) {
+    w.chunk_table = reinterpret_cast<int*>(take((E + P / 16 + 1) * 4));
+    w.n_chunks = reinterpret_cast<int*>(take(4));
+  }
   if (ws) *ws = w;
   return off;
 }
@@ -1047,6 +1270,20 @@ int q3_moe_experts(const void* x, const void* gate_up, const void* down, const i
   moe_ws_layout(T, H, I, E, k, &w, static_cast<char*>(workspace));
   const int64_t P = T * k;
   const int64_t max_tiles = q3_cdiv(P, kMoeBM) + E;
+  if (moe_small(T, H, I, k)) {  // decode: the weights as an even stream
+    hipLaunchKernelGGL(moe_dispatch_small_kernel, dim3(1), dim3(kSmallP), 2 * (E + 1) * sizeof(int), st,
+                       top_idx, static_cast<const bf16*>(top_w), (int)P, (int)k, (int)E, w);
+    Q3_LAUNCH_CHECK();
+    MoeGemvP g{static_cast<const bf16*>(x), static_cast<const bf16*>(gate_up), nullptr, w.act, w.sorted_token,
+               w.chunk_table, w.n_chunks, w.offsets, (int)I, (int)H, (int)H, (int)T};
+    int rc = launch_moe_gemv<true>(g, st);
+    if (rc != Q3_OK) return rc;
+    g = {w.act, static_cast<const bf16*>(down), w.sorted_w, w.y_perm, nullptr, w.chunk_table, w.n_chunks, w.offsets,
+         (int)H, (int)I, (int)I, (int)P};
+    if ((rc = launch_moe_gemv<false>(g, st)) != Q3_OK) return rc;
+    return launch_combine(top_idx, w.pos_of, w.y_perm, static_cast<const bf16*>(residual), static_cast<bf16*>(out), T,
+                          H, E, k, st);
+  }
   {
     const int rc = moe_dispatch(top_idx, static_cast<const bf16*>(top_w), T, k, E, w, st);
     if (rc != Q3_OK) return rc;

@@ -671,6 +671,34 @@ def test_moe_route_exact_indices():
     assert_bf16_close(w, rv / rv.sum(-1, keepdim=True), max_abs=4e-3, what="routing weights")
 
 
+@pytest.mark.parametrize("T,H,I,E,k,skew", [(1, 2048, 768, 128, 8, False), (16, 2048, 768, 128, 8, False),
+                                            (32, 2048, 768, 128, 8, False), (17, 264, 40, 8, 2, True),
+                                            (32, 136, 24, 4, 3, True), (5, 1032, 520, 16, 4, False),
+                                            (32, 512, 1544, 4, 1, True), (2, 8, 8, 2, 2, False)])
+def test_moe_experts_decode_rows(T, H, I, E, k, skew):
+    """At most 32 tokens (the weight-streaming kernels: one to 32 rows per expert, experts without rows, widths that
+    are no multiple of a 128-wide stage or a 32-row unit) against the tile GEMMs, which 64 tokens run: the same fp32
+    sums in another order, so activations and expert outputs may round to the neighbouring bf16 value (2^-8 of it,
+    through the down projection 2^-8 of the row's scale)."""
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x = torch.randn(64, H, generator=g, device="cuda").bfloat16()
+    gu = (torch.randn(E, 2 * I, H, generator=g, device="cuda") * H ** -0.5).bfloat16()
+    dn = (torch.randn(E, H, I, generator=g, device="cuda") * I ** -0.5).bfloat16()
+    p = torch.rand(64, E, generator=g, device="cuda")
+    if skew:
+        p[:, 0] += 10.0  # every token picks expert 0
+    idx = p.topk(k, dim=-1).indices.to(torch.int32)
+    w = torch.rand(64, k, generator=g, device="cuda").bfloat16()
+    res = torch.randn(64, H, generator=g, device="cuda").bfloat16()
+    got = K.moe_experts(x[:T], gu, dn, idx[:T], w[:T], res[:T]).float()
+    ref = K.moe_experts(x, gu, dn, idx, w, res)[:T].float()
+    err = (got - ref).abs()
+    tol = 2.0 ** -7 * ref.abs() + 2.0 ** -7 * float((ref - res[:T].float()).abs().max())
+    assert bool((err <= tol).all()), float((err - tol).max())
+    assert float(err.mean()) <= 2.0 ** -9 * float(ref.abs().mean())
+    assert torch.equal(K.moe_experts(x[:T], gu, dn, idx[:T], w[:T], res[:T]).float(), got)
+
+
 @pytest.mark.parametrize("E,k,norm", [(8, 1, True), (8, 8, True), (64, 4, False), (100, 8, True), (256, 32, True),
                                       (500, 16, False), (500, 32, True)])
 def test_moe_route_ties_and_widths(E, k, norm):
