@@ -531,6 +531,30 @@ int q3_flash_attention_backward(const void* q, const void* k, const void* v, con
                                 const void* grad_out, void* grad_q, void* grad_k, void* grad_v, int64_t B, int64_t Hq,
                                 int64_t Hkv, int64_t Sq, int64_t Sk, int64_t D, float scale, int is_causal,
                                 int dtype, void* workspace, int64_t workspace_bytes, void* stream);
+/* The same on (B, H, S, D) views: strides = (b, h, s) of q, k, v, o, grad_out,
+ * grad_q, grad_k, grad_v (24 values, the head dim contiguous). The matrix-core
+ * kernels only: bf16, D as above, 16-byte aligned bases, strides in multiples
+ * of 8, row strides of at least D, rows within 2 GiB of a head's first, else
+ * Q3_ERR_UNSUPPORTED. */
+int q3_flash_attention_backward_strided(const void* q, const void* k, const void* v, const void* o, const float* lse,
+                                        const void* grad_out, void* grad_q, void* grad_k, void* grad_v, int64_t B,
+                                        int64_t Hq, int64_t Hkv, int64_t Sq, int64_t Sk, int64_t D,
+                                        const int64_t* strides, float scale, int is_causal, int dtype,
+                                        void* workspace, int64_t workspace_bytes, void* stream);
+
+/* Gradients of q3_qk_norm_rope without a cache and with both norm weights (the
+ * reference differentiates its norm and rotation ops one by one): grad_q, q_in,
+ * dq (B, S, Hq, D) and grad_k, k_in, dk (B, S, Hkv, D) views, strides = (b, s, h)
+ * of grad_q, grad_k, q_in, k_in, dq, dk, grad_v, dv (24 values); grad_v, dv
+ * (B, S, Hkv, D), both or neither: copied; dw (2, D): q_weight's gradient, then
+ * k_weight's. D in {64, 128, 256}. */
+int64_t q3_qk_norm_rope_backward_workspace_bytes(int64_t B, int64_t S, int64_t D);
+int q3_qk_norm_rope_backward(const void* grad_q, const void* grad_k, const void* grad_v, const void* q_in,
+                             const void* k_in,
+                             const void* q_weight, const void* k_weight, const int* positions, const float* inv_freq,
+                             void* dq, void* dk, void* dv, void* dw, int64_t B, int64_t S, int64_t Hq, int64_t Hkv, int64_t D,
+                             const int64_t* section, float eps, const int64_t* strides, int dtype, void* workspace,
+                             int64_t workspace_bytes, void* stream);
 
 #ifdef __cplusplus
 }

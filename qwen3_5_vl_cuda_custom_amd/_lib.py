@@ -104,6 +104,11 @@ _SIGS: dict[str, tuple] = {
     "q3_moe_train_workspace_bytes": (c_int64, [_I, _I, _I, _I, _I, c_int]),
     "q3_moe_train_forward": (c_int, [_V, _V, _V, _i32p, _V, _V, _I, _I, _I, _I, _I, _V, _I, _V, _I, _V]),
     "q3_moe_train_backward": (c_int, [_V, _V, _V, _V, _V, _V, _V, _V, _I, _I, _I, _I, _I, _V, _I, _V, _I, _V]),
+    "q3_flash_attention_backward_strided": (c_int, [_V, _V, _V, _V, _f32p, _V, _V, _V, _V, _I, _I, _I, _I, _I, _I,
+                                                    _i64p, c_float, c_int, c_int, _V, _I, _V]),
+    "q3_qk_norm_rope_backward_workspace_bytes": (c_int64, [_I, _I, _I]),
+    "q3_qk_norm_rope_backward": (c_int, [_V, _V, _V, _V, _V, _V, _V, _i32p, _f32p, _V, _V, _V, _V, _I, _I, _I, _I, _I,
+                                         _i64p, c_float, _i64p, c_int, _V, _I, _V]),
     "q3_flash_attention_backward_workspace_bytes": (c_int64, [_I, _I, _I]),
     "q3_flash_attention_backward_mfma_workspace_bytes": (c_int64, [_I, _I, _I, _I, _I, _I, c_int]),
     "q3_flash_attention_backward": (c_int, [_V, _V, _V, _V, _f32p, _V, _V, _V, _V, _I, _I, _I, _I, _I, _I, c_float,

@@ -312,6 +312,10 @@ __device__ __forceinline__ void dma4(__amdgpu_buffer_rsrc_t r, uint32_t voff, ui
                : "memory");
 }
 
+struct Str {
+  int64_t b, h, s;  // element strides of (batch, head, row); rows are contiguous
+};
+
 struct P {
   const bf16 *q, *k, *v, *o, *dout;
   const float* lse;
@@ -321,6 +325,7 @@ struct P {
   int B, Hq, Hkv, Sq, Sk, groups, n_qt, hs;
   float scale, scale_log2;
   int causal;
+  Str sq, sk, sv, so, sg, sdq, sdk, sdv;  // q, k, v, o, dout and the gradients
 };
 
 // Blocks in order of falling work (causal), dealt back and forth over the
@@ -361,9 +366,9 @@ __global__ __launch_bounds__(256) void stats_kernel(const P p) {
   if (bh >= (int64_t)p.B * p.Hq) return;
   float acc = 0.f;
   if (i < p.Sq && part * 8 < D) {
-    const int64_t at = (bh * p.Sq + i) * D + part * 8;
-    const bf16x8 o = *reinterpret_cast<const bf16x8*>(p.o + at);
-    const bf16x8 g = *reinterpret_cast<const bf16x8*>(p.dout + at);
+    const int64_t b = bh / p.Hq, h = bh - b * p.Hq;
+    const bf16x8 o = *reinterpret_cast<const bf16x8*>(p.o + b * p.so.b + h * p.so.h + i * p.so.s + part * 8);
+    const bf16x8 g = *reinterpret_cast<const bf16x8*>(p.dout + b * p.sg.b + h * p.sg.h + i * p.sg.s + part * 8);
 #pragma unroll
     for (int e = 0; e < 8; ++e) acc = fmaf(bf2f(o[e]), bf2f(g[e]), acc);
   }
@@ -396,19 +401,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   r /= p.hs;
   const int kvh = r % p.Hkv, b = r / p.Hkv;
   const int gper = p.groups / p.hs;
-  const int h0 = b * p.Hq + kvh * p.groups + sp * gper;  // first (batch, query head) of the split
+  const int h0 = kvh * p.groups + sp * gper;  // first query head of the split
   const int j0 = kt * kOwn, kw0 = j0 + 32 * wave, key = kw0 + l32;
   const int64_t kv_row = ((int64_t)b * p.Hkv + kvh) * p.Sk;
 
   // K and V rows of the wave as B fragments
   bf16x8 kf[KSTEPS], vf[KSTEPS];
   {
-    const int64_t at = (kv_row + (key < p.Sk ? key : 0)) * D;
+    const int64_t row = key < p.Sk ? key : 0;
+    const bf16* kr = p.k + b * p.sk.b + kvh * p.sk.h + row * p.sk.s;
+    const bf16* vr = p.v + b * p.sv.b + kvh * p.sv.h + row * p.sv.s;
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ++ks) {
       const bool ok = key < p.Sk && ks * 16 + 8 * h < D;
-      kf[ks] = ok ? *reinterpret_cast<const bf16x8*>(p.k + at + ks * 16 + 8 * h) : bf16x8{};
-      vf[ks] = ok ? *reinterpret_cast<const bf16x8*>(p.v + at + ks * 16 + 8 * h) : bf16x8{};
+      kf[ks] = ok ? *reinterpret_cast<const bf16x8*>(kr + ks * 16 + 8 * h) : bf16x8{};
+      vf[ks] = ok ? *reinterpret_cast<const bf16x8*>(vr + ks * 16 + 8 * h) : bf16x8{};
     }
   }
   floatx16 dk[OT], dv[OT];
@@ -421,23 +428,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
   const uint32_t lring = q3::lds_addr(ring), lstat = q3::lds_addr(s_stat);
   const int cs = lane & 15;
+  const int sq2 = (int)p.sq.s * 2, sg2 = (int)p.sg.s * 2;  // host: Sq * stride * 2 < 2^31
   int ig = 0, it = t_first;  // (head of the split, tile) the next issue takes
   auto issue = [&](int step) {
     const int slot = step % kStg;
     const bool live = step < n;
     const int64_t hd = h0 + (live ? ig : 0);
-    const __amdgpu_buffer_rsrc_t qrs = q3::make_rsrc(p.q + hd * p.Sq * D, (int64_t)p.Sq * D * 2);
-    const __amdgpu_buffer_rsrc_t grs = q3::make_rsrc(p.dout + hd * p.Sq * D, (int64_t)p.Sq * D * 2);
-    const __amdgpu_buffer_rsrc_t srs = q3::make_rsrc(p.stats + hd * p.n_qt * 64, (int64_t)p.n_qt * 256);
+    const __amdgpu_buffer_rsrc_t qrs =
+        q3::make_rsrc(p.q + b * p.sq.b + hd * p.sq.h, ((int64_t)(p.Sq - 1) * p.sq.s + D) * 2);
+    const __amdgpu_buffer_rsrc_t grs =
+        q3::make_rsrc(p.dout + b * p.sg.b + hd * p.sg.h, ((int64_t)(p.Sq - 1) * p.sg.s + D) * 2);
+    const __amdgpu_buffer_rsrc_t srs =
+        q3::make_rsrc(p.stats + ((int64_t)b * p.Hq + hd) * p.n_qt * 64, (int64_t)p.n_qt * 256);
     const uint32_t lq = lring + (uint32_t)(slot * 2 * kTileE * 2);
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int rr = 8 * wave + 4 * i + (lane >> 4);
       const int c = cs ^ swz(rr);
-      const uint32_t vo = live && c * 8 < D ? (uint32_t)((it * kT32 + rr) * (D * 2) + c * 16) : q3::kOOB;
+      const bool ok = live && c * 8 < D;  // rows past Sq lie past the resources' ends
       const uint32_t at = (uint32_t)((8 * wave + 4 * i) * kRow * 2);
-      q3::dma16(qrs, vo, lq + at);
-      q3::dma16(grs, vo, lq + kTileE * 2 + at);
+      q3::dma16(qrs, ok ? (uint32_t)((it * kT32 + rr) * sq2 + c * 16) : q3::kOOB, lq + at);
+      q3::dma16(grs, ok ? (uint32_t)((it * kT32 + rr) * sg2 + c * 16) : q3::kOOB, lq + kTileE * 2 + at);
     }
     // every wave writes the same 64 floats: one load per wave keeps the counts equal
     dma4(srs, live ? (uint32_t)(it * 256 + lane * 4) : q3::kOOB, lstat + (uint32_t)(slot * 256));
@@ -515,8 +526,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   q3::vm_wait<0>();  // no load may still target this block's LDS when the wave retires
   if (key >= p.Sk) return;
   if (p.hs == 1) {
-    bf16* ko = p.dk + (kv_row + key) * D;
-    bf16* vo = p.dv + (kv_row + key) * D;
+    bf16* ko = p.dk + b * p.sdk.b + kvh * p.sdk.h + key * p.sdk.s;
+    bf16* vo = p.dv + b * p.sdv.b + kvh * p.sdv.h + key * p.sdv.s;
 #pragma unroll
     for (int t = 0; t < OT; ++t)
 #pragma unroll
@@ -556,8 +567,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
 }
 
-// dK, dV = the head splits' partials in split order, rounded once. n4: floatx4 elements of one plane.
-__global__ __launch_bounds__(256) void dkdv_reduce_kernel(const P p, int64_t n4) {
+// dK, dV = the head splits' partials in split order, rounded once. n4: floatx4 elements of one plane, d4 of one row.
+__global__ __launch_bounds__(256) void dkdv_reduce_kernel(const P p, int64_t n4, int d4) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= 2 * n4) return;
   const floatx4* src = reinterpret_cast<const floatx4*>(p.part) + i;
@@ -568,7 +579,11 @@ __global__ __launch_bounds__(256) void dkdv_reduce_kernel(const P p, int64_t n4)
   bf16x4 o;
 #pragma unroll
   for (int e = 0; e < 4; ++e) o[e] = f2bf(a[e] * f);
-  reinterpret_cast<bf16x4*>(is_v ? p.dv : p.dk)[is_v ? i - n4 : i] = o;
+  const int64_t r = (is_v ? i - n4 : i) / d4, bh = r / p.Sk, b = bh / p.Hkv;
+  const int c = (int)((is_v ? i - n4 : i) - r * d4);
+  const Str st = is_v ? p.sdv : p.sdk;
+  bf16* out = (is_v ? p.dv : p.dk) + b * st.b + (bh - b * p.Hkv) * st.h + (r - bh * p.Sk) * st.s + c * 4;
+  *reinterpret_cast<bf16x4*>(out) = o;
 }
 
 // dQ of 128 queries of one head.
@@ -588,17 +603,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int qt = p.causal ? n_own - 1 - blk / nh : blk / nh;  // the last queries see the most keys
   const int bh = blk % nh, b = bh / p.Hq, kvh = (bh % p.Hq) / p.groups;
   const int q0 = qt * kOwn, qw0 = q0 + 32 * wave, qi = qw0 + l32;
-  const int64_t q_row = (int64_t)bh * p.Sq;
-  const int64_t kv_row = ((int64_t)b * p.Hkv + kvh) * p.Sk;
+  const int hq = bh - b * p.Hq;
 
   bf16x8 qf[KSTEPS], gf[KSTEPS];
   {
-    const int64_t at = (q_row + (qi < p.Sq ? qi : 0)) * D;
+    const int64_t row = qi < p.Sq ? qi : 0;
+    const bf16* qr = p.q + b * p.sq.b + hq * p.sq.h + row * p.sq.s;
+    const bf16* gr = p.dout + b * p.sg.b + hq * p.sg.h + row * p.sg.s;
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ++ks) {
       const bool ok = qi < p.Sq && ks * 16 + 8 * h < D;
-      qf[ks] = ok ? *reinterpret_cast<const bf16x8*>(p.q + at + ks * 16 + 8 * h) : bf16x8{};
-      gf[ks] = ok ? *reinterpret_cast<const bf16x8*>(p.dout + at + ks * 16 + 8 * h) : bf16x8{};
+      qf[ks] = ok ? *reinterpret_cast<const bf16x8*>(qr + ks * 16 + 8 * h) : bf16x8{};
+      gf[ks] = ok ? *reinterpret_cast<const bf16x8*>(gr + ks * 16 + 8 * h) : bf16x8{};
     }
   }
   float lse2 = 1.0e30f, dvi = 0.f;
@@ -615,18 +631,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int n = (klimit + kT32 - 1) / kT32;
   const uint32_t lring = q3::lds_addr(ring);
   const int cs = lane & 15;
-  const __amdgpu_buffer_rsrc_t krs = q3::make_rsrc(p.k + kv_row * D, (int64_t)p.Sk * D * 2);
-  const __amdgpu_buffer_rsrc_t vrs = q3::make_rsrc(p.v + kv_row * D, (int64_t)p.Sk * D * 2);
+  const __amdgpu_buffer_rsrc_t krs =
+      q3::make_rsrc(p.k + b * p.sk.b + kvh * p.sk.h, ((int64_t)(p.Sk - 1) * p.sk.s + D) * 2);
+  const __amdgpu_buffer_rsrc_t vrs =
+      q3::make_rsrc(p.v + b * p.sv.b + kvh * p.sv.h, ((int64_t)(p.Sk - 1) * p.sv.s + D) * 2);
+  const int sk2 = (int)p.sk.s * 2, sv2 = (int)p.sv.s * 2;  // host: Sk * stride * 2 < 2^31
   auto issue = [&](int t) {
     const uint32_t lk = lring + (uint32_t)((t % kStg) * 2 * kTileE * 2);
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int rr = 8 * wave + 4 * i + (lane >> 4);
       const int c = cs ^ swz(rr);
-      const uint32_t vo = t < n && c * 8 < D ? (uint32_t)((t * kT32 + rr) * (D * 2) + c * 16) : q3::kOOB;
+      const bool ok = t < n && c * 8 < D;
       const uint32_t at = (uint32_t)((8 * wave + 4 * i) * kRow * 2);
-      q3::dma16(krs, vo, lk + at);
-      q3::dma16(vrs, vo, lk + kTileE * 2 + at);
+      q3::dma16(krs, ok ? (uint32_t)((t * kT32 + rr) * sk2 + c * 16) : q3::kOOB, lk + at);
+      q3::dma16(vrs, ok ? (uint32_t)((t * kT32 + rr) * sv2 + c * 16) : q3::kOOB, lk + kTileE * 2 + at);
     }
   };
   int ro[KSTEPS];
@@ -680,7 +699,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
   q3::vm_wait<0>();
   if (qi >= p.Sq) return;
-  bf16* qo = p.dq + (q_row + qi) * D;
+  bf16* qo = p.dq + b * p.sdq.b + hq * p.sdq.h + qi * p.sdq.s;
 #pragma unroll
   for (int t = 0; t < OT; ++t)
 #pragma unroll
@@ -720,7 +739,8 @@ int launch_d(const P& p, hipStream_t st) {
   Q3_LAUNCH_CHECK();
   if (p.hs > 1) {
     const int64_t n4 = (int64_t)p.B * p.Hkv * p.Sk * D / 4;
-    hipLaunchKernelGGL(dkdv_reduce_kernel, dim3((unsigned)q3_cdiv(2 * n4, 256)), dim3(256), 0, st, p, n4);
+    hipLaunchKernelGGL(dkdv_reduce_kernel, dim3((unsigned)q3_cdiv(2 * n4, 256)), dim3(256), 0, st, p, n4,
+                       D / 4);
     Q3_LAUNCH_CHECK();
   }
   hipLaunchKernelGGL(dq_kernel<D>, dim3((unsigned)nq), dim3(256), 0, st, p);
@@ -734,6 +754,59 @@ int launch(const P& p, int D, hipStream_t st) {
   if (D == 80) return launch_d<80>(p, st);
   if (D == 96) return launch_d<96>(p, st);
   return launch_d<128>(p, st);
+}
+
+// 16-byte loads (aligned bases, strides in multiples of 8; 8-byte stores), 32-bit byte offsets within a head, and a
+// workspace that holds the row statistics. strides: (b, h, s) of q, k, v, o, grad_out, grad_q, grad_k, grad_v.
+bool takes(const void* q, const void* k, const void* v, const void* o, const void* g, const void* dq, const void* dk,
+           const void* dv, int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t Sk, int64_t D,
+           const int64_t* strides, int dtype, const void* ws, int64_t ws_bytes) {
+  if (dtype != Q3_BF16 || !head_dim_ok(D) || Sk < 1 || ws_bytes < stats_bytes(B, Hq, Sq) || !q3_aligned(ws, 16))
+    return false;
+  for (const void* x : {q, k, v, o, g})
+    if (!q3_aligned(x, 16)) return false;
+  for (const void* x : {dq, dk, dv})
+    if (!q3_aligned(x, 8)) return false;
+  for (int i = 0; i < 24; ++i)
+    if (strides[i] % 8 != 0 || strides[i] < 0) return false;
+  for (int t = 0; t < 8; ++t)
+    if (strides[3 * t + 2] < D) return false;  // row r of a tile past the last one is past the resource's end
+  const int64_t lim = 1ll << 31;
+  for (int t : {0, 1, 2, 4})
+    if (((t == 1 || t == 2 ? Sk : Sq) + kT32) * strides[3 * t + 2] * 2 >= lim) return false;
+  return q3_cdiv(Sk, kOwn) * B * Hq < lim && q3_cdiv(Sq, kOwn) * B * Hq < lim;
+}
+
+int run(const void* q, const void* k, const void* v, const void* o, const float* lse, const void* g, void* dq,
+        void* dk, void* dv, int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t Sk, int64_t D,
+        const int64_t* strides, float scale, int is_causal, void* ws, int64_t ws_bytes, hipStream_t st) {
+  P m{};
+  m.q = static_cast<const bf16*>(q);
+  m.k = static_cast<const bf16*>(k);
+  m.v = static_cast<const bf16*>(v);
+  m.o = static_cast<const bf16*>(o);
+  m.dout = static_cast<const bf16*>(g);
+  m.lse = lse;
+  m.stats = static_cast<float*>(ws);
+  m.part = m.stats + stats_bytes(B, Hq, Sq) / 4;
+  m.dq = static_cast<bf16*>(dq);
+  m.dk = static_cast<bf16*>(dk);
+  m.dv = static_cast<bf16*>(dv);
+  m.B = (int)B;
+  m.Hq = (int)Hq;
+  m.Hkv = (int)Hkv;
+  m.Sq = (int)Sq;
+  m.Sk = (int)Sk;
+  m.groups = (int)(Hq / Hkv);
+  m.n_qt = (int)q3_cdiv(Sq, kT32);
+  m.hs = (int)head_splits(B, Hkv, Hq / Hkv, Sk);
+  if (ws_bytes < stats_bytes(B, Hq, Sq) + part_bytes(B, Hkv, m.hs, Sk, D)) m.hs = 1;
+  m.scale = scale;
+  m.scale_log2 = scale * kLog2e;
+  m.causal = is_causal ? 1 : 0;
+  Str* const to[8] = {&m.sq, &m.sk, &m.sv, &m.so, &m.sg, &m.sdq, &m.sdk, &m.sdv};
+  for (int t = 0; t < 8; ++t) *to[t] = {strides[3 * t], strides[3 * t + 1], strides[3 * t + 2]};
+  return launch(m, (int)D, st);
 }
 
 }  // namespace bmf
@@ -790,43 +863,35 @@ int q3_flash_attention_backward(const void* q, const void* k, const void* v, con
   p.scale = scale;
   p.causal = is_causal ? 1 : 0;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  // The MFMA kernels: 16-byte loads (rows of a multiple of 8 elements from aligned bases), 32-bit offsets within
-  // a head, a workspace for the row statistics (a caller that sized it by the fp32-per-row query alone gets the
-  // SIMT kernels) and, where it is large enough, the head splits' partials.
-  const int64_t stats = bmf::stats_bytes(B, Hq, Sq);
-  if (dtype == Q3_BF16 && bmf::head_dim_ok(D) && Sk > 0 && workspace_bytes >= stats && q3_aligned(workspace, 16) &&
-      q3_aligned(q, 16) && q3_aligned(k, 16) && q3_aligned(v, 16) && q3_aligned(o, 16) && q3_aligned(grad_out, 16) &&
-      q3_aligned(grad_q, 8) && q3_aligned(grad_k, 8) && q3_aligned(grad_v, 8) && (Sq + bmf::kT32) * D * 2 < (1ll << 31) &&
-      (Sk + bmf::kT32) * D * 2 < (1ll << 31) && q3_cdiv(Sk, bmf::kOwn) * B * Hq < (1ll << 31) &&
-      q3_cdiv(Sq, bmf::kOwn) * B * Hq < (1ll << 31) && stats < (1ll << 40)) {
-    bmf::P m{};
-    m.q = static_cast<const bf16*>(q);
-    m.k = static_cast<const bf16*>(k);
-    m.v = static_cast<const bf16*>(v);
-    m.o = static_cast<const bf16*>(o);
-    m.dout = static_cast<const bf16*>(grad_out);
-    m.lse = lse;
-    m.stats = static_cast<float*>(workspace);
-    m.part = m.stats + stats / 4;
-    m.dq = static_cast<bf16*>(grad_q);
-    m.dk = static_cast<bf16*>(grad_k);
-    m.dv = static_cast<bf16*>(grad_v);
-    m.B = (int)B;
-    m.Hq = (int)Hq;
-    m.Hkv = (int)Hkv;
-    m.Sq = (int)Sq;
-    m.Sk = (int)Sk;
-    m.groups = (int)(Hq / Hkv);
-    m.n_qt = (int)q3_cdiv(Sq, bmf::kT32);
-    m.hs = (int)bmf::head_splits(B, Hkv, Hq / Hkv, Sk);
-    if (workspace_bytes < stats + bmf::part_bytes(B, Hkv, m.hs, Sk, D)) m.hs = 1;
-    m.scale = scale;
-    m.scale_log2 = scale * bmf::kLog2e;
-    m.causal = is_causal ? 1 : 0;
-    return bmf::launch(m, (int)D, st);
-  }
+  // The MFMA kernels where they take the call (a caller that sized the workspace by the fp32-per-row query alone gets
+  // the SIMT kernels).
+  const int64_t sq[3] = {Hq * Sq * D, Sq * D, D}, sk[3] = {Hkv * Sk * D, Sk * D, D};
+  int64_t strides[24];
+  for (int t = 0; t < 8; ++t)
+    for (int i = 0; i < 3; ++i) strides[3 * t + i] = (t == 1 || t == 2 || t == 6 || t == 7) ? sk[i] : sq[i];
+  if (bmf::takes(q, k, v, o, grad_out, grad_q, grad_k, grad_v, B, Hq, Hkv, Sq, Sk, D, strides, dtype, workspace,
+                 workspace_bytes))
+    return bmf::run(q, k, v, o, lse, grad_out, grad_q, grad_k, grad_v, B, Hq, Hkv, Sq, Sk, D, strides, scale,
+                    is_causal, workspace, workspace_bytes, st);
   if (dtype == Q3_BF16) return attn_bwd_d<bf16>(p, st);
   return attn_bwd_d<float>(p, st);
+}
+
+int q3_flash_attention_backward_strided(const void* q, const void* k, const void* v, const void* o, const float* lse,
+                                        const void* grad_out, void* grad_q, void* grad_k, void* grad_v, int64_t B,
+                                        int64_t Hq, int64_t Hkv, int64_t Sq, int64_t Sk, int64_t D,
+                                        const int64_t* strides, float scale, int is_causal, int dtype,
+                                        void* workspace, int64_t workspace_bytes, void* stream) {
+  Q3_REQUIRE(q && k && v && o && lse && grad_out && grad_q && grad_k && grad_v && strides, Q3_ERR_NULL);
+  Q3_REQUIRE(B >= 0 && Hq >= 1 && Hkv >= 1 && Sq >= 0 && Sk >= 0 && D >= 1, Q3_ERR_SHAPE);
+  Q3_REQUIRE(Hq % Hkv == 0 && B * Hq < 65536 && Sq < (1ll << 30) && Sk < (1ll << 30), Q3_ERR_SHAPE);
+  if (B == 0 || Sq == 0) return Q3_OK;
+  Q3_REQUIRE(workspace && workspace_bytes >= bmf::stats_bytes(B, Hq, Sq), Q3_ERR_WORKSPACE);
+  Q3_REQUIRE(bmf::takes(q, k, v, o, grad_out, grad_q, grad_k, grad_v, B, Hq, Hkv, Sq, Sk, D, strides, dtype,
+                        workspace, workspace_bytes),
+             Q3_ERR_UNSUPPORTED);
+  return bmf::run(q, k, v, o, lse, grad_out, grad_q, grad_k, grad_v, B, Hq, Hkv, Sq, Sk, D, strides, scale, is_causal,
+                  workspace, workspace_bytes, static_cast<hipStream_t>(stream));
 }
 
 }  // extern "C"

@@ -27,4 +27,7 @@ int gemm_tn_ranges(const void* x, const void* w, void* y, int64_t M, int64_t N, 
 bool gemm_f32_t_ok(const void* x, int64_t M, int64_t K, bool xt);
 int gemm_f32_t(const void* x, const void* w, void* y, int64_t M, int64_t N, int64_t K, bool xt, hipStream_t st);
 
+// out[c] = the sum of the nparts rows of `part` (cols fp32 each), in a fixed order, rounded once (train.hip).
+int colsum_reduce_rows(const float* part, void* out, int64_t nparts, int64_t cols, int dtype, hipStream_t st);
+
 }  // namespace q3

@@ -919,6 +919,13 @@ bool mm_bwd_direct_w(const void* x, const void* dy, int64_t M, int64_t N, int64_
 
 }  // namespace
 
+namespace q3 {
+int colsum_reduce_rows(const float* part, void* out, int64_t nparts, int64_t cols, int dtype, hipStream_t st) {
+  return dtype == Q3_BF16 ? colsum_reduce<bf16>(part, out, nparts, cols, st)
+                          : colsum_reduce<float>(part, out, nparts, cols, st);
+}
+}  // namespace q3
+
 extern "C" {
 
 int q3_sigmoid_mul(const void* x, const void* gate, void* y, int64_t n, int dtype, void* stream) {

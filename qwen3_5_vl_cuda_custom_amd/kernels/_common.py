@@ -3,6 +3,9 @@ from __future__ import annotations
 
 import torch
 
+# head dims of the MFMA attention kernels, forward and backward
+MFMA_HEAD_DIMS = (64, 72, 80, 96, 128)
+
 
 def require_device(op: str, *tensors: torch.Tensor | None) -> None:
     for t in tensors:

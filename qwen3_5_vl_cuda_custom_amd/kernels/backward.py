@@ -13,6 +13,7 @@ from __future__ import annotations
 import torch
 
 from .. import _lib
+from ._common import MFMA_HEAD_DIMS
 
 
 def needs_grad(*tensors) -> bool:
@@ -87,16 +88,50 @@ class BatchedGemmFunction(torch.autograd.Function):
 
 
 # ------------------------------------------------------------------ attention
+def _bhs(t: torch.Tensor):  # strides of the dims before the contiguous head dim
+    return t.stride(0), t.stride(1), t.stride(2)
+
+
+def attention_bshd_ok(q: torch.Tensor, D: int, rows: int, row_stride: int) -> bool:
+    """Whether attention gradients run on (B, S, H, D) storage as it is: the matrix-core backward
+    (bf16, its head dims), rows of `row_stride` elements within the kernels' 32-bit offsets."""
+    return q.dtype == torch.bfloat16 and D in MFMA_HEAD_DIMS and (rows + 32) * row_stride * 2 < 2 ** 31
+
+
+def _attn_grad_operand(t: torch.Tensor) -> torch.Tensor:
+    ok = (t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all(s % 8 == 0 and s >= 0 for s in t.stride()[:3])
+          and t.stride(2) >= t.shape[3] and (t.shape[2] + 32) * t.stride(2) * 2 < 2 ** 31)
+    return t if ok else t.clone(memory_format=torch.contiguous_format)
+
+
+def _attn_backward_strided(q, k, v, o, lse, do, dq, dk, dv, scale: float, is_causal: bool) -> None:
+    """Attention gradients on (B, H, S, D) views of any layout (the matrix-core kernels)."""
+    B, Hq, Sq, D = q.shape
+    Hkv, Sk = k.shape[1], k.shape[2]
+    q, k, v, o, do = (_attn_grad_operand(t) for t in (q, k, v, o, do))
+    ws, nws = _lib.workspace(_lib.lib().q3_flash_attention_backward_mfma_workspace_bytes(
+        B, Hq, Hkv, Sq, Sk, D, _dt(q)), q.device)
+    _lib.call("q3_flash_attention_backward_strided", q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
+              lse.data_ptr(), do.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), B, Hq, Hkv, Sq, Sk, D,
+              _lib.i64s(*_bhs(q), *_bhs(k), *_bhs(v), *_bhs(o), *_bhs(do), *_bhs(dq), *_bhs(dk), *_bhs(dv)),
+              scale, int(is_causal), _dt(q), _lib.ptr(ws), nws, _lib.stream())
+
+
 class FlashAttentionFunction(torch.autograd.Function):
-    """Reference: kernels/flash_attention.py:21-78, csrc/flash_attention_op.cu:235-390."""
+    """Reference: kernels/flash_attention.py:21-78, csrc/flash_attention_op.cu:235-390.
+    bshd: the output is a (B, Hq, Sq, D) view of (B, Sq, Hq, D) storage (attention_bshd_ok), so that
+    the projection after it reads it as it is."""
 
     @staticmethod
-    def forward(ctx, q, k, v, scale, is_causal, num_kv_groups):
-        from .flash_attention import flash_attention_lse
+    def forward(ctx, q, k, v, scale, is_causal, num_kv_groups, bshd=False):
+        from .flash_attention import _flash_fwd
         q, k, v = _c(q), _c(k), _c(v)
-        o, lse = flash_attention_lse(q, k, v, scale, is_causal, num_kv_groups)
+        B, Hq, Sq, D = q.shape
+        lse = torch.empty((B, Hq, Sq), dtype=torch.float32, device=q.device)
+        out = torch.empty((B, Sq, Hq, D), dtype=q.dtype, device=q.device).transpose(1, 2) if bshd else None
+        o = _flash_fwd(q, k, v, scale, is_causal, num_kv_groups, out, lse)
         ctx.save_for_backward(q, k, v, o, lse)
-        ctx.scale, ctx.is_causal = float(scale), bool(is_causal)
+        ctx.scale, ctx.is_causal, ctx.bshd = float(scale), bool(is_causal), bool(bshd)
         return o
 
     @staticmethod
@@ -105,12 +140,85 @@ class FlashAttentionFunction(torch.autograd.Function):
         B, Hq, Sq, D = q.shape
         Hkv, Sk = k.shape[1], k.shape[2]
         dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
+        if ctx.bshd:
+            _attn_backward_strided(q, k, v, o, lse, do.to(q.dtype), dq, dk, dv, ctx.scale, ctx.is_causal)
+            return dq, dk, dv, None, None, None, None
         ws, nws = _lib.workspace(_lib.lib().q3_flash_attention_backward_mfma_workspace_bytes(
             B, Hq, Hkv, Sq, Sk, D, _dt(q)), q.device)
         _lib.call("q3_flash_attention_backward", q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
                   lse.data_ptr(), _c(do).to(q.dtype).data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), B, Hq,
                   Hkv, Sq, Sk, D, ctx.scale, int(ctx.is_causal), _dt(q), _lib.ptr(ws), nws, _lib.stream())
-        return dq, dk, dv, None, None, None
+        return dq, dk, dv, None, None, None, None
+
+
+class RopeAttentionFunction(torch.autograd.Function):
+    """Vision attention on the fused projection: rotation of q and k, attention (not causal), o (B, S, H, D)
+    from qkv (B, S, 3, H, D) (reference modules/attention.py:34-42: two rotations, attention and three
+    slices, each with its own backward). The gradients are written into the qkv layout as they are made:
+    no slice gradients to fill, add and transpose. attention_bshd_ok calls only."""
+
+    @staticmethod
+    def forward(ctx, qkv, cos, sin, scale):
+        from .flash_attention import _flash_fwd
+        from .rotary import apply_rope
+        B, S, _, H, D = qkv.shape
+        qk = apply_rope(qkv[:, :, :2].reshape(B, S, 2 * H, D).transpose(1, 2), cos, sin)
+        lse = torch.empty((B, H, S), dtype=torch.float32, device=qkv.device)
+        o = torch.empty((B, S, H, D), dtype=qkv.dtype, device=qkv.device)
+        _flash_fwd(qk[:, :H], qk[:, H:], qkv[:, :, 2].transpose(1, 2), scale, False, 1, o.transpose(1, 2), lse)
+        ctx.save_for_backward(qkv, qk, o, lse, cos, sin)
+        ctx.scale = float(scale)
+        return o
+
+    @staticmethod
+    def backward(ctx, do):
+        from .rotary import rope_into
+        qkv, qk, o, lse, cos, sin = ctx.saved_tensors
+        B, S, _, H, D = qkv.shape
+        dqkv = torch.empty_like(qkv, memory_format=torch.contiguous_format)
+        dqk = torch.empty((B, 2 * H, S, D), dtype=qkv.dtype, device=qkv.device)
+        _attn_backward_strided(qk[:, :H], qk[:, H:], qkv[:, :, 2].transpose(1, 2), o.transpose(1, 2), lse,
+                               do.to(qkv.dtype).transpose(1, 2), dqk[:, :H], dqk[:, H:],
+                               dqkv[:, :, 2].transpose(1, 2), ctx.scale, False)
+        rope_into(dqk, cos, -sin, dqkv.view(B, S, 3 * H, D)[:, :, :2 * H].transpose(1, 2))
+        return dqkv, None, None, None
+
+
+class QKNormRopeFunction(torch.autograd.Function):
+    """Per-head RMSNorm and mRoPE of q and k, and v, from the projections' (B, S, H, D) outputs to contiguous
+    (B, H, S, D) (reference modules/attention.py:83-88 as single ops). Angles are computed from the integer
+    positions in fp32 in both directions."""
+
+    @staticmethod
+    def forward(ctx, q, k, v, q_weight, k_weight, positions, inv_freq, mrope_section, eps):
+        from .rotary import qk_norm_rope
+        B, S, Hq, D = q.shape
+        Hkv = k.shape[2]
+        qo, ko, vo = (torch.empty((B, h, S, D), dtype=q.dtype, device=q.device) for h in (Hq, Hkv, Hkv))
+        qk_norm_rope(q, k, v, qo.transpose(1, 2), ko.transpose(1, 2), vo.transpose(1, 2), q_weight, k_weight,
+                     positions, inv_freq, mrope_section, eps)
+        ctx.save_for_backward(q, k, q_weight, k_weight, positions, inv_freq)
+        ctx.section, ctx.eps = tuple(mrope_section), float(eps)
+        return qo, ko, vo
+
+    @staticmethod
+    def backward(ctx, gq, gk, gv):
+        q, k, qw, kw, pos, inv_freq = ctx.saved_tensors
+        B, S, Hq, D = q.shape
+        Hkv = k.shape[2]
+        gq, gk, gv = (g.to(q.dtype) if g.stride(-1) == 1 else g.to(q.dtype).contiguous() for g in (gq, gk, gv))
+        dq, dk = torch.empty_like(q, memory_format=torch.contiguous_format), torch.empty(
+            (B, S, Hkv, D), dtype=q.dtype, device=q.device)
+        dv = torch.empty_like(dk)
+        dw = torch.empty((2, D), dtype=qw.dtype, device=q.device)
+        ws, nws = _lib.workspace(_lib.lib().q3_qk_norm_rope_backward_workspace_bytes(B, S, D), q.device)
+        gt = [g.transpose(1, 2) for g in (gq, gk, gv)]  # (B, S, H, D) views
+        strides = [x for t in (gt[0], gt[1], q, k, dq, dk, gt[2], dv) for x in _bhs(t)]
+        _lib.call("q3_qk_norm_rope_backward", gq.data_ptr(), gk.data_ptr(), gv.data_ptr(), q.data_ptr(), k.data_ptr(),
+                  qw.data_ptr(), kw.data_ptr(), pos.data_ptr(), inv_freq.data_ptr(), dq.data_ptr(), dk.data_ptr(),
+                  dv.data_ptr(), dw.data_ptr(), B, S, Hq, Hkv, D, _lib.i64s(*ctx.section), ctx.eps,
+                  _lib.i64s(*strides), _dt(q), _lib.ptr(ws), nws, _lib.stream())
+        return dq, dk, dv, dw[0], dw[1], None, None, None, None
 
 
 # ------------------------------------------------------------------ norms / softmax

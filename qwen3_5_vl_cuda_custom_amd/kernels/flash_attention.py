@@ -4,11 +4,8 @@ from __future__ import annotations
 import torch
 
 from .. import _lib
-from ._common import check, mfma_operand, note_slow_path
+from ._common import MFMA_HEAD_DIMS, check, mfma_operand, note_slow_path
 from .backward import FlashAttentionFunction, needs_grad
-
-
-MFMA_HEAD_DIMS = (64, 72, 80, 96, 128)
 
 
 def _attn_operands(op: str, D: int, o: torch.Tensor | None, *ts):

@@ -25,6 +25,12 @@ def apply_rope(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.T
     """
     if needs_grad(x):
         return RopeFunction.apply(x, cos, sin)
+    B, H, S, D = x.shape
+    return rope_into(x, cos, sin, torch.empty((B, H, S, D), dtype=x.dtype, device=x.device))
+
+
+def rope_into(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, y: torch.Tensor) -> torch.Tensor:
+    """apply_rope into y, a (B, H, S, D) view with a contiguous head dim that x does not overlap."""
     check("apply_rope", x)
     if not cos.is_cuda or not sin.is_cuda:
         raise RuntimeError("apply_rope: cos/sin must be on the GPU")
@@ -42,7 +48,6 @@ def apply_rope(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.T
         raise ValueError(f"apply_rope: cos {tuple(cos.shape)} must be (S, Dr) or (B|1, S, Dr)")
     if cos.shape[-2] != S or sin.shape != cos.shape or Dr > D or Dr % 2:
         raise ValueError("apply_rope: cos/sin shape mismatch")
-    y = torch.empty((B, H, S, D), dtype=x.dtype, device=x.device)
     _lib.call("q3_rope", x.data_ptr(), cos.data_ptr(), sin.data_ptr(), y.data_ptr(), B, H, S, D, Dr,
               _lib.i64s(*_bhsd_strides(x)), _lib.i64s(*_bhsd_strides(y)), cb, cos.stride(-2),
               _lib.dtype_code(x.dtype), _cos_dtype(cos), _lib.stream())

@@ -482,6 +482,104 @@ def test_rope_and_mrope_backward():
     assert_close(gx, rx, atol=1e-4, what="rope dx")
 
 
+@pytest.mark.parametrize("B,S,Hq,Hkv,D,dtype", [
+    (1, 1, 1, 1, 64, torch.float32), (2, 5, 4, 2, 64, torch.bfloat16), (1, 300, 3, 1, 128, torch.bfloat16),
+    (2, 600, 8, 2, 128, torch.float32), (1, 17, 5, 5, 256, torch.bfloat16),
+])
+@torch.enable_grad()
+def test_qk_norm_rope_trains_like_the_single_ops_in_fp64(B, S, Hq, Hkv, D, dtype):
+    """The fused q/k norm + rotation and its gradients at one token, fewer tokens than blocks and more, and rows
+    that are no whole pass, on column views of one projection. Against fp64 with the same fp32 angles (sincosf: 2
+    ulp, 2^-22, of rotated values up to max|y|): fp32 sums of up to D terms stay within (D + 8) 2^-24 of their
+    magnitude, so 2^-15 of the largest value bounds them for D <= 256; the weight gradients add B S H terms; bf16
+    adds one rounding, 2^-8 of the value."""
+    from qwen3_5_vl_cuda_custom_amd.kernels.backward import QKNormRopeFunction
+    sec, eps, H = (D // 2 - 2 * (D // 6), D // 6, D // 6), 1e-6, Hq + 2 * Hkv
+    qkv = rnd(B, S, H, D, seed=80).to(dtype)
+    w = [(1 + 0.1 * rnd(D, seed=81 + i)).to(dtype) for i in range(2)]
+    dy = rnd(B, H, S, D, seed=83).to(dtype)
+    pos = torch.randint(0, 5000, (3, B, S), generator=torch.Generator().manual_seed(84), dtype=torch.int32)
+    inv = 1.0 / (5e6 ** (torch.arange(0, D, 2, dtype=torch.float32) / D))
+    ins = [t.to(DEV).requires_grad_(True) for t in (qkv, *w)]
+    out = torch.cat(QKNormRopeFunction.apply(ins[0][:, :, :Hq], ins[0][:, :, Hq:Hq + Hkv], ins[0][:, :, Hq + Hkv:],
+                                             ins[1], ins[2], pos.to(DEV), inv.to(DEV), sec, eps), dim=1)
+    got = torch.autograd.grad(out, ins, dy.to(DEV))
+    x, wq, wk = (t.double().requires_grad_(True) for t in (qkv, *w))
+    axis = torch.tensor([0] * sec[0] + [1] * sec[1] + [2] * sec[2])
+    ang = (pos.float()[axis] * inv[:, None, None]).double().permute(1, 2, 0)[:, :, None]  # (B, S, 1, D / 2)
+
+    def part(t, wt):
+        n = t * torch.rsqrt(t.pow(2).mean(-1, keepdim=True) + eps) * wt
+        a, b = n[..., :D // 2], n[..., D // 2:]
+        return torch.cat([a * ang.cos() - b * ang.sin(), b * ang.cos() + a * ang.sin()], dim=-1).transpose(1, 2)
+
+    ref_out = torch.cat([part(x[:, :, :Hq], wq), part(x[:, :, Hq:Hq + Hkv], wk), x[:, :, Hq + Hkv:].transpose(1, 2)], 1)
+    ref = torch.autograd.grad(ref_out, (x, wq, wk), dy.double())
+    rounding = 2.0 ** -8 if dtype == torch.bfloat16 else 0.0
+    for a, r, n in ((out, ref_out, 1), (got[0], ref[0], 1), (got[1], ref[1], B * S * Hq), (got[2], ref[2], B * S * Hkv)):
+        mag = r.abs().max() if n == 1 else n ** 0.5 * 16 + r.abs().max()
+        over = float(((a.detach().cpu().double() - r.detach()).abs() - rounding * r.abs() - 2.0 ** -15 * mag).max())
+        assert over <= 0, over
+
+
+@pytest.mark.parametrize("B,H,Hkv,S,D,causal", [(1, 2, 2, 1, 72, False), (2, 4, 4, 130, 72, False),
+                                                (1, 4, 1, 257, 128, True), (2, 4, 2, 64, 64, True)])
+@torch.enable_grad()
+def test_attention_gradients_on_token_major_storage(B, H, Hkv, S, D, causal):
+    """The same kernels on (B, S, H, D) storage as on (B, H, S, D): the same bits, also for the vision block's
+    rotation and attention on the fused projection against its single ops."""
+    from qwen3_5_vl_cuda_custom_amd.kernels.backward import FlashAttentionFunction, RopeAttentionFunction
+    q, k, v = (rnd(B, h, S, D, seed=85 + i).bfloat16().to(DEV).requires_grad_(True) for i, h in
+               enumerate((H, Hkv, Hkv)))
+    dy = rnd(B, S, H, D, seed=88).bfloat16().to(DEV).transpose(1, 2)
+    outs = []
+    for bshd in (False, True):
+        o = FlashAttentionFunction.apply(q, k, v, D ** -0.5, causal, H // Hkv, bshd)
+        outs.append((o.contiguous(), *torch.autograd.grad(o, (q, k, v), dy)))
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)
+    if causal:
+        return
+    qkv = rnd(B, S, 3, H, D, seed=89).bfloat16().to(DEV).requires_grad_(True)
+    ang = rnd(S, D, seed=90).to(DEV)
+    cos, sin = ang.cos(), ang.sin()
+    o1 = RopeAttentionFunction.apply(qkv, cos, sin, D ** -0.5)
+    qs, ks, vs = (qkv[:, :, i].transpose(1, 2) for i in range(3))
+    o2 = K.flash_attention(K.apply_rope(qs, cos, sin), K.apply_rope(ks, cos, sin), vs, D ** -0.5, False,
+                           1).transpose(1, 2)
+    assert torch.equal(o1, o2)
+    assert torch.equal(*(torch.autograd.grad(o, qkv, dy.transpose(1, 2))[0] for o in (o1, o2)))
+
+
+@torch.enable_grad()
+def test_text_attention_training_routes_agree():
+    """Positions as floats, a hook on a norm and a frozen norm weight: the first two take the single ops, and every
+    route gives the fused one's result up to the roundings between its single ops (three of 2^-8 of the largest)."""
+    from qwen3_5_vl_cuda_custom_amd.modules import CudaFullAttention, TextMRoPE
+    torch.manual_seed(0)
+    att = CudaFullAttention(256, 4, 2, 64).to(DEV, torch.bfloat16)
+    rope = TextMRoPE(64, 5e6, [12, 10, 10]).to(DEV)
+    x = rnd(2, 70, 256, seed=91).bfloat16().to(DEV)
+    pos = torch.arange(70, device=DEV).expand(3, 1, 70).contiguous()
+
+    def run(p):
+        xi = x.clone().requires_grad_(True)
+        out, _ = att(xi, rope.bind(p))
+        return out.detach(), torch.autograd.grad(out.float().pow(2).sum(), xi)[0]
+
+    want, runs = run(pos), [run(pos.float()), run(pos.int())]
+    seen = []
+    h = att.q_norm.register_forward_hook(lambda *a: seen.append(1))
+    runs.append(run(pos))
+    h.remove()
+    assert seen
+    att.q_norm.weight.requires_grad_(False)
+    runs.append(run(pos))
+    for got in runs:
+        for a, b in zip(got, want):
+            assert float((a.float() - b.float()).abs().max()) <= 3 * 2.0 ** -8 * float(b.float().abs().max())
+
+
 def test_topk_and_index_add_backward():
     x = rnd(64, 128, seed=77)
     gv = rnd(64, 8, seed=78)
