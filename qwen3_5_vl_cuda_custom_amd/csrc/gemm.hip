@@ -254,12 +254,12 @@ bool f32_grid_ok(int64_t M) { return q3_cdiv(M, 32) <= 65535; }
 // Tiled MFMA path.
 // =====================================================================
 template <int BM, int BN, int WM, int WN, int EPI, int NST, int BKT, int NSTW = NST, bool MF16 = false,
-          bool XT = false, bool WT = false>
+          bool XT = false, bool WT = false, bool STREAM = false>
 int launch_tiled_cfg(GemmParams p, int64_t batch, hipStream_t st) {
   constexpr int BN_OUT = (EPI == kEpiSwiGLU) ? BN / 2 : BN;
   const int64_t tiles = q3_cdiv(p.M, BM) * q3_cdiv(p.N, BN_OUT);
   p.group_m = 4;  // 4 along M: S=4096 gate/up 587 -> 582 us, o 112 -> 110, S=1024 layer 430.6 -> 425.4 (8 and 16: slower)
-  hipLaunchKernelGGL((gemm_bf16_dma_kernel<BM, BN, WM, WN, EPI, false, NST, BKT, NSTW, MF16, XT, WT>),
+  hipLaunchKernelGGL((gemm_bf16_dma_kernel<BM, BN, WM, WN, EPI, false, NST, BKT, NSTW, MF16, XT, WT, STREAM>),
                      dim3((unsigned)tiles, 1, (unsigned)batch), dim3(WM * WN * 64), 0, st, p);
   Q3_LAUNCH_CHECK();
   return Q3_OK;
@@ -727,7 +727,7 @@ int gemm_tn_ranges(const void* x, const void* w, void* y, int64_t M, int64_t N, 
   p.ldc = N;
   p.bsC = M * N;
   p.k_off = k_off;
-  return launch_tiled_cfg<256, 256, 2, 4, kEpiStore, 2, 64, 3, true, true, true>(p, nz, st);
+  return launch_tiled_cfg<256, 256, 2, 4, kEpiStore, 2, 64, 3, true, true, true, true>(p, nz, st);
 }
 
 }  // namespace q3

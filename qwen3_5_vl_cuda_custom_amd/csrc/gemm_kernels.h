@@ -356,7 +356,13 @@ __device__ __forceinline__ bool epi_rounds_first(const GemmParams& p, const Tile
 // flight before its stores. Values are those of store_tile_lds (one rounding,
 // same arithmetic). LDS rows are BN_OUT bf16; 16-byte chunk c of row r sits
 // at chunk c ^ (r & SWZ).
-template <int BM, int BN_OUT, int EPI, int NW, int LDS_BYTES, typename VISIT>
+//
+// STREAM: whole chunks are stored past the caches. The weight gradients of many
+// experts are far more than the caches hold and are read next by the optimizer,
+// after the whole backward, while their lines push the operands' out of L2: 128
+// experts, 16384 routed rows, (1536 and 768) x 2048 a gradient 253 -> 231 us on
+// average. One layer's gradient is not stored so: lm_head's step was 0.6% slower.
+template <int BM, int BN_OUT, int EPI, int NW, int LDS_BYTES, bool STREAM, typename VISIT>
 __device__ __forceinline__ void store_tile_lds_bf16(const GemmParams& p, const TileCtx& t, VISIT&& visit, bf16* lds) {
   constexpr int RP0 = LDS_BYTES / (BN_OUT * 2);
   constexpr int RP1 = RP0 >= 256 ? 256 : RP0 >= 128 ? 128 : RP0 >= 64 ? 64 : 32;
@@ -387,7 +393,10 @@ __device__ __forceinline__ void store_tile_lds_bf16(const GemmParams& p, const T
     }
     bf16* crow = t.C + (int64_t)m * p.ldc;
     if (whole || (vec_ok && n + 7 < N)) {
-      *reinterpret_cast<bf16x8*>(crow + n) = v;
+      if constexpr (STREAM)
+        __builtin_nontemporal_store(v, reinterpret_cast<bf16x8*>(crow + n));
+      else
+        *reinterpret_cast<bf16x8*>(crow + n) = v;
     } else {
 #pragma unroll
       for (int q = 0; q < 8; ++q)
@@ -479,7 +488,7 @@ __device__ __forceinline__ tr_short4 lds_tr16(uint32_t byte) {
 // under the power cap a pure MFMA loop sustains ~2.03 PFLOP/s with it against
 // ~1.80 with 32x32x16 (MI355X), and these GEMMs run power-limited.
 template <int BM, int BN, int WM, int WN, int EPI, bool GROUPED, int NST, int BKT, int NSTW = NST, bool MF16 = false,
-          bool XT = false, bool WT = false>
+          bool XT = false, bool WT = false, bool STREAM = false>
 __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_dma_kernel(const GemmParams p) {
   static_assert(MF16 || (!XT && !WT), "operands with the reduction as rows: the 16x16x32 loop");
   static_assert(!WT || EPI != kEpiSwiGLU, "no gate/up pairing of a transposed operand");
@@ -835,7 +844,7 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_dma_kernel(const GemmPa
 
     auto visit = [&](auto&& f) { visit_acc16<EPI, WTM, WTN, T16N, T16M>(a16, wm, wn, lane, f); };
     if (epi_rounds_first<EPI>(p, tc))
-      store_tile_lds_bf16<BM, BN_OUT, EPI, NW, kRing * 2>(p, tc, visit, smem);
+      store_tile_lds_bf16<BM, BN_OUT, EPI, NW, kRing * 2, STREAM>(p, tc, visit, smem);
     else if constexpr (EPI == kEpiStore || EPI == kEpiStoreF32)
       store_tile_lds<BM, BN_OUT, EPI, NW, kRing * 2>(p, tc, visit, reinterpret_cast<float*>(smem));
   } else {
@@ -1100,7 +1109,7 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_dma_kernel(const GemmPa
 
   auto visit = [&](auto&& f) { visit_acc32<EPI, WTM, WTN, TN, TM>(acc.c, wm, wn, lane, f); };
   if (epi_rounds_first<EPI>(p, tc))
-    store_tile_lds_bf16<BM, BN_OUT, EPI, NW, kRing * 2>(p, tc, visit, smem);
+    store_tile_lds_bf16<BM, BN_OUT, EPI, NW, kRing * 2, STREAM>(p, tc, visit, smem);
   else if constexpr (EPI == kEpiStore || EPI == kEpiStoreF32)
     store_tile_lds<BM, BN_OUT, EPI, NW, kRing * 2>(p, tc, visit, reinterpret_cast<float*>(smem));
   }  // 32x32x16 loop
