@@ -334,18 +334,69 @@ __device__ __forceinline__ void store_tile_lds(const GemmParams& p, const TileCt
 
 // True when the stored value takes no fp32 arithmetic after its one rounding:
 // SwiGLU, the row scale (whose first step rounds the accumulator), a plain
-// store without bias, activation or residual.
+// store without residual (bias and activation are applied to the accumulators,
+// bias_act_acc).
 template <int EPI>
-__device__ __forceinline__ bool epi_rounds_first(const GemmParams& p, const TileCtx& t) {
+__device__ __forceinline__ bool epi_rounds_first(const GemmParams& p) {
   if constexpr (EPI == kEpiSwiGLU || EPI == kEpiRowScale) {
     return true;
   } else if constexpr (EPI == kEpiStoreF32) {
     return false;
   } else {
-    bool bias = p.seg.n > 1 ? false : t.bias != nullptr;
+    return p.R == nullptr;
+  }
+}
+
+// Bias of output columns n .. n + 3 (n a multiple of 4); zeros past the last column.
+__device__ __forceinline__ floatx4 bias4(const GemmParams& p, const TileCtx& t, int n) {
+  const bf16* b = t.bias;
+  if (p.seg.n > 1) {  // per lane: the lanes' columns may lie in different segments (their starts: multiples of 16)
+    const int sgi = segment_of(p.seg, n);
+    b = pick4(sgi, p.seg.b[0], p.seg.b[1], p.seg.b[2], p.seg.b[3]);
+    if (b) b -= pick4(sgi, p.seg.start[0], p.seg.start[1], p.seg.start[2], p.seg.start[3]);
+  }
+  floatx4 v = {0.f, 0.f, 0.f, 0.f};
+  if (b) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) bias = bias || (p.seg.n > 1 && i < p.seg.n && p.seg.b[i] != nullptr);
-    return !bias && !p.act && p.R == nullptr;
+    for (int q = 0; q < 4; ++q)
+      if (n + q < p.N) v[q] = bf2f(b[n + q]);
+  }
+  return v;
+}
+__device__ __forceinline__ bool has_bias(const GemmParams& p, const TileCtx& t) {
+  bool bias = p.seg.n > 1 ? false : t.bias != nullptr;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) bias = bias || (p.seg.n > 1 && i < p.seg.n && p.seg.b[i] != nullptr);
+  return bias;
+}
+
+// Bias, then GELU, on a wave's accumulators of a plain store without residual,
+// so that its tile leaves by the bf16 staging below instead of the fp32 one
+// (twice the LDS bytes, two passes for a 256x256 tile). Group g (4 columns) of
+// tile i covers columns col0 + TSTEP i + GSTEP g. With the shorter GELU, the
+// vision tower's fc1 (M=2884, N=4304, K=1152) 46.9 -> 38.7 us, the tower of
+// three images 6000 -> 5770; its qkv (bias alone, 256x192 tiles) stayed at 31.4.
+template <int TSTEP, int GSTEP, int G, typename ACC, int TN, int TM>
+__device__ __forceinline__ void bias_act_acc(const GemmParams& p, const TileCtx& t, ACC (&c)[TN][TM], int col0) {
+  if (has_bias(p, t)) {
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        const floatx4 b = bias4(p, t, col0 + TSTEP * i + GSTEP * g);
+#pragma unroll
+        for (int j = 0; j < TM; ++j)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) c[i][j][4 * g + q] += b[q];
+      }
+  }
+  if (p.act) {
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int j = 0; j < TM; ++j)
+#pragma unroll
+        for (int q = 0; q < 4 * G; ++q) c[i][j][q] = gelu_tanh_fast(c[i][j][q]);
   }
 }
 
@@ -843,9 +894,11 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_dma_kernel(const GemmPa
     vm_wait<0>();  // the trailing zero-fill DMAs must land before the block's LDS is reused
 
     auto visit = [&](auto&& f) { visit_acc16<EPI, WTM, WTN, T16N, T16M>(a16, wm, wn, lane, f); };
-    if (epi_rounds_first<EPI>(p, tc))
+    if (epi_rounds_first<EPI>(p)) {
+      if constexpr (EPI == kEpiStore && !GROUPED)
+        bias_act_acc<16, 0, 1>(p, tc, a16, n0_out + wn * WTN + 4 * (lane >> 4));
       store_tile_lds_bf16<BM, BN_OUT, EPI, NW, kRing * 2, STREAM>(p, tc, visit, smem);
-    else if constexpr (EPI == kEpiStore || EPI == kEpiStoreF32)
+    } else if constexpr (EPI == kEpiStore || EPI == kEpiStoreF32)
       store_tile_lds<BM, BN_OUT, EPI, NW, kRing * 2>(p, tc, visit, reinterpret_cast<float*>(smem));
   } else {
   WaveAcc<TN, TM> acc;
@@ -1108,9 +1161,11 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_bf16_dma_kernel(const GemmPa
   vm_wait<0>();  // the trailing zero-fill DMAs must land before the block's LDS is reused
 
   auto visit = [&](auto&& f) { visit_acc32<EPI, WTM, WTN, TN, TM>(acc.c, wm, wn, lane, f); };
-  if (epi_rounds_first<EPI>(p, tc))
+  if (epi_rounds_first<EPI>(p)) {
+    if constexpr (EPI == kEpiStore && !GROUPED)
+      bias_act_acc<32, 8, 4>(p, tc, acc.c, n0_out + wn * WTN + 4 * (lane >> 5));
     store_tile_lds_bf16<BM, BN_OUT, EPI, NW, kRing * 2, STREAM>(p, tc, visit, smem);
-  else if constexpr (EPI == kEpiStore || EPI == kEpiStoreF32)
+  } else if constexpr (EPI == kEpiStore || EPI == kEpiStoreF32)
     store_tile_lds<BM, BN_OUT, EPI, NW, kRing * 2>(p, tc, visit, reinterpret_cast<float*>(smem));
   }  // 32x32x16 loop
 }

@@ -90,16 +90,17 @@ __device__ __forceinline__ float wave_max(float v) {
   for (int o = 32; o >= 1; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
   return v;
 }
-// gelu_tanh of the fused GEMM epilogue (vision fc1, patch mergers): tanh(u) =
-// 1 - 2 / (exp(2u) + 1) with the fast exponential and the hardware reciprocal
-// (absolute error ~1e-7 against tanhf, far below the bf16 rounding that
-// follows), instead of the libm tanhf the op-level kernel keeps. exp(2u)
-// overflowing to inf gives 1, underflowing to 0 gives -1.
+// gelu_tanh of the fused GEMM epilogue (vision fc1, patch mergers): 0.5 a (1 +
+// tanh(u)) = a / (1 + exp(-2u)), u = sqrt(2/pi) (a + 0.044715 a^3), with the
+// hardware exp2 and reciprocal instead of the libm tanhf the op-level kernel
+// keeps; one product, so large negative a keep their relative precision (as
+// 1 + tanh they cancelled: absolute error ~1e-7 a). exp2 overflowing to inf
+// gives a signed zero, underflowing to 0 gives a. 13 issue slots an element
+// instead of 20 (exp2 and rcp take four each); a tile's epilogue is bound by them.
 __device__ __forceinline__ float gelu_tanh_fast(float a) {
-  const float k0 = 0.7978845608028654f;
-  const float inner = k0 * (a + 0.044715f * a * a * a);
-  const float t = 1.0f - 2.0f * __builtin_amdgcn_rcpf(__expf(2.0f * inner) + 1.0f);
-  return 0.5f * a * (1.0f + t);
+  // -2 sqrt(2/pi) log2(e) and that times 0.044715
+  const float z = a * fmaf(a * a, -0.10294324f, -2.3022082f);
+  return a * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(z));
 }
 
 // silu(g) * u of the fused SwiGLU epilogues (GEMM tiles, decode GEMVs), in

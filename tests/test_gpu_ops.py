@@ -171,6 +171,29 @@ def test_decode_gemv_shapes(M):
                         bf16_round(bf16_round(d32) + f32(r)), what=f"decode down+residual M={M}")
 
 
+@pytest.mark.parametrize("M,N,K_", [(33, 20, 8), (65, 100, 64), (129, 257, 72), (300, 1003, 128), (777, 4304, 136),
+                                    (2884, 3456, 72), (1030, 6150, 2056)])
+def test_tile_epilogue_bias_and_gelu(M, N, K_):
+    """Bias, bias + GELU and biased segments of the tile GEMMs (more than 32 rows) at ragged edges of every tile
+    size, against fp64: one bf16 rounding (2^-8 of the value), the fp32 sums' error ((K + 4) 2^-24 of the sum of
+    absolute products) times GELU's slope (at most 1.13), and exp2's 2^-22 relative error in GELU's exponent."""
+    torch.manual_seed(7)
+    x, w, b = torch.randn(M, K_).bfloat16(), (torch.randn(N, K_) * K_ ** -0.5).bfloat16(), torch.randn(N).bfloat16()
+    z = x.double() @ w.double().t() + b.double()
+    mag = x.double().abs() @ w.double().abs().t() + b.double().abs()
+    gelu = torch.nn.functional.gelu(z, approximate="tanh")
+    xd, wd, bd = gpu(x), gpu(w), gpu(b)
+    cut = [16 * (N // 48), 16 * (N // 24)]
+    got = [(K.matmul(xd, wd, bd), z), (K.matmul_gelu(xd, wd, bd), gelu)]
+    parts = [(wd[i:j].contiguous(), bd[i:j].contiguous()) for i, j in ((0, cut[0]), (cut[0], cut[1]), (cut[1], N))]
+    parts = [q for q in parts if len(q[0])]
+    got.append((K.matmul_segments(xd, [q[0] for q in parts], [q[1] for q in parts]), z))
+    for y, ref in got:
+        tol = 2.0 ** -8 * ref.abs() + 1.13 * (K_ + 4) * 2.0 ** -24 * mag + 2.0 ** -19 * z.abs()
+        over = float(((y.cpu().double() - ref).abs() - tol).max())
+        assert over <= 0, over
+
+
 @pytest.mark.parametrize("M,ns,Kd,kind", [
     (9, (1024, 256, 256), 520, "bias"),    # X staged (one 16-row group), K tail inside a 32-step
     (3, (20000,), 1032, "residual"),       # X direct; 64-row blocks, more blocks than CUs
