@@ -6,6 +6,7 @@ from torch import nn
 
 from ..kernels import gelu_tanh, matmul_gelu, matmul_swiglu, rmsnorm_matmul_swiglu, swiglu
 from ..kernels.backward import needs_grad
+from ..kernels.matmul import line_padded_rows
 from .linear import CudaLinear
 from .norms import CudaRMSNorm, fused_norm_ok
 
@@ -52,4 +53,6 @@ class CudaVisionMLP(nn.Module):
     def forward(self, x: torch.Tensor, residual: torch.Tensor | None = None) -> torch.Tensor:
         if needs_grad(x, residual, *self.parameters()):  # training: modules/mlp.py:33-34 on differentiable ops
             return self.linear_fc2(gelu_tanh(self.linear_fc1(x)), residual=residual)
-        return self.linear_fc2(matmul_gelu(x, self.linear_fc1.weight, self.linear_fc1.bias), residual=residual)
+        w1 = self.linear_fc1.weight
+        h = matmul_gelu(x, w1, self.linear_fc1.bias, out=line_padded_rows(x, w1.shape[0]))
+        return self.linear_fc2(h, residual=residual)

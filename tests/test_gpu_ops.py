@@ -171,6 +171,23 @@ def test_decode_gemv_shapes(M):
                         bf16_round(bf16_round(d32) + f32(r)), what=f"decode down+residual M={M}")
 
 
+@pytest.mark.parametrize("lead,I", [((1, 5), 264), ((33,), 264), ((2, 150), 4304), ((40,), 256), ((40,), 20)])
+def test_gelu_rows_padded_to_whole_lines(lead, I):
+    """fc1 + GELU into rows padded to 128-byte lines and fc2 from them: the same bits as on plain rows; no padding
+    for few rows, whole lines or rows of odd pieces."""
+    from qwen3_5_vl_cuda_custom_amd.kernels.matmul import line_padded_rows
+    torch.manual_seed(8)
+    x, w1, b1 = gpu(torch.randn(*lead, 72).bfloat16()), gpu(torch.randn(I, 72).bfloat16()), gpu(torch.randn(I).bfloat16())
+    w2 = gpu(torch.randn(48, I).bfloat16())
+    out = line_padded_rows(x, I)
+    assert (out is not None) == (x.numel() // 72 > 32 and I % 64 != 0 and I % 8 == 0)
+    h = K.matmul_gelu(x, w1, b1, out=out)
+    if out is not None:
+        assert h.data_ptr() == out.data_ptr() and h.stride(-2) % 64 == 0
+    plain = K.matmul_gelu(x, w1, b1)
+    assert torch.equal(h, plain) and torch.equal(K.matmul(h, w2), K.matmul(plain, w2))
+
+
 @pytest.mark.parametrize("M,N,K_", [(33, 20, 8), (65, 100, 64), (129, 257, 72), (300, 1003, 128), (777, 4304, 136),
                                     (2884, 3456, 72), (1030, 6150, 2056)])
 def test_tile_epilogue_bias_and_gelu(M, N, K_):
