@@ -498,12 +498,13 @@ int q3_batched_gemm_backward(const void* x, const void* w, const void* dy, void*
  * reference differentiates its per-expert loop, modules/moe.py:70-83): out (T, H)
  * = sum over the token's experts, ascending, of bf16(bf16(swiglu) . down^T * w)
  * with a bf16 rounding per add; bf16, contiguous: x, grad_out (T, H), gate_up
- * (E, 2I, H), down (E, H, I), top_idx (T, k) int32 in [0, E), top_w (T, k). The
- * forward leaves what the backward reads in `state` (q3_moe_train_state_bytes).
- * Any of the gradients may be null. H and I multiples of 8, k <= 32, E < 2048,
- * T k < 2^20 and operands below 2 GiB (the byte queries return 0 otherwise);
- * state and workspace 256-byte aligned. Experts without tokens get zero
- * gradients. */
+ * (E, 2I, H), down (E, H, I), top_idx (T, k) int32, top_w (T, k). An id outside
+ * [0, E) (the top-k of a NaN row) is not dispatched: it adds nothing to out and
+ * to the gradients, and its grad_top_w is zero. The forward leaves what the
+ * backward reads in `state` (q3_moe_train_state_bytes). Any of the gradients may
+ * be null. H and I multiples of 8, k <= 32, E < 2048, T k < 2^20 and operands
+ * below 2 GiB (the byte queries return 0 otherwise); state and workspace
+ * 256-byte aligned. Experts without tokens get zero gradients. */
 int64_t q3_moe_train_state_bytes(int64_t T, int64_t H, int64_t I, int64_t E, int64_t k);
 int64_t q3_moe_train_workspace_bytes(int64_t T, int64_t H, int64_t I, int64_t E, int64_t k, int backward);
 int q3_moe_train_forward(const void* x, const void* gate_up, const void* down, const int* top_idx, const void* top_w,

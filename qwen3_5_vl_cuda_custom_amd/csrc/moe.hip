@@ -312,10 +312,11 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(const int* __restrict__ 
 
 // Wave per chunk: every (token, slot) entry of an expert gets the next row of
 // that expert's block, in (token, slot) order: the order of nonzero() on the
-// (T, k) routing matrix. Lane l of every wave holds token l's k expert ids in
-// registers and the chunk's histogram and start rows sit in LDS; the block's
-// waves split the experts, and per expert present in the chunk one ballot per
-// slot counts the entries of the lanes below.
+// (T, k) routing matrix. An id outside [0, E) gets no row: its pos_of entry is
+// -1 with mark_unplaced, else left as it is. Lane l of every wave holds token
+// l's k expert ids in registers and the chunk's histogram and start rows sit in
+// LDS; the block's waves split the experts, and per expert present in the chunk
+// one ballot per slot counts the entries of the lanes below.
 constexpr int kPlaceWaves = 8;  // waves per chunk; wave w places experts e = w (mod 8)
 
 template <int KMAX>
@@ -323,7 +324,7 @@ __global__ __launch_bounds__(kPlaceWaves * 64) void moe_place_kernel(const int* 
                                                        const bf16* __restrict__ top_w, int T, int k, int E,
                                                        const int* __restrict__ hist, const int* __restrict__ cstart,
                                                        int* __restrict__ sorted_token, bf16* __restrict__ sorted_w,
-                                                       int* __restrict__ pos_of) {
+                                                       int* __restrict__ pos_of, bool mark_unplaced) {
   extern __shared__ int s_row[];  // [0, E): the chunk's counts, [E, 2E): its start rows
   const int c = blockIdx.x, lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -360,14 +361,17 @@ __global__ __launch_bounds__(kPlaceWaves * 64) void moe_place_kernel(const int* 
       if (ex[s] == e) dst[s] = pos++;
   }
   // One store per slot and array, all lanes together (a slot's row was set
-  // by the wave that owns its expert).
+  // by the wave that owns its expert; wave 0 marks the entries without a row).
 #pragma unroll
-  for (int s = 0; s < KMAX; ++s)
+  for (int s = 0; s < KMAX; ++s) {
     if (dst[s] >= 0) {
       sorted_token[dst[s]] = t;
       sorted_w[dst[s]] = wv[s];
       pos_of[(int64_t)t * k + s] = dst[s];
+    } else if (mark_unplaced && wave == 0 && t < T && s < k && (ex[s] < 0 || ex[s] >= E)) {
+      pos_of[(int64_t)t * k + s] = -1;
     }
+  }
 }
 
 // One wave per token: add its k expert rows in ascending expert order.
@@ -762,7 +766,7 @@ int64_t moe_permute_ws_layout(int64_t T, int64_t E, int64_t k, MoeWs* ws, char* 
 // (token, slot) entry's row in expert-major, (token, slot)-ascending order
 // (the order of the reference's per-expert nonzero(), modules/moe.py:75).
 int moe_dispatch(const int* top_idx, const bf16* top_w, int64_t T, int64_t k, int64_t E, const MoeWs& w,
-                 hipStream_t st) {
+                 hipStream_t st, bool mark_unplaced = false) {
   const int NC = (int)q3_cdiv(T, kMoeChunk);
   hipLaunchKernelGGL(moe_hist_kernel, dim3((unsigned)NC), dim3(64), E * sizeof(int), st, top_idx, (int)T, (int)k,
                      (int)E, w.hist);
@@ -772,10 +776,10 @@ int moe_dispatch(const int* top_idx, const bf16* top_w, int64_t T, int64_t k, in
   const size_t place_lds = 2 * E * sizeof(int);
   if (k <= 8)
     hipLaunchKernelGGL(moe_place_kernel<8>, dim3((unsigned)NC), place_blk, place_lds, st, top_idx, top_w, (int)T,
-                       (int)k, (int)E, w.hist, w.cstart, w.sorted_token, w.sorted_w, w.pos_of);
+                       (int)k, (int)E, w.hist, w.cstart, w.sorted_token, w.sorted_w, w.pos_of, mark_unplaced);
   else
     hipLaunchKernelGGL(moe_place_kernel<32>, dim3((unsigned)NC), place_blk, place_lds, st, top_idx, top_w, (int)T,
-                       (int)k, (int)E, w.hist, w.cstart, w.sorted_token, w.sorted_w, w.pos_of);
+                       (int)k, (int)E, w.hist, w.cstart, w.sorted_token, w.sorted_w, w.pos_of, mark_unplaced);
   Q3_LAUNCH_CHECK();
   return Q3_OK;
 }
@@ -978,7 +982,9 @@ int launch_combine(const int* top_idx, const int* pos_of, const bf16* y_perm, co
 //             dgate_up[e] = dgu_e^T . x[token]_e    ddown[e] = dout[token]_e^T . aw_e
 // The products are grouped MFMA GEMMs on the weights as they are stored: dh
 // and dxp read an expert's matrix with the reduction as its rows, the weight
-// gradients reduce over an expert's row range (gemm_bwd.h). Bound by the
+// gradients reduce over an expert's row range (gemm_bwd.h). Entries whose id
+// lies outside [0, E) (the top-k of a NaN row) have no row: the dispatched
+// rows are the first offsets[E] of P, nothing is read of the others. Bound by the
 // weights: gate_up and down are read twice and their gradients written once.
 // Built as a loop over the experts from the single ops instead, every expert's
 // slice gradient filled and added a tensor of all experts: T = 2048, H = 2048,
@@ -1054,11 +1060,11 @@ int64_t moe_train_ws_layout(int64_t T, int64_t H, int64_t I, int64_t E, int64_t 
 // a = bf16(silu(g) u) of the (P, 2I) gate | up rows, 8 columns per thread.
 __device__ __forceinline__ float moe_act(float g, float u) { return g / (1.0f + expf(-g)) * u; }
 
-__global__ __launch_bounds__(256) void moe_act_kernel(const bf16* __restrict__ gu, bf16* __restrict__ act, int64_t P,
-                                                      int I) {
+__global__ __launch_bounds__(256) void moe_act_kernel(const bf16* __restrict__ gu, bf16* __restrict__ act,
+                                                      const int* __restrict__ n_rows, int I) {
   const int c8 = I / 8;
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= P * c8) return;
+  if (i >= (int64_t)*n_rows * c8) return;
   const int64_t row = i / c8;
   const int c = (int)(i - row * c8) * 8;
   const bf16x8 g = *reinterpret_cast<const bf16x8*>(gu + row * 2 * I + c);
@@ -1072,11 +1078,11 @@ __global__ __launch_bounds__(256) void moe_act_kernel(const bf16* __restrict__ g
 // One wave per row: dgu, aw and dw of the header above.
 __global__ __launch_bounds__(256) void moe_act_bwd_kernel(const bf16* __restrict__ gu, const bf16* __restrict__ dh,
                                                           const bf16* __restrict__ sorted_w, bf16* __restrict__ dgu,
-                                                          bf16* __restrict__ aw, float* __restrict__ dw, int64_t P,
-                                                          int I) {
+                                                          bf16* __restrict__ aw, float* __restrict__ dw,
+                                                          const int* __restrict__ n_rows, int I) {
   const int lane = threadIdx.x & 63;
   const int64_t row = ((int64_t)blockIdx.x * 256 + threadIdx.x) >> 6;
-  if (row >= P) return;
+  if (row >= *n_rows) return;
   const float w = bf2f(sorted_w[row]);
   float acc = 0.f;
   for (int c = lane * 8; c < I; c += 512) {
@@ -1105,10 +1111,11 @@ __global__ __launch_bounds__(256) void moe_act_bwd_kernel(const bf16* __restrict
 // Rows of two (T, H) matrices gathered by the sorted token list: xg = x[token], dog = dout[token].
 __global__ __launch_bounds__(256) void moe_gather2_kernel(const bf16* __restrict__ x, const bf16* __restrict__ dout,
                                                           const int* __restrict__ token, bf16* __restrict__ xg,
-                                                          bf16* __restrict__ dog, int64_t P, int H) {
+                                                          bf16* __restrict__ dog, const int* __restrict__ n_rows,
+                                                          int H) {
   const int c8 = H / 8;
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= P * c8) return;
+  if (i >= (int64_t)*n_rows * c8) return;
   const int64_t row = i / c8;
   const int c = (int)(i - row * c8) * 8;
   const int64_t src = (int64_t)token[row] * H + c, dst = row * H + c;
@@ -1380,13 +1387,13 @@ int q3_moe_train_forward(const void* x, const void* gate_up, const void* down, c
   d.sorted_token = s.sorted_token;
   d.sorted_w = s.sorted_w;
   d.pos_of = s.pos_of;
-  if ((rc = moe_dispatch(top_idx, static_cast<const bf16*>(top_w), T, k, E, d, st)) != Q3_OK) return rc;
+  if ((rc = moe_dispatch(top_idx, static_cast<const bf16*>(top_w), T, k, E, d, st, true)) != Q3_OK) return rc;
   if ((rc = launch_grouped<kEpiStore, false>(static_cast<const bf16*>(x), static_cast<const bf16*>(gate_up), s.gu,
                                              nullptr, P, 2 * I, H, s.sorted_token, T, s.tile_table, s.offsets,
                                              s.n_tiles, E, st)) != Q3_OK)
     return rc;
-  hipLaunchKernelGGL(moe_act_kernel, dim3((unsigned)q3_cdiv(P * (I / 8), 256)), dim3(256), 0, st, s.gu, w.act, P,
-                     (int)I);
+  hipLaunchKernelGGL(moe_act_kernel, dim3((unsigned)q3_cdiv(P * (I / 8), 256)), dim3(256), 0, st, s.gu, w.act,
+                     s.offsets + E, (int)I);
   Q3_LAUNCH_CHECK();
   if ((rc = launch_grouped<kEpiRowScale, false>(w.act, static_cast<const bf16*>(down), w.y_perm, s.sorted_w, P, H, I,
                                                 nullptr, 0, s.tile_table, s.offsets, s.n_tiles, E, st)) != Q3_OK)
@@ -1420,7 +1427,7 @@ int q3_moe_train_backward(const void* x, const void* gate_up, const void* down, 
                                             s.sorted_token, T, s.tile_table, s.offsets, s.n_tiles, E, st)) != Q3_OK)
     return rc;
   hipLaunchKernelGGL(moe_act_bwd_kernel, dim3((unsigned)q3_cdiv(P, 4)), dim3(256), 0, st, s.gu, w.dh, s.sorted_w,
-                     w.dgu, w.aw, w.dw, P, (int)I);
+                     w.dgu, w.aw, w.dw, s.offsets + E, (int)I);
   Q3_LAUNCH_CHECK();
   if (grad_x) {
     if ((rc = launch_grouped<kEpiStore, true>(w.dgu, static_cast<const bf16*>(gate_up), w.dxp, nullptr, P, H, 2 * I,
@@ -1434,7 +1441,7 @@ int q3_moe_train_backward(const void* x, const void* gate_up, const void* down, 
   }
   if (grad_gate_up || grad_down) {
     hipLaunchKernelGGL(moe_gather2_kernel, dim3((unsigned)q3_cdiv(P * (H / 8), 256)), dim3(256), 0, st,
-                       static_cast<const bf16*>(x), dout, s.sorted_token, w.xg, w.dog, P, (int)H);
+                       static_cast<const bf16*>(x), dout, s.sorted_token, w.xg, w.dog, s.offsets + E, (int)H);
     Q3_LAUNCH_CHECK();
   }
   if (grad_gate_up) {

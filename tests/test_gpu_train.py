@@ -718,6 +718,59 @@ def test_moe_training_gradients_are_reproducible_and_partial():
             assert torch.equal(a, b) if i in which else a is None
 
 
+def test_moe_training_leaves_out_ids_that_are_no_experts():
+    """Ids outside [0, E) (a NaN router row's top-k gives 0x7fffffff) are not dispatched: no output, no gradient and
+    nothing read for them, whatever the state's memory held before (zeros here: an entry taken from it would name row
+    0). Against the loop over the experts in fp32; a slot's product rounds its ~6 bf16 intermediates (a layer's bounds)."""
+    from qwen3_5_vl_cuda_custom_amd import _lib
+    from qwen3_5_vl_cuda_custom_amd.kernels.moe_routing import moe_experts_train
+    T, H, I, E, k = 150, 128, 64, 6, 2
+    x, gu, dn = (rnd(*s, seed=i, std=0.3).bfloat16() for i, s in enumerate([(T, H), (E, 2 * I, H), (E, H, I)]))
+    idx = torch.stack([torch.randperm(E, generator=torch.Generator().manual_seed(t))[:k] for t in range(T)])
+    idx[3] = 0x7fffffff
+    idx[70, 1], idx[149, 0], idx[149, 1] = -1, E, 2
+    w, dy = torch.rand(T, k, generator=torch.Generator().manual_seed(4)).bfloat16(), rnd(T, H, seed=5).bfloat16()
+
+    def loop(x, gu, dn, w):
+        out = torch.zeros(T, H)
+        for e in range(E):
+            t, s = (idx == e).nonzero(as_tuple=True)
+            g, u = (x[t] @ gu[e].t()).chunk(2, dim=-1)
+            out = out.index_add(0, t, (F.silu(g) * u @ dn[e].t()) * w[t, s, None])
+        return out
+
+    def block(x, gu, dn, w):
+        before = torch.zeros(_lib.lib().q3_moe_train_state_bytes(T, H, I, E, k), dtype=torch.uint8, device=DEV)
+        del before
+        return moe_experts_train(x, gu, dn, idx.to(DEV), w)
+
+    out, got = run_grads(block, (x, gu, dn, w), dy)
+    ref_out, ref = ref_grads(loop, (x, gu, dn, w), dy)
+    for a, b, n in zip((out, *got), (ref_out, *ref), ("out", "dx", "dgate_up", "ddown", "dw")):
+        assert_grad_close(a, b, n, max_rel=5e-2, mean_rel=1.5e-2)
+    assert not out[3].any() and not got[0][3].any()
+    assert not got[3][3].any() and not got[3][70, 1] and not got[3][149, 0]
+
+
+def test_moe_block_trains_past_a_nan_token():
+    """One token of NaN: its expert part is zero, the other tokens' outputs and the experts' weight gradients are those
+    of the block without it (the same rows and tiles: equal up to the order of sums, one bf16 rounding)."""
+    from qwen3_5_vl_cuda_custom_amd.modules import CudaSparseMoE
+    torch.manual_seed(0)
+    T, bad = 80, 7
+    moe = CudaSparseMoE(hidden_size=128, moe_intermediate_size=64, num_experts=8, top_k=2).to(DEV).bfloat16()
+    x, dy = rnd(1, T, 128, seed=91).bfloat16(), rnd(1, T, 128, seed=92).bfloat16()
+    keep = torch.arange(T) != bad
+    ref_y, _, ref = _module_grads(moe, lambda m, t: m(t)[0], x[:, keep], dy[:, keep])
+    moe.zero_grad()
+    x[0, bad] = float("nan")
+    y, _, got = _module_grads(moe, lambda m, t: m(t)[0], x, dy)
+    assert not y[0, bad].any()
+    assert_grad_close(y[0, keep], ref_y[0], "other tokens' outputs", max_rel=2.0 ** -7, mean_rel=2.0 ** -8)
+    for n in ("gate_up_proj", "down_proj"):
+        assert_grad_close(got[n], ref[n], n, max_rel=2.0 ** -7, mean_rel=2.0 ** -8)
+
+
 def test_vision_block_trains_like_the_oracle():
     from oracle import layers as L
     from qwen3_5_vl_cuda_custom_amd.modules import CudaVisionBlock
