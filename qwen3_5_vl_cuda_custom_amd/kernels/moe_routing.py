@@ -5,7 +5,7 @@ from __future__ import annotations
 import torch
 
 from .. import _lib
-from ._common import check, mfma_operand, note_slow_path
+from ._common import check, mfma_operand, note_slow_path, require_device, require_same_dtype
 from .backward import MoEExpertsFunction, BatchedGemmFunction, IndexAddFunction, TopKFunction, needs_grad
 
 
@@ -130,6 +130,24 @@ def moe_router(x: torch.Tensor, gate_weight: torch.Tensor, top_k: int, norm_topk
     return logits, idx, w
 
 
+def _expert_shapes(op: str, x, gate_up, down, top_idx, top_w, idx_dtypes) -> tuple[int, int, int, int, int]:
+    """(T, H, I, E, k) of the routed experts' operands, or the error of the first that does not fit."""
+    if x.dim() != 2 or gate_up.dim() != 3 or down.dim() != 3:
+        raise ValueError(f"{op}: x (T, H), gate_up (E, 2I, H), down (E, H, I)")
+    T, H = x.shape
+    E, I2, _ = gate_up.shape
+    I = I2 // 2
+    if gate_up.shape[2] != H or tuple(down.shape) != (E, H, I) or I2 % 2:
+        raise ValueError(f"{op}: gate_up {tuple(gate_up.shape)} / down {tuple(down.shape)} do not match H={H}")
+    if top_idx.dtype not in idx_dtypes or not top_idx.is_cuda or top_idx.dim() != 2 or top_idx.shape[0] != T:
+        raise ValueError(f"{op}: top_idx must be a (T={T}, k) device tensor of {idx_dtypes}, got {top_idx.dtype} "
+                         f"{tuple(top_idx.shape)} on {top_idx.device}")
+    k = top_idx.shape[1]
+    if tuple(top_w.shape) != (T, k):
+        raise ValueError(f"{op}: top_w must be ({T}, {k}), got {tuple(top_w.shape)}")
+    return T, H, I, E, k
+
+
 def moe_experts(x: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, top_idx: torch.Tensor,
                 top_w: torch.Tensor, residual: torch.Tensor | None = None) -> torch.Tensor:
     """Dispatch, per-expert SwiGLU MLPs and combine (modules/moe.py:70-83) for routed tokens.
@@ -138,20 +156,7 @@ def moe_experts(x: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, top_
     top_w (T, k) bf16. Returns (T, H) (+ residual).
     """
     check("moe_experts", x, gate_up, down, top_w, residual)
-    if x.dim() != 2 or gate_up.dim() != 3 or down.dim() != 3:
-        raise ValueError("moe_experts: x (T, H), gate_up (E, 2I, H), down (E, H, I)")
-    T, H = x.shape
-    E, I2, _ = gate_up.shape
-    I = I2 // 2
-    if gate_up.shape[2] != H or tuple(down.shape) != (E, H, I) or I2 % 2:
-        raise ValueError(f"moe_experts: gate_up {tuple(gate_up.shape)} / down {tuple(down.shape)} do not match "
-                         f"H={H}")
-    if top_idx.dtype != torch.int32 or not top_idx.is_cuda or top_idx.dim() != 2 or top_idx.shape[0] != T:
-        raise ValueError(f"moe_experts: top_idx must be an int32 (T={T}, k) device tensor, got {top_idx.dtype} "
-                         f"{tuple(top_idx.shape)}")
-    k = top_idx.shape[1]
-    if tuple(top_w.shape) != (T, k):
-        raise ValueError(f"moe_experts: top_w must be ({T}, {k}), got {tuple(top_w.shape)}")
+    T, H, I, E, k = _expert_shapes("moe_experts", x, gate_up, down, top_idx, top_w, (torch.int32,))
     if residual is not None and tuple(residual.shape) != (T, H):
         raise ValueError(f"moe_experts: residual must be ({T}, {H})")
     x = x.contiguous()
@@ -169,15 +174,13 @@ def moe_experts_train(x: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor
                       top_w: torch.Tensor) -> torch.Tensor | None:
     """moe_experts with a backward (x, gate_up, down and top_w), every expert in a few grouped launches; None where it
     does not cover the operands (fp32, widths that are no multiple of 8, unaligned views, 2 GiB and more): the caller
-    then runs the experts one by one on the single ops. top_idx (T, k), distinct experts in [0, E) per token."""
-    ts = (x, gate_up, down, top_w)
-    T, H = x.shape
-    E, I2, _ = gate_up.shape
-    k = top_idx.shape[1]
-    if (not all(t.is_cuda and t.dtype == torch.bfloat16 for t in ts) or gate_up.shape[2] != H or I2 % 2
-            or tuple(down.shape) != (E, H, I2 // 2) or tuple(top_w.shape) != (T, k)
-            or any(t.data_ptr() % 16 for t in ts[:3])
-            or _lib.lib().q3_moe_train_state_bytes(T, H, I2 // 2, E, k) == 0):
+    then runs the experts one by one on the single ops. top_idx (T, k) int32 or int64, distinct experts per token;
+    ids outside [0, E) are left out, in the output and in every gradient."""
+    require_device("moe_experts_train", x, gate_up, down, top_w)
+    require_same_dtype("moe_experts_train", x, gate_up, down, top_w)
+    T, H, I, E, k = _expert_shapes("moe_experts_train", x, gate_up, down, top_idx, top_w, (torch.int32, torch.int64))
+    if (x.dtype != torch.bfloat16 or any(t.data_ptr() % 16 for t in (x, gate_up, down))
+            or _lib.lib().q3_moe_train_state_bytes(T, H, I, E, k) == 0):
         return None
     return MoEExpertsFunction.apply(x, gate_up, down, top_idx.to(torch.int32), top_w)
 

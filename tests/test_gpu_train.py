@@ -752,6 +752,25 @@ def test_moe_training_leaves_out_ids_that_are_no_experts():
     assert not got[3][3].any() and not got[3][70, 1] and not got[3][149, 0]
 
 
+def test_moe_training_checks_its_operands():
+    """What the inference entry refuses (routing on the host, other shapes, mixed types) is refused before a launch."""
+    from qwen3_5_vl_cuda_custom_amd.kernels.moe_routing import moe_experts_train
+    T, H, I, E, k = 6, 64, 32, 4, 2
+    x, gu, dn, w = (torch.zeros(*s, device=DEV, dtype=torch.bfloat16) for s in ((T, H), (E, 2 * I, H), (E, H, I),
+                                                                                 (T, k)))
+    idx = torch.tensor([[0, 1]] * T, device=DEV)
+    assert moe_experts_train(x, gu, dn, idx, w).shape == (T, H)
+    for bad in ((x, gu, dn, idx.cpu(), w), (x, gu, dn, idx[:4], w[:4]), (x, gu, dn, idx[:4], w), (x, gu, dn, idx, w[:4]),
+                (x, gu, dn, idx.float(), w), (x, gu, dn, idx[:, 0], w), (x, gu[:, :, :32], dn, idx, w),
+                (x, gu, dn[:3], idx, w), (x[0], gu, dn, idx, w)):
+        with pytest.raises(ValueError):
+            moe_experts_train(*bad)
+    with pytest.raises(RuntimeError):
+        moe_experts_train(x, gu, dn, idx, w.cpu())
+    with pytest.raises(TypeError):
+        moe_experts_train(x, gu.float(), dn, idx, w)
+
+
 def test_moe_block_trains_past_a_nan_token():
     """One token of NaN: its expert part is zero, the other tokens' outputs and the experts' weight gradients are those
     of the block without it (the same rows and tiles: equal up to the order of sums, one bf16 rounding)."""
