@@ -570,7 +570,8 @@ struct MoeGemvP {
 // weights through a private LDS ring of kRing stages (16 rows x 128 k, 4 KB) by
 // non-temporal direct-to-LDS loads that run on across units, no barrier in
 // between; the halves (and gate and up) meet in LDS once per unit, two buffers
-// in turn. Chunk c of a stage row r sits at slot c ^ r (conflict-free fragment
+// in turn. A stage is issued into the slot that the step before has read, so the
+// issue first waits for that step's LDS reads (its MFMAs wait for them as well). Chunk c of a stage row r sits at slot c ^ r (conflict-free fragment
 // reads). SPLIT false (K <= 1024, plain): a unit is 64 rows, each wave takes 16
 // of them over all of K and stores them alone, with no exchange or barrier.
 // Bound by the weight stream: 16
@@ -604,6 +605,7 @@ __global__ __launch_bounds__(256) void moe_gemv_kernel(const MoeGemvP p) {
     const int r0 = SWIGLU ? (grp ? N : 0) + 16 * ig : kUnit * ig + 16 * grp;
     const int rlim = (SWIGLU ? 16 * ig : r0) + 16 <= N ? 16 : N - (SWIGLU ? 16 * ig : r0);  // live rows (may be <= 0)
     const uint32_t dst = lring + (uint32_t)(slot_i * kStage * 2);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the slot's last fragment reads have returned
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int r = 4 * i + lrow, k = kbeg + is * 128 + ((l16 ^ r) << 3);
