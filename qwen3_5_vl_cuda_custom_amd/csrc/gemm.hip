@@ -355,21 +355,27 @@ int launch_tiled(GemmParams p, int64_t batch, hipStream_t st) {
 // 256x256 tiles would leave most CUs idle and whose fallback, the one-wave
 // 128x128 ring, is bound by each CU's operand stream over a long K (M=1024,
 // N=4096, K=12288: 6.3 MB per tile, 135 us) runs as S splits of 256x256 tiles
-// (the tile GEMM's batch dimension: split z reads X and W columns
-// [z K/S, (z + 1) K/S) and writes fp32 partial plane z), then one kernel sums
-// the planes in split order, adds bias and residual and rounds once, the
+// (the tile GEMM's batch dimension: split z takes k from z L to min(K, (z + 1) L)
+// with L = split_k_len(K, S) and writes fp32 partial plane z), then one kernel
+// sums the planes in split order, adds bias and residual and rounds once, the
 // order of the unsplit epilogue. Chosen by estimates from measured rates: a
 // wave of 256x256 tiles takes ~9.8 + 0.0243 K us, +4 us for an fp32 epilogue;
 // the 128x128 ring ~0.45 of that at full K; the reduction moves its bytes
 // (planes, residual, output) at ~5 TB/s after a ~4 us launch (the estimate
 // counts a residual, so the plan and workspace size depend on M, N, K only). The partial planes follow the GEMM
 // workspace's 16 KiB counter region, which they never touch.
+//
+// The forward splits only into equal runs of whole 64-wide stages. A shorter
+// last split would serve the vision block's fc2 (N=1152, K=4304; 784 rows 33 us
+// against 42 unsplit, 36 on padded rows), but a tower of so few rows is bound
+// by its launches (27 more), and its fc2 would then write the workspace that
+// every stream's calls share.
 constexpr int64_t kSplitWsOffset = 16 << 10;
 
 // Columns per split: whole 64-wide stages, the last split the rest.
 int64_t split_k_len(int64_t K, int64_t s) { return q3_cdiv(q3_cdiv(K, s), 64) * 64; }
 
-int split_k_plan(int64_t M, int64_t N, int64_t K) {
+int split_k_plan(int64_t M, int64_t N, int64_t K, bool equal) {
   if (M <= kGemvMaxRows || K < 2048 || M >= (1 << 20) || N >= (1 << 20)) return 1;
   const int64_t tiles_a = q3_cdiv(M, 256) * q3_cdiv(N, 256);
   if (q3_cdiv(M, 128) * q3_cdiv(N, 128) > 256) return 1;  // not the one-wave 128x128 case
@@ -378,7 +384,7 @@ int split_k_plan(int64_t M, int64_t N, int64_t K) {
   double t_best = t_c;
   for (int s = 2; s <= 8; s *= 2) {
     const int64_t ks = split_k_len(K, s);
-    if (tiles_a * s > 256 || ks * (s - 1) >= K) continue;
+    if (tiles_a * s > 256 || ks * (s - 1) >= K || (equal && ks * s != K)) continue;
     const double bytes = (double)s * M * N * 4 + (double)M * N * 4;  // planes, residual in, C out
     const double t = 9.8 + 0.0243 * (double)ks + 4.0 + bytes / 5e6 + 4.0;
     if (t < t_best) {
@@ -389,8 +395,8 @@ int split_k_plan(int64_t M, int64_t N, int64_t K) {
   return best;
 }
 
-int64_t split_k_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-  const int s = split_k_plan(M, N, K);
+int64_t split_k_workspace_bytes(int64_t M, int64_t N, int64_t K, bool equal) {
+  const int s = split_k_plan(M, N, K, equal);
   return s > 1 ? kSplitWsOffset + (int64_t)s * M * N * 4 : 0;
 }
 
@@ -555,8 +561,8 @@ int matmul_impl(const void* x, const void* w, const void* w2, const void* bias, 
   p.bsC = bsC;
   p.act = act;
   if (!swiglu && !act && batch == 1) {
-    const int S = split_k_plan(M, N, K);
-    if (S > 1 && ws != nullptr && q3_aligned(ws, 16) && ws_bytes >= split_k_workspace_bytes(M, N, K))
+    const int S = split_k_plan(M, N, K, true);
+    if (S > 1 && ws != nullptr && q3_aligned(ws, 16) && ws_bytes >= split_k_workspace_bytes(M, N, K, true))
       return launch_split_k(p, S, ws, st);
   }
   return swiglu ? launch_tiled<kEpiSwiGLU>(p, batch, st) : launch_tiled<kEpiStore>(p, batch, st);
@@ -672,7 +678,7 @@ bool gemm_t_ok(const void* x, const void* w, int64_t M, int64_t N, int64_t K, bo
          (K + 64) * N * 2 < (1ll << 31) && ((xt ? K : M) + 256) * (xt ? M : K) * 2 < (1ll << 31);
 }
 
-int64_t gemm_t_workspace_bytes(int64_t M, int64_t N, int64_t K) { return split_k_workspace_bytes(M, N, K); }
+int64_t gemm_t_workspace_bytes(int64_t M, int64_t N, int64_t K) { return split_k_workspace_bytes(M, N, K, false); }
 
 template <bool XT>
 static int gemm_t(const void* x, const void* w, void* y, int64_t M, int64_t N, int64_t K, void* ws, int64_t ws_bytes,
@@ -687,8 +693,8 @@ static int gemm_t(const void* x, const void* w, void* y, int64_t M, int64_t N, i
   p.ldx = XT ? M : K;
   p.ldw = N;
   p.ldc = N;
-  const int S = split_k_plan(M, N, K);
-  if (S > 1 && ws != nullptr && q3_aligned(ws, 16) && ws_bytes >= split_k_workspace_bytes(M, N, K))
+  const int S = split_k_plan(M, N, K, false);
+  if (S > 1 && ws != nullptr && q3_aligned(ws, 16) && ws_bytes >= split_k_workspace_bytes(M, N, K, false))
     return launch_split_k<XT, true>(p, S, ws, st);
   return launch_tiled_t<XT, true>(p, 1, st);
 }
@@ -755,7 +761,7 @@ int q3_matmul_segments(const void* x, const void* const* w, const void* const* b
 
 int64_t q3_matmul_workspace_bytes(int64_t M, int64_t N, int64_t K, int dtype, int swiglu) {
   if (dtype != Q3_BF16 || M <= 0 || N <= 0 || K <= 0) return 0;
-  if (M > kGemvMaxRows) return swiglu ? 0 : split_k_workspace_bytes(M, N, K);
+  if (M > kGemvMaxRows) return swiglu ? 0 : split_k_workspace_bytes(M, N, K, true);
   return gemv_workspace_bytes(M, N, K, swiglu != 0);
 }
 

@@ -64,6 +64,10 @@ def test_matmul_validation():
     assert L.q3_matmul_workspace_bytes(1024, 4096, 4096, 1, 0) == 0
     assert L.q3_matmul_workspace_bytes(4096, 4096, 12288, 1, 0) == 0
     assert L.q3_matmul_workspace_bytes(1024, 4096, 12288, 1, 1) == 0  # SwiGLU: never split
+    # a K that has no equal splits of whole 64-wide stages (the vision block's fc2) runs unsplit, without a workspace
+    for rows in (33, 256, 784, 1500):
+        assert L.q3_matmul_workspace_bytes(rows, 1152, 4304, 1, 0) == 0
+    assert L.q3_matmul_workspace_bytes(1024, 4096, 12352, 1, 0) == 0
     assert L.q3_matmul_workspace_bytes(8, 4096, 20480, 1, 0) == 0
     ws = L.q3_matmul_workspace_bytes(32, 4096, 20480, 1, 0)
     assert ws > 0

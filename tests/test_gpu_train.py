@@ -291,9 +291,10 @@ def test_matmul_backward_untransposed_against_transposed(M, N, K_):
 
 @pytest.mark.parametrize("M,N,K_", [(1024, 4096, 12352), (512, 2048, 8256)])
 def test_matmul_split_with_shorter_last_split(M, N, K_):
-    """A K that no split count divides into whole 64-wide stages: the last split is shorter. Outputs reach |11|, where
-    half a bf16 step is 0.031: the bound is one rounding of each value (2^-8 of it) plus the fp32 sums' order (2^-16 of
-    the largest), not the fixed 0.02 of unit-sized outputs."""
+    """A K that no split count divides into whole 64-wide stages: the forward runs it unsplit (the backward's products
+    split such a reduction: test_matmul_backward_untransposed_against_transposed). Outputs reach |11|, where half a
+    bf16 step is 0.031: the bound is one rounding of each value (2^-8 of it) plus the fp32 sums' order (2^-16 of the
+    largest), not the fixed 0.02 of unit-sized outputs."""
     x, w = rnd(M, K_, seed=44).bfloat16(), rnd(N, K_, seed=45, std=0.02).bfloat16()
     got, ref = K.matmul(x.to(DEV), w.to(DEV)).float().cpu(), O.linear(x.float(), w.float())
     over = float(((got - ref).abs() - 2.0 ** -8 * ref.abs() - 2.0 ** -16 * ref.abs().max()).max())
