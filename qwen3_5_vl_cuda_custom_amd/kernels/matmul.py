@@ -91,13 +91,16 @@ def matmul_gelu(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None
         x2 = x2.contiguous()
     w = weight if weight.stride(-1) == 1 else weight.contiguous()
     x2, w = _gemm_rows("matmul_gelu", K, x2, w)
-    y = out if out is not None else torch.empty((*x.shape[:-1], N), dtype=x.dtype, device=x.device)
-    if y.shape != (*x.shape[:-1], N) or y.stride(-1) != 1:
-        raise ValueError(f"matmul_gelu: out {tuple(y.shape)} must be {(*x.shape[:-1], N)} with contiguous elements")
-    y2 = y.view(-1, N)
+    if out is None:
+        y, ldc = torch.empty((*x.shape[:-1], N), dtype=x.dtype, device=x.device), N
+    else:
+        if out.shape != (*x.shape[:-1], N) or out.stride(-1) != 1:
+            raise ValueError(f"matmul_gelu: out {tuple(out.shape)} must be {(*x.shape[:-1], N)} with contiguous "
+                             "elements")
+        y, ldc = out, out.view(-1, N).stride(0)
     b = bias.contiguous() if bias is not None else None
-    _lib.call("q3_matmul_gelu", x2.data_ptr(), w.data_ptr(), _lib.ptr(b), y2.data_ptr(), x2.shape[0], N, K,
-              x2.stride(0), w.stride(0), y2.stride(0), _lib.dtype_code(x.dtype), _lib.stream())
+    _lib.call("q3_matmul_gelu", x2.data_ptr(), w.data_ptr(), _lib.ptr(b), y.data_ptr(), x2.shape[0], N, K,
+              x2.stride(0), w.stride(0), ldc, _lib.dtype_code(x.dtype), _lib.stream())
     return y
 
 

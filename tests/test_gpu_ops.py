@@ -188,6 +188,21 @@ def test_gelu_rows_padded_to_whole_lines(lead, I):
     assert torch.equal(h, plain) and torch.equal(K.matmul(h, w2), K.matmul(plain, w2))
 
 
+@pytest.mark.parametrize("lead", [(1, 784), (3, 511), (3, 512), (1, 1537)])
+def test_vision_mlp_pads_only_many_rows(lead, monkeypatch):
+    """The vision MLP's hidden rows are padded from PAD_ROWS rows on and plain below; the same bits either way."""
+    from qwen3_5_vl_cuda_custom_amd.modules import CudaVisionMLP, mlp
+    torch.manual_seed(9)
+    m = gpu(CudaVisionMLP(72, 264).bfloat16()).requires_grad_(False)
+    x = gpu(torch.randn(*lead, 72).bfloat16())
+    outs = []
+    monkeypatch.setattr(mlp, "matmul_gelu", lambda *a, out=None: outs.append(out) or K.matmul_gelu(*a, out=out))
+    y = m(x)
+    assert [o is not None for o in outs] == [lead[0] * lead[1] >= mlp.PAD_ROWS]
+    h = K.matmul_gelu(x, m.linear_fc1.weight, m.linear_fc1.bias)
+    assert torch.equal(y, m.linear_fc2(h))
+
+
 @pytest.mark.parametrize("M,N,K_", [(33, 20, 8), (65, 100, 64), (129, 257, 72), (300, 1003, 128), (777, 4304, 136),
                                     (2884, 3456, 72), (1030, 6150, 2056)])
 def test_tile_epilogue_bias_and_gelu(M, N, K_):
