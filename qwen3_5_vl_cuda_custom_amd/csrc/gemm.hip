@@ -369,14 +369,21 @@ int launch_tiled(GemmParams p, int64_t batch, hipStream_t st) {
 // last split would serve the vision block's fc2 (N=1152, K=4304; 784 rows 33 us
 // against 42 unsplit, 36 on padded rows), but a tower of so few rows is bound
 // by its launches (27 more), and its fc2 would then write the workspace that
-// every stream's calls share.
+// every stream's calls share. At most 32 rows are the GEMVs' there.
+//
+// The backward's products (equal = false) split into any whole stages and at
+// any row count, since no GEMV takes an untransposed operand: a dX of few rows
+// is otherwise a few tiles, each walking the whole reduction. dX at 16 rows,
+// unsplit -> split, us (transposing W for the GEMV): N=4304, K=1152 26 -> 17
+// (19), N=3456, K=1152 22 -> 15 (15), N=K=4096 25 -> 18 (30), N=12288, K=4096
+// 67 -> 30 (71), N=151936, K=4096 963 -> 283 (1260).
 constexpr int64_t kSplitWsOffset = 16 << 10;
 
 // Columns per split: whole 64-wide stages, the last split the rest.
 int64_t split_k_len(int64_t K, int64_t s) { return q3_cdiv(q3_cdiv(K, s), 64) * 64; }
 
 int split_k_plan(int64_t M, int64_t N, int64_t K, bool equal) {
-  if (M <= kGemvMaxRows || K < 2048 || M >= (1 << 20) || N >= (1 << 20)) return 1;
+  if ((equal && M <= kGemvMaxRows) || K < 2048 || M >= (1 << 20) || N >= (1 << 20)) return 1;
   const int64_t tiles_a = q3_cdiv(M, 256) * q3_cdiv(N, 256);
   if (q3_cdiv(M, 128) * q3_cdiv(N, 128) > 256) return 1;  // not the one-wave 128x128 case
   const double t_c = 0.45 * (9.8 + 0.0243 * (double)K);

@@ -68,6 +68,9 @@ def test_matmul_validation():
     for rows in (33, 256, 784, 1500):
         assert L.q3_matmul_workspace_bytes(rows, 1152, 4304, 1, 0) == 0
     assert L.q3_matmul_workspace_bytes(1024, 4096, 12352, 1, 0) == 0
+    # the backward's products split at any row count: dX of 16 rows of the vocabulary head in 8 planes
+    for rows in (1, 16, 32, 33):
+        assert L.q3_matmul_backward_gemm_workspace_bytes(rows, 151936, 4096, 1) >= (16 << 10) + 8 * rows * 4096 * 4
     assert L.q3_matmul_workspace_bytes(8, 4096, 20480, 1, 0) == 0
     ws = L.q3_matmul_workspace_bytes(32, 4096, 20480, 1, 0)
     assert ws > 0

@@ -271,10 +271,12 @@ def test_matmul_backward_odd_rows_bf16(M, N, K_):
 
 
 @pytest.mark.parametrize("M,N,K_", [(1, 8, 8), (63, 136, 264), (64, 264, 136), (65, 520, 248), (129, 1032, 776),
-                                    (300, 4096, 1160), (40, 8192, 512), (1000, 512, 2056), (33, 40, 16456)])
+                                    (300, 4096, 1160), (40, 8192, 512), (1000, 512, 2056), (33, 40, 16456),
+                                    (1, 4304, 1152), (2, 8208, 40), (17, 4104, 520), (32, 3456, 264),
+                                    (4104, 24, 520), (2056, 8, 264), (4097, 264, 136)])
 def test_matmul_backward_untransposed_against_transposed(M, N, K_):
     """dX and dW on the operands as they are (tile edges in every dimension, the three tile shapes, splits over K with
-    a shorter last split) against q3_matmul on transposed copies, which sums each element's products in fp32 too: the
+    a shorter last split, also of products of at most 32 rows) against q3_matmul on transposed copies, which sums each element's products in fp32 too: the
     two may differ by one bf16 rounding of the element (2^-7) and the fp32 sums' order (2^-16 of the largest)."""
     x, w, dy = (rnd(M, K_, seed=44).bfloat16().to(DEV), rnd(N, K_, seed=45, std=0.1).bfloat16().to(DEV),
                 rnd(M, N, seed=47).bfloat16().to(DEV))
