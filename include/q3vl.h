@@ -475,12 +475,18 @@ int q3_transpose(const void* a, void* b, int64_t E, int64_t R, int64_t C, int dt
  * and multiplied by q3_matmul, which may
  * use `gemm_ws` as q3_matmul's workspace (zero-filled before first use, as
  * there; size at least q3_matmul_workspace_bytes of both products;
- * q3_matmul_backward_gemm_workspace_bytes also covers the split form of the
- * products on untransposed operands and the padded row count of the others). */
+ * q3_matmul_backward_gemm_workspace_bytes also covers the padded row count).
+ * Operands that are multiplied as they are need no gemm_ws
+ * (q3_matmul_backward_gemm_workspace_bytes_for is 0): the fp32 planes of a
+ * product split over K lie in a `workspace` of the _for size, so backward passes
+ * on several streams share nothing; with a smaller one they go to gemm_ws if
+ * that holds them, else the product runs unsplit. */
 int64_t q3_matmul_backward_workspace_bytes(int64_t M, int64_t N, int64_t K, int dtype);
 int64_t q3_matmul_backward_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int dtype);
 int64_t q3_matmul_backward_workspace_bytes_for(const void* x, const void* w, const void* dy, int64_t M, int64_t N,
                                                int64_t K, int dtype);
+int64_t q3_matmul_backward_gemm_workspace_bytes_for(const void* x, const void* w, const void* dy, int64_t M, int64_t N,
+                                                    int64_t K, int dtype);
 int q3_matmul_backward(const void* x, const void* w, const void* dy, void* gx, void* gw, void* gb, int64_t M,
                        int64_t N, int64_t K, int dtype, void* workspace, int64_t workspace_bytes, void* gemm_ws,
                        int64_t gemm_ws_bytes, void* stream);

@@ -97,6 +97,7 @@ _SIGS: dict[str, tuple] = {
     "q3_matmul_backward_workspace_bytes": (c_int64, [_I, _I, _I, c_int]),
     "q3_matmul_backward_gemm_workspace_bytes": (c_int64, [_I, _I, _I, c_int]),
     "q3_matmul_backward_workspace_bytes_for": (c_int64, [_V, _V, _V, _I, _I, _I, c_int]),
+    "q3_matmul_backward_gemm_workspace_bytes_for": (c_int64, [_V, _V, _V, _I, _I, _I, c_int]),
     "q3_matmul_backward": (c_int, [_V, _V, _V, _V, _V, _V, _I, _I, _I, c_int, _V, _I, _V, _I, _V]),
     "q3_batched_gemm_backward_workspace_bytes": (c_int64, [_I, _I, _I, _I, c_int]),
     "q3_batched_gemm_backward": (c_int, [_V, _V, _V, _V, _V, _I, _I, _I, _I, c_int, _V, _I, _V]),
@@ -194,7 +195,9 @@ def workspace(nbytes: int, device: torch.device) -> tuple[torch.Tensor | None, i
 # planes lie behind them). A larger request allocates a new buffer; the old
 # ones are kept, because captured HIP graphs may still point at them. Calls on
 # different streams that run at the same time must not share one: these serve
-# stream-ordered work (a layer's GEMMs, the decode step).
+# stream-ordered work (a layer's GEMMs, the decode step). The backward's products
+# on untransposed operands do not use them (their planes lie in the call's own
+# workspace).
 _gemm_ws: dict[tuple[str, int | None], list[torch.Tensor]] = {}
 
 

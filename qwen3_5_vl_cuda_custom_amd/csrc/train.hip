@@ -916,6 +916,13 @@ bool mm_bwd_direct_x(const void* w, const void* dy, int64_t M, int64_t N, int64_
 bool mm_bwd_direct_w(const void* x, const void* dy, int64_t M, int64_t N, int64_t K, int dtype) {
   return dtype == Q3_BF16 ? q3::gemm_t_ok(dy, x, N, K, M, true) : q3::gemm_f32_t_ok(dy, N, M, true);
 }
+bool mm_bwd_direct(const void* x, const void* w, const void* dy, int64_t M, int64_t N, int64_t K, int dtype) {
+  return mm_bwd_direct_x(w, dy, M, N, K, dtype) && mm_bwd_direct_w(x, dy, M, N, K, dtype);
+}
+// The fp32 planes of whichever of the two untransposed products splits over K into more.
+int64_t mm_bwd_planes(int64_t M, int64_t N, int64_t K, int dtype) {
+  return dtype == Q3_BF16 ? std::max(q3::gemm_t_workspace_bytes(M, K, N), q3::gemm_t_workspace_bytes(N, K, M)) : 0;
+}
 
 }  // namespace
 
@@ -1082,16 +1089,20 @@ int64_t q3_matmul_backward_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K,
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   int64_t need = std::max(q3_matmul_workspace_bytes(M, K, N, dtype, 0),
                           q3_matmul_workspace_bytes(N, K, padded_rows(M, dtype), dtype, 0));
-  if (dtype == Q3_BF16)
-    need = std::max({need, q3::gemm_t_workspace_bytes(M, K, N), q3::gemm_t_workspace_bytes(N, K, M)});
-  return need;
+  return std::max(need, mm_bwd_planes(M, N, K, dtype));
 }
 
 int64_t q3_matmul_backward_workspace_bytes_for(const void* x, const void* w, const void* dy, int64_t M, int64_t N,
                                                int64_t K, int dtype) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
-  const bool direct = mm_bwd_direct_x(w, dy, M, N, K, dtype) && mm_bwd_direct_w(x, dy, M, N, K, dtype);
-  return direct ? align256(colsum_parts(M) * N * 4) : mm_bwd_layout(M, N, K, dtype).total;
+  if (!mm_bwd_direct(x, w, dy, M, N, K, dtype)) return mm_bwd_layout(M, N, K, dtype).total;
+  return align256(colsum_parts(M) * N * 4) + mm_bwd_planes(M, N, K, dtype);
+}
+
+int64_t q3_matmul_backward_gemm_workspace_bytes_for(const void* x, const void* w, const void* dy, int64_t M, int64_t N,
+                                                    int64_t K, int dtype) {
+  if (M <= 0 || N <= 0 || K <= 0 || mm_bwd_direct(x, w, dy, M, N, K, dtype)) return 0;
+  return q3_matmul_backward_gemm_workspace_bytes(M, N, K, dtype);
 }
 
 int q3_matmul_backward(const void* x, const void* w, const void* dy, void* gx, void* gw, void* gb, int64_t M,
@@ -1103,9 +1114,14 @@ int q3_matmul_backward(const void* x, const void* w, const void* dy, void* gx, v
   if (M == 0 || N == 0 || K == 0) return Q3_OK;
   const bool dir_x = mm_bwd_direct_x(w, dy, M, N, K, dtype), dir_w = mm_bwd_direct_w(x, dy, M, N, K, dtype);
   MmBwdLayout l = mm_bwd_layout(M, N, K, dtype);
-  if (dir_x && dir_w) {  // no operand is transposed: the workspace holds the bias gradient's partial sums alone
+  if (dir_x && dir_w) {  // no operand is transposed: the bias gradient's partial sums, then the products' planes
     l.part = 0;
     l.total = align256(colsum_parts(M) * N * 4);
+    const int64_t planes = mm_bwd_planes(M, N, K, dtype);
+    if (planes > 0 && workspace_bytes >= l.total + planes) {  // (else the planes go to gemm_ws)
+      gemm_ws = static_cast<char*>(workspace) + l.total;
+      gemm_ws_bytes = planes;
+    }
   }
   Q3_REQUIRE(workspace && workspace_bytes >= l.total, Q3_ERR_WORKSPACE);
   Q3_REQUIRE(q3_aligned(workspace, 256), Q3_ERR_ALIGN);

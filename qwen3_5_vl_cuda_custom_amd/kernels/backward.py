@@ -55,9 +55,9 @@ class MatmulFunction(torch.autograd.Function):
         gb = torch.empty((N,), dtype=w.dtype, device=w.device) if (need_b and ctx.has_bias) else None
         lib = _lib.lib()
         wc = _c(w)
-        ws, nws = _lib.workspace(lib.q3_matmul_backward_workspace_bytes_for(
-            x2.data_ptr(), wc.data_ptr(), dy2.data_ptr(), M, N, K, _dt(x)), x.device)
-        gws, gnws = _lib.gemm_workspace(lib.q3_matmul_backward_gemm_workspace_bytes(M, N, K, _dt(x)), x.device)
+        ops = (x2.data_ptr(), wc.data_ptr(), dy2.data_ptr(), M, N, K, _dt(x))
+        ws, nws = _lib.workspace(lib.q3_matmul_backward_workspace_bytes_for(*ops), x.device)
+        gws, gnws = _lib.gemm_workspace(lib.q3_matmul_backward_gemm_workspace_bytes_for(*ops), x.device)
         _lib.call("q3_matmul_backward", x2.data_ptr(), wc.data_ptr(), dy2.data_ptr(), _lib.ptr(gx), _lib.ptr(gw),
                   _lib.ptr(gb), M, N, K, _dt(x), _lib.ptr(ws), nws, _lib.ptr(gws), gnws, _lib.stream())
         gr = dy if (need_r and ctx.has_residual) else None

@@ -71,6 +71,13 @@ def test_matmul_validation():
     # the backward's products split at any row count: dX of 16 rows of the vocabulary head in 8 planes
     for rows in (1, 16, 32, 33):
         assert L.q3_matmul_backward_gemm_workspace_bytes(rows, 151936, 4096, 1) >= (16 << 10) + 8 * rows * 4096 * 4
+    # ... which lie in the call's own workspace where the operands are multiplied as they are, not in the one that
+    # calls on every stream share
+    for M, N, K, planes in ((16, 151936, 4096, 8 * 16 * 4096), (4104, 24, 520, 8 * 24 * 520), (64, 256, 256, 0)):
+        assert L.q3_matmul_backward_gemm_workspace_bytes_for(FAKE, FAKE, FAKE, M, N, K, 1) == 0
+        assert L.q3_matmul_backward_workspace_bytes_for(FAKE, FAKE, FAKE, M, N, K, 1) >= planes * 4
+    assert L.q3_matmul_backward_gemm_workspace_bytes_for(FAKE, FAKE, FAKE, 16, 20480, 4098, 1) == \
+        L.q3_matmul_backward_gemm_workspace_bytes(16, 20480, 4098, 1)
     assert L.q3_matmul_workspace_bytes(8, 4096, 20480, 1, 0) == 0
     ws = L.q3_matmul_workspace_bytes(32, 4096, 20480, 1, 0)
     assert ws > 0

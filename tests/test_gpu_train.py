@@ -291,6 +291,28 @@ def test_matmul_backward_untransposed_against_transposed(M, N, K_):
         assert over <= 0, f"{n} {(M, N, K_)}: {over:.3e} over"
 
 
+def test_matmul_backward_on_two_streams_shares_no_workspace():
+    """Backward passes whose products split over K, in turn on two streams that are not ordered against each other:
+    each gives the bits of a pass of its own (their partial planes lie in the call's memory)."""
+    from qwen3_5_vl_cuda_custom_amd import _lib
+    sets = [[t.bfloat16().to(DEV) for t in (rnd(33, 1160, seed=s), rnd(8208, 1160, seed=s + 1, std=0.1),
+                                             rnd(33, 8208, seed=s + 2))] for s in (60, 70)]
+    assert _lib.lib().q3_matmul_backward_workspace_bytes_for(*(t.data_ptr() for t in (sets[0][0], sets[0][1],
+                                                                                      sets[0][2])),
+                                                             33, 8208, 1160, _lib.Q3_BF16) >= 8 * 33 * 1160 * 4
+    want = [run_grads(K.matmul, s[:2], s[2])[1] for s in sets]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in sets]
+    got = [[], []]
+    for _ in range(8):
+        for i, st in enumerate(streams):
+            with torch.cuda.stream(st):
+                got[i].append(run_grads(K.matmul, sets[i][:2], sets[i][2])[1])
+    torch.cuda.synchronize()
+    for g, w in zip(got, want):
+        assert all(torch.equal(a, b) for run in g for a, b in zip(run, w))
+
+
 @pytest.mark.parametrize("M,N,K_", [(1024, 4096, 12352), (512, 2048, 8256)])
 def test_matmul_split_with_shorter_last_split(M, N, K_):
     """A K that no split count divides into whole 64-wide stages: the forward runs it unsplit (the backward's products
