@@ -396,6 +396,21 @@ def test_flash_attention_backward_bf16(B, Hq, Hkv, Sq, Sk, D, causal):
     twice_equal(lambda: run_grads(_fa(Hq // Hkv, causal, s), [q, k, v], dy)[1])
 
 
+def _attention_backward_simt(q, k, v, dy, scale, causal):
+    """(dq, dk, dv) of the SIMT kernels, which a workspace of one float per row selects."""
+    from qwen3_5_vl_cuda_custom_amd import _lib
+    from qwen3_5_vl_cuda_custom_amd.kernels.flash_attention import flash_attention_lse
+    (B, Hq, Sq, D), (_, Hkv, Sk, _) = q.shape, k.shape
+    qd, kd, vd, dyd = (t.to(DEV) for t in (q, k, v, dy))
+    o, lse = flash_attention_lse(qd, kd, vd, scale, causal, Hq // Hkv)
+    out = [torch.empty_like(t) for t in (qd, kd, vd)]
+    nws = _lib.lib().q3_flash_attention_backward_workspace_bytes(B, Hq, Sq)
+    ws = torch.empty(nws, dtype=torch.uint8, device=DEV)
+    _lib.call("q3_flash_attention_backward", *(t.data_ptr() for t in (qd, kd, vd, o, lse, dyd, *out)), B, Hq, Hkv,
+              Sq, Sk, D, scale, int(causal), _lib.dtype_code(q.dtype), ws.data_ptr(), nws, _lib.stream())
+    return out
+
+
 @pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,D,causal", [
     (1, 4, 1, 1, 1, 128, True), (2, 2, 2, 31, 33, 64, False), (1, 8, 2, 129, 129, 128, True),
     (1, 8, 2, 64, 200, 128, True), (1, 8, 2, 200, 64, 128, True), (1, 6, 2, 97, 127, 96, False),
@@ -409,21 +424,13 @@ def test_flash_attention_backward_mfma_against_simt(B, Hq, Hkv, Sq, Sk, D, causa
     (2^-7 of it), the fp32 sums' error over terms up to the largest result (2^-14 of it), and, where dP - Dv cancels
     (one key: dS is 0 up to rounding), the fp32 rounding of dP and Dv (a few 2^-24 of the largest dP, here 2^-21)
     times the largest |scale * q| or |scale * k|."""
-    from qwen3_5_vl_cuda_custom_amd import _lib
-    from qwen3_5_vl_cuda_custom_amd.kernels.flash_attention import flash_attention_lse
     q, k, v = (rnd(B, Hq, Sq, D, seed=64).bfloat16(), rnd(B, Hkv, Sk, D, seed=65).bfloat16(),
                rnd(B, Hkv, Sk, D, seed=66).bfloat16())
     dy = rnd(B, Hq, Sq, D, seed=67).bfloat16()
     s = D ** -0.5
     _, got = run_grads(_fa(Hq // Hkv, causal, s), [q, k, v], dy)
     _, ref = ref_grads(_fa_ref(Hq // Hkv, causal, s), [q, k, v], dy)
-    qd, kd, vd, dyd = (t.to(DEV) for t in (q, k, v, dy))
-    o, lse = flash_attention_lse(qd, kd, vd, s, causal, Hq // Hkv)
-    simt = [torch.empty_like(t) for t in (qd, kd, vd)]
-    nws = _lib.lib().q3_flash_attention_backward_workspace_bytes(B, Hq, Sq)
-    ws = torch.empty(nws, dtype=torch.uint8, device=DEV)
-    _lib.call("q3_flash_attention_backward", *(t.data_ptr() for t in (qd, kd, vd, o, lse, dyd, *simt)), B, Hq, Hkv,
-              Sq, Sk, D, s, int(causal), _lib.dtype_code(q.dtype), ws.data_ptr(), nws, _lib.stream())
+    simt = _attention_backward_simt(q, k, v, dy, s, causal)
     dp = (dy.float() @ v.float().repeat_interleave(Hq // Hkv, dim=1).transpose(-1, -2)).abs().max()
     noise = 2.0 ** -21 * float(dp * torch.maximum(q.abs().max(), k.abs().max())) * s
     for a, r, b, n in zip(got, ref, simt, ("dq", "dk", "dv")):
@@ -433,6 +440,25 @@ def test_flash_attention_backward_mfma_against_simt(B, Hq, Hkv, Sq, Sk, D, causa
         assert over <= 0, f"{n} vs SIMT: {over:.3e} over"
         if float(r.abs().max()) > 1e-6:  # one key: P = 1, dS = 0 up to rounding
             assert_grad_close(a, r, f"flash {n} D={D}")
+
+
+@pytest.mark.parametrize("D,where", [(64, (5, 7)), (72, (40, 70)), (128, (95, 127)), (128, (0, 0))])
+def test_flash_attention_backward_keeps_infinities(D, where):
+    """One infinite element of dO: the gradients of the matrix-core kernels are infinite, NaN and finite where the SIMT
+    kernels' are, with the same signs, and the finite ones agree as without it (the bounds of the test above)."""
+    q, k, v, dy = (rnd(1, 2, 96, D, seed=64 + i).bfloat16() for i in range(4))
+    dy[0, 1][where] = float("inf")
+    _, got = run_grads(_fa(1, False, D ** -0.5), [q, k, v], dy)
+    simt = _attention_backward_simt(q, k, v, dy, D ** -0.5, False)
+    assert any(bool(b.isinf().any()) for b in simt)
+    noise = 2.0 ** -21 * 8 * D ** 0.5 * D ** -0.5
+    for a, b, n in zip(got, simt, ("dq", "dk", "dv")):
+        x, y = a.float(), b.float()
+        assert torch.equal(x.isnan(), y.isnan()) and torch.equal(x.isinf(), y.isinf()), n
+        assert torch.equal(x[x.isinf()], y[y.isinf()]), n
+        x, y = x[x.isfinite()], y[y.isfinite()]
+        tol = 2.0 ** -7 * torch.maximum(x.abs(), y.abs()) + 2.0 ** -14 * y.abs().max() + noise
+        assert bool(((x - y).abs() <= tol).all()), n
 
 
 @pytest.mark.parametrize("M,N,K_", [(1, 4, 4), (31, 33, 36), (33, 31, 132), (128, 256, 688), (130, 66, 260),
