@@ -3,6 +3,7 @@ from __future__ import annotations
 
 import torch
 from torch import nn
+from torch.nn.modules import module as nn_module
 
 from ..kernels.backward import (FlashAttentionFunction, QKNormRopeFunction, RopeAttentionFunction, attention_bshd_ok,
                                 needs_grad)
@@ -13,11 +14,15 @@ from ..kernels import (apply_rope, decode_attention, decode_attention_paged, fla
 from .kv_cache import PagedKVCache, StaticKVCache
 from .linear import CudaLinear
 from .norms import CudaRMSNorm, fused_norm_ok
-from .rotary import MRoPEBinding
+from .rotary import MRoPEBinding, TextMRoPE
 
 
-def _has_hooks(m: nn.Module) -> bool:
-    return bool(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
+def _called_plainly(m: nn.Module) -> bool:
+    """Whether calling m is its class's forward and nothing else: no hooks, its own or global, no forward of the
+    instance's own."""
+    return not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
+                or nn_module._global_forward_hooks or nn_module._global_forward_pre_hooks
+                or nn_module._global_backward_hooks or nn_module._global_backward_pre_hooks or "forward" in m.__dict__)
 
 
 class CudaVisionAttention(nn.Module):
@@ -231,12 +236,12 @@ class CudaFullAttention(nn.Module):
 
     def _train_positions(self, mrope_apply, q, k, v) -> torch.Tensor | None:
         """(3, B, S) int32 positions when the q/k norms and the rotation can train as one op
-        (QKNormRopeFunction), else None: a binding with integer positions on the GPU, plain norm
-        modules (no hooks, one eps), one dtype, head dims of the backward kernel, contiguous rows. The
+        (QKNormRopeFunction), else None: a plain binding with integer positions on the GPU, plain norm
+        modules (nothing else called with them, one eps), one dtype, head dims of the backward kernel, contiguous rows. The
         positions are a copy: the caller may reuse its tensor before the backward runs."""
         norms = (self.q_norm, self.k_norm)
         if not (self._fusable(mrope_apply, q) and self.head_dim in (64, 128, 256)
-                and all(type(n) is CudaRMSNorm and not _has_hooks(n) and n.weight.dtype == q.dtype
+                and all(type(n) is CudaRMSNorm and _called_plainly(n) and n.weight.dtype == q.dtype
                         and n.weight.shape == (self.head_dim,) and n.weight.is_contiguous() for n in norms)
                 and norms[0].eps == norms[1].eps and q.dtype == k.dtype == v.dtype
                 and q.dtype in (torch.bfloat16, torch.float32)
@@ -246,7 +251,8 @@ class CudaFullAttention(nn.Module):
         pid, rope = mrope_apply.position_ids, mrope_apply.rope
         if (pid.device != q.device or pid.dtype not in (torch.int32, torch.int64) or pid.dim() != 3 or pid.shape[0] != 3
                 or pid.shape[1] not in (1, B) or pid.shape[2] != S or B * S == 0 or B * S >= 2 ** 31
-                or type(mrope_apply) is not MRoPEBinding or len(rope.mrope_section) != 3
+                or type(mrope_apply) is not MRoPEBinding or type(rope) is not TextMRoPE
+                or not rope.__dict__.keys().isdisjoint(("apply", "compute_cos_sin")) or len(rope.mrope_section) != 3
                 or sum(rope.mrope_section) * 2 != self.head_dim or min(rope.mrope_section) < 0
                 or rope.inv_freq.dtype != torch.float32 or rope.inv_freq.numel() * 2 != self.head_dim):
             return None

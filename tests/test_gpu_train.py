@@ -604,8 +604,8 @@ def test_attention_gradients_on_token_major_storage(B, H, Hkv, S, D, causal):
 
 @torch.enable_grad()
 def test_text_attention_training_routes_agree():
-    """Positions as floats, a hook on a norm and a frozen norm weight: the first two take the single ops, and every
-    route gives the fused one's result up to the roundings between its single ops (three of 2^-8 of the largest)."""
+    """Positions as floats, a hook on a norm and a frozen norm weight: every route gives the fused one's result up to
+    the roundings between its single ops (three of 2^-8 of the largest). Which route each takes: the test below."""
     from qwen3_5_vl_cuda_custom_amd.modules import CudaFullAttention, TextMRoPE
     torch.manual_seed(0)
     att = CudaFullAttention(256, 4, 2, 64).to(DEV, torch.bfloat16)
@@ -629,6 +629,60 @@ def test_text_attention_training_routes_agree():
     for got in runs:
         for a, b in zip(got, want):
             assert float((a.float() - b.float()).abs().max()) <= 3 * 2.0 ** -8 * float(b.float().abs().max())
+
+
+@torch.enable_grad()
+@pytest.mark.parametrize("case", ["plain", "frozen weight", "float positions", "norm hook", "global hook",
+                                  "global pre-hook", "replaced forward", "other rotary"])
+def test_text_attention_training_fuses_only_plain_norms(case):
+    """Norm and rotation train as one op only where nothing else is called with them and the positions are whole
+    numbers; what the single ops would have called (hooks, a replaced forward, another rotary's angles, fractional
+    positions) takes effect."""
+    from torch.nn.modules import module as nn_module
+    from qwen3_5_vl_cuda_custom_amd.modules import CudaFullAttention, CudaRMSNorm, TextMRoPE
+    torch.manual_seed(0)
+    att = CudaFullAttention(256, 4, 2, 64).to(DEV, torch.bfloat16)
+    rope = TextMRoPE(64, 5e6, [12, 10, 10]).to(DEV)
+    x = rnd(2, 70, 256, seed=91).bfloat16().to(DEV)
+    pos, seen, handle = torch.arange(70, device=DEV).expand(3, 1, 70).contiguous(), [], None
+    base = att(x, rope.bind(pos))[0].detach()
+    hook = lambda m, *a: seen.append(1) if m is att.q_norm else None  # noqa: E731
+    if case == "frozen weight":
+        att.q_norm.weight.requires_grad_(False)
+    elif case == "float positions":
+        pos = pos + 0.5
+    elif case == "norm hook":
+        handle = att.q_norm.register_forward_hook(hook)
+    elif case == "global hook":
+        handle = nn_module.register_module_forward_hook(hook)
+    elif case == "global pre-hook":
+        handle = nn_module.register_module_forward_pre_hook(hook)
+    elif case == "replaced forward":
+        att.q_norm.forward = lambda t: seen.append(1) or CudaRMSNorm.forward(att.q_norm, t)
+    elif case == "other rotary":
+        class Halved(TextMRoPE):
+            def compute_cos_sin(self, position_ids):
+                return super().compute_cos_sin(position_ids.float() / 2)
+        rope = Halved(64, 5e6, [12, 10, 10]).to(DEV)
+    try:
+        q, k, v = (torch.zeros(2, 70, h, 64, device=DEV, dtype=torch.bfloat16) for h in (4, 2, 2))
+        fused = att._train_positions(rope.bind(pos), q, k, v) is not None
+        assert fused == (case in ("plain", "frozen weight"))
+        out = att(x, rope.bind(pos))[0].detach()
+    finally:
+        if handle is not None:
+            handle.remove()
+    assert bool(seen) == ("hook" in case or case == "replaced forward")
+    q, k, v = (p(x).view(2, 70, -1, 64) for p in (att.q_proj, att.k_proj, att.v_proj))
+    cos, sin = rope.compute_cos_sin(pos)
+    q, k = (K.apply_mrope(K.rmsnorm(t, n.weight, n.eps).transpose(1, 2), cos, sin, [12, 10, 10])
+            for t, n in ((q, att.q_norm), (k, att.k_norm)))
+    ref = K.flash_attention(q, k, v.transpose(1, 2), scale=att.scale, is_causal=True, num_kv_groups=2)
+    ref = att.o_proj(ref.transpose(1, 2).reshape(2, 70, 256)).detach().float()
+    # the single ops' two roundings more than the fused one: three of 2^-8 of the largest
+    assert float((out.float() - ref).abs().max()) <= 3 * 2.0 ** -8 * float(ref.abs().max())
+    if case in ("float positions", "other rotary"):
+        assert float((out.float() - base.float()).abs().max()) > 0
 
 
 def test_topk_and_index_add_backward():
