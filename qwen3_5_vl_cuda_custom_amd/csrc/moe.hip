@@ -978,8 +978,8 @@ int launch_combine(const int* top_idx, const int* pos_of, const bf16* y_perm, co
 // (token, slot) entries in expert-major order (P = T k), as the inference path.
 //   forward   gu = x[token] . gate_up[e]^T     a = bf16(silu(g) u)
 //             out = sum over the token's experts of bf16(bf16(a . down[e]^T) w)
-//   backward  dh = dout[token] . down[e]       dw = sum_i dh a
-//             dgu = swiglu'(g, u) (w dh)       aw = bf16(a w)
+//   backward  dh = dout[token] . down[e]       dw = sum_i dh silu(g) u
+//             dgu = swiglu'(g, u) (w dh)       aw = bf16(silu(g) u w)
 //             dx[t] = sum over its rows of dgu . gate_up[e]   (fp32, rounded once)
 //             dgate_up[e] = dgu_e^T . x[token]_e    ddown[e] = dout[token]_e^T . aw_e
 // The products are grouped MFMA GEMMs on the weights as they are stored: dh
@@ -1096,7 +1096,7 @@ __global__ __launch_bounds__(256) void moe_act_bwd_kernel(const bf16* __restrict
     for (int q = 0; q < 8; ++q) {
       const float g = bf2f(g8[q]), u = bf2f(u8[q]), d = bf2f(d8[q]);
       const float s = 1.0f / (1.0f + expf(-g));
-      const float a = bf2f(f2bf(moe_act(g, u)));
+      const float a = moe_act(g, u);  // unrounded: aw and dw round once, not after the forward's rounding
       acc += d * a;
       a8[q] = f2bf(a * w);
       dg[q] = f2bf(d * w * u * s * (1.0f + g * (1.0f - s)));

@@ -857,6 +857,24 @@ def test_moe_training_leaves_out_ids_that_are_no_experts():
     assert not got[3][3].any() and not got[3][70, 1] and not got[3][149, 0]
 
 
+def test_moe_down_gradient_rounds_its_operand_once():
+    """The weight gradient of down multiplies grad_out with w silu(g) u rounded to bf16 once. One token per expert, x a
+    unit vector (g and u are entries of gate_up, exact) and a gradient of ones: each element is that operand itself,
+    within half a bf16 step (8 significant bits: 2^-8 of it; expf's 2^-20 beside it). A rounding of silu(g) u before it would double that."""
+    from qwen3_5_vl_cuda_custom_amd.kernels.moe_routing import moe_experts_train
+    E, H, I = 16, 64, 128
+    x = torch.zeros(E, H).bfloat16()
+    x[:, 0] = 1
+    gu, dn = rnd(E, 2 * I, H, seed=1).bfloat16(), rnd(E, H, I, seed=2).bfloat16()
+    w = (torch.rand(E, 1, generator=torch.Generator().manual_seed(3)) + 0.1).bfloat16()
+    idx = torch.arange(E, device=DEV).view(E, 1)
+    _, got = run_grads(lambda *a: moe_experts_train(a[0], a[1], a[2], idx, a[3]), (x, gu, dn, w),
+                       torch.ones(E, H).bfloat16())
+    g, u = gu[:, :, 0].double().chunk(2, dim=1)
+    ref = (F.silu(g) * u * w.double()).unsqueeze(1)
+    assert bool(((got[2].cpu().double() - ref).abs() <= (2.0 ** -8 + 2.0 ** -20) * ref.abs()).all())
+
+
 def test_moe_training_checks_its_operands():
     """What the inference entry refuses (routing on the host, other shapes, mixed types) is refused before a launch."""
     from qwen3_5_vl_cuda_custom_amd.kernels.moe_routing import moe_experts_train
