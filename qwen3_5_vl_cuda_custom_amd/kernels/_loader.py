@@ -6,7 +6,8 @@ CPU fallback: an op whose kernel cannot run raises. What it records instead are
 the slower device paths a call can take: `aligned_copy` (a bf16 operand that
 misses the MFMA kernels' 16-byte alignment, copied into an aligned buffer
 first) and `simt_kernel: ...` (a bf16 call whose shape or layout only the SIMT
-kernel takes). Under CUDA_QWEN3_VL_STRICT=1 those raise.
+kernel takes). Under CUDA_QWEN3_VL_STRICT=1 those raise. `experts_one_by_one: ...`
+(bf16 MoE training outside the grouped kernels' sizes) is recorded only.
 """
 from __future__ import annotations
 

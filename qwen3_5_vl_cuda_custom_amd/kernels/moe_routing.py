@@ -6,6 +6,7 @@ import torch
 
 from .. import _lib
 from ._common import check, mfma_operand, note_slow_path, require_device, require_same_dtype
+from ._loader import record_fallback
 from .backward import MoEExpertsFunction, BatchedGemmFunction, IndexAddFunction, TopKFunction, needs_grad
 
 
@@ -173,14 +174,21 @@ def moe_experts(x: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, top_
 def moe_experts_train(x: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, top_idx: torch.Tensor,
                       top_w: torch.Tensor) -> torch.Tensor | None:
     """moe_experts with a backward (x, gate_up, down and top_w), every expert in a few grouped launches; None where it
-    does not cover the operands (fp32, widths that are no multiple of 8, unaligned views, 2 GiB and more): the caller
-    then runs the experts one by one on the single ops. top_idx (T, k) int32 or int64, distinct experts per token;
+    does not cover the operands (fp32; in bf16, recorded in FALLBACK_LOG: widths that are no multiple of 8, unaligned
+    views, 2 GiB and more, which H = 2048, I = 768, k = 8 reach at 65,472 tokens): the caller then runs the experts one
+    by one on the single ops, 100 times slower with 128 experts. top_idx (T, k) int32 or int64, distinct experts per token;
     ids outside [0, E) are left out, in the output and in every gradient."""
     require_device("moe_experts_train", x, gate_up, down, top_w)
     require_same_dtype("moe_experts_train", x, gate_up, down, top_w)
     T, H, I, E, k = _expert_shapes("moe_experts_train", x, gate_up, down, top_idx, top_w, (torch.int32, torch.int64))
-    if (x.dtype != torch.bfloat16 or any(t.data_ptr() % 16 for t in (x, gate_up, down))
-            or _lib.lib().q3_moe_train_state_bytes(T, H, I, E, k) == 0):
+    if x.dtype != torch.bfloat16 or T == 0:
+        return None
+    unaligned = any(t.data_ptr() % 16 for t in (x, gate_up, down))
+    if unaligned or _lib.lib().q3_moe_train_state_bytes(T, H, I, E, k) == 0:
+        # recorded, not refused in strict mode: each expert's products still run on the MFMA kernels (or refuse there)
+        record_fallback("moe_experts_train", "experts_one_by_one: " + (
+            "an operand is not 16-byte aligned" if unaligned else f"T={T} H={H} I={I} E={E} k={k} is outside the "
+            "grouped kernels (widths in multiples of 8, k <= 32, E < 2048, T k < 2^20, operands below 2 GiB)"))
         return None
     return MoEExpertsFunction.apply(x, gate_up, down, top_idx.to(torch.int32), top_w)
 

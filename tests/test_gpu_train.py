@@ -894,6 +894,29 @@ def test_moe_training_checks_its_operands():
         moe_experts_train(x, gu.float(), dn, idx, w)
 
 
+def test_moe_training_records_what_it_declines(monkeypatch):
+    """A bf16 call outside the grouped kernels is recorded, and in strict mode too left to the loop over the experts;
+    fp32 and empty calls, which have no other path, are not recorded."""
+    from qwen3_5_vl_cuda_custom_amd.kernels import _loader
+    from qwen3_5_vl_cuda_custom_amd.kernels.moe_routing import moe_experts_train
+    monkeypatch.setattr(_loader, "FALLBACK_LOG", [])
+    monkeypatch.setenv("CUDA_QWEN3_VL_STRICT", "1")
+
+    def call(T, H, I, dtype=torch.bfloat16, off=0):
+        x, gu, dn, w = (torch.zeros(*s, device=DEV, dtype=dtype) for s in ((T * H + off,), (4, 2 * I, H), (4, H, I),
+                                                                           (T, 2)))
+        idx = torch.zeros(T, 2, dtype=torch.int32, device=DEV)
+        idx[:, 1] = 1
+        return moe_experts_train(x[off:].view(T, H), gu, dn, idx, w)
+
+    assert call(6, 64, 32) is not None
+    assert call(6, 64, 32, torch.float32) is None and call(0, 64, 32) is None
+    assert _loader.FALLBACK_LOG == []
+    assert call(6, 64, 20) is None and call(6, 64, 32, off=1) is None
+    assert [(op, r.split(":")[0]) for op, r, _ in _loader.FALLBACK_LOG] == [("moe_experts_train",
+                                                                             "experts_one_by_one")] * 2
+
+
 def test_moe_block_trains_past_a_nan_token():
     """One token of NaN: its expert part is zero, the other tokens' outputs and the experts' weight gradients are those
     of the block without it (the same rows and tiles: equal up to the order of sums, one bf16 rounding)."""
