@@ -460,34 +460,46 @@ __global__ __launch_bounds__(kT) void colsum_partial_vec_kernel(const T* __restr
   }
 }
 
-// out[c] = sum over the nparts partial rows, rounded once: 16 columns x 16
-// lanes per block, lane l takes rows l, l + 16, ... in order, the lanes' sums
-// are added in lane order. (One thread per column walked the rows one
-// dependent load at a time: 2048 partial rows of 128 columns, ~0.6 ms.)
-template <typename T>
+// out[c] = sum over the nparts partial rows, rounded once. PL lanes per column:
+// lane l takes rows l, l + PL, ... in order, the lanes' sums are added in lane
+// order. (One thread per column walked the rows one dependent load at a time:
+// 2048 partial rows of 128 columns, ~0.6 ms.)
+template <typename T, int PL>
 __global__ __launch_bounds__(kT) void colsum_reduce_kernel(const float* __restrict__ part, T* __restrict__ out,
                                                            int64_t nparts, int64_t cols) {
-  __shared__ float s_red[16][17];
-  const int cl = threadIdx.x & 15, pl = threadIdx.x >> 4;
-  const int64_t c = (int64_t)blockIdx.x * 16 + cl;
+  constexpr int COLS = kT / PL;
+  __shared__ float s_red[PL][COLS + 1];
+  const int cl = threadIdx.x % COLS, pl = threadIdx.x / COLS;
+  const int64_t c = (int64_t)blockIdx.x * COLS + cl;
   float acc = 0.f;
   if (c < cols) {
 #pragma unroll 8
-    for (int64_t p = pl; p < nparts; p += 16) acc += part[p * cols + c];
+    for (int64_t p = pl; p < nparts; p += PL) acc += part[p * cols + c];
   }
-  s_red[pl][cl] = acc;
-  __syncthreads();
-  if (pl != 0 || c >= cols) return;
-  float v = s_red[0][cl];
+  if constexpr (PL > 1) {
+    s_red[pl][cl] = acc;
+    __syncthreads();
+    if (pl != 0) return;
+    acc = s_red[0][cl];
 #pragma unroll
-  for (int u = 1; u < 16; ++u) v += s_red[u][cl];
-  out[c] = from_f<T>(v);
+    for (int u = 1; u < PL; ++u) acc += s_red[u][cl];
+  }
+  if (c < cols) out[c] = from_f<T>(acc);
 }
 
+// One lane per column where the rows are few, or where the columns fill the
+// chip: with 16 lanes most of a block has nothing to load. One lane / 16, the
+// whole column sum in us: 1 row of 128 columns 3.8 / 4.0, of 151,936 4.1 / 7.2; 4
+// rows of 1152 4.5 / 4.4, 6 rows 5.1 / 4.4; of 12,288, 8 rows 4.5 / 5.0, 16 rows
+// 5.1 / 5.6, 32 rows 12.4 / 12.0.
 template <typename T>
 int colsum_reduce(const float* part, void* out, int64_t nparts, int64_t cols, hipStream_t st) {
-  hipLaunchKernelGGL(colsum_reduce_kernel<T>, dim3((unsigned)q3_cdiv(cols, 16)), dim3(kT), 0, st, part,
-                     static_cast<T*>(out), nparts, cols);
+  if (nparts <= 4 || (cols >= 4096 && nparts <= 16))
+    hipLaunchKernelGGL((colsum_reduce_kernel<T, 1>), dim3((unsigned)q3_cdiv(cols, kT)), dim3(kT), 0, st, part,
+                       static_cast<T*>(out), nparts, cols);
+  else
+    hipLaunchKernelGGL((colsum_reduce_kernel<T, 16>), dim3((unsigned)q3_cdiv(cols, kT / 16)), dim3(kT), 0, st, part,
+                       static_cast<T*>(out), nparts, cols);
   Q3_LAUNCH_CHECK();
   return Q3_OK;
 }

@@ -291,6 +291,19 @@ def test_matmul_backward_untransposed_against_transposed(M, N, K_):
         assert over <= 0, f"{n} {(M, N, K_)}: {over:.3e} over"
 
 
+@pytest.mark.parametrize("M,N", [(1, 40), (256, 40), (257, 40), (64, 5000), (1024, 4096), (1025, 4096), (1088, 4104),
+                                 (300, 77), (1300, 77)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_bias_gradient_partial_rows(M, N, dtype):
+    """Column sums on both sides of the rule for their second pass (few partial rows, many columns), whole 16-byte
+    pieces and not: one rounding (2^-8 or 2^-24 of the sum) and the fp32 sums' error (M 2^-24 of the absolute sum)."""
+    x, w, b, dy = (rnd(*s, seed=i).to(dtype) for i, s in enumerate([(M, 8), (N, 8), (N,), (M, N)]))
+    gb = run_grads(K.matmul, [x, w, b], dy)[1][2].double().cpu()
+    ref, mag = dy.double().sum(0), dy.double().abs().sum(0)
+    ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -24
+    assert bool(((gb - ref).abs() <= ulp * ref.abs() + M * 2.0 ** -24 * mag).all())
+
+
 def test_matmul_backward_on_two_streams_shares_no_workspace():
     """Backward passes whose products split over K, in turn on two streams that are not ordered against each other:
     each gives the bits of a pass of its own (their partial planes lie in the call's memory)."""
