@@ -206,6 +206,26 @@ def test_cross_entropy_rows_and_masked_logits_bf16(N, V):
     assert bool((err <= 2.0 ** -8 * r.grad.abs() + 2.0 ** -20).all())
 
 
+@pytest.mark.parametrize("V", [1, 3, 255, 257, 1023, 1025, 2049, 5003])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_cross_entropy_scalar_rows(V, dtype):
+    """Rows that are no whole 16-byte pieces, around the 4 x 256 values of one pass: the loss and its gradient against
+    float64 (the bounds of the test above; fp32 gradients 2^-20), masked values, and a NaN, which the loss keeps."""
+    x = rnd(3, V, seed=97, std=2.0).to(dtype)
+    x[0, V // 3:-1] = float("-inf")
+    tg = torch.tensor([V - 1, V // 2, 0])
+    with torch.enable_grad():
+        a, r = x.to(DEV).requires_grad_(True), x.double().requires_grad_(True)
+        loss, want = K.cross_entropy(a, tg.to(DEV)), F.cross_entropy(r, tg)
+        loss.backward()
+        want.backward()
+    assert abs(float(loss) - float(want)) <= 1e-5 * max(1e-2, abs(float(want)))
+    ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -20
+    assert bool(((a.grad.double().cpu() - r.grad).abs() <= ulp * r.grad.abs() + 2.0 ** -20).all())
+    x[1, V - 1] = float("nan")
+    assert torch.isnan(K.cross_entropy(x.to(DEV), tg.to(DEV)))
+
+
 @pytest.mark.parametrize("rows,cols,dtype", [(8, 256, torch.float32), (4096, 128, torch.bfloat16)])
 def test_softmax_backward(rows, cols, dtype):
     x, dy = rnd(rows, cols, seed=30, dtype=dtype), rnd(rows, cols, seed=31, dtype=dtype)
