@@ -35,6 +35,11 @@ constexpr int kIlp = 2;       // rows of a step in flight per thread: with the 1
                               // 512 x 64 fp32 903 -> 752 us (797 with one row, 747 with 4 rows, which spill nothing
                               // but cost occupancy: 2 x 1024 tokens of 128 5036, 4875, 5141 us for 1, 2, 4)
 constexpr int kMaxD = 128;
+// Whether a last, partial tile takes all kTile steps (rows past the end are not live). Its own rows only, in a second
+// loop: 33 rows of 40 dims 49 -> 38 us, 500 of 64 458 -> 425; with 24 dims per lane the second loop costs more than
+// it saves (400 rows of 72 543 -> 561).
+template <int DS>
+constexpr bool kWholeTiles = DS == 24;
 
 struct BwdParams {
   const void *q, *k, *v, *o, *dout;
@@ -112,7 +117,7 @@ __global__ __launch_bounds__(kBT) void attn_bwd_dkdv_kernel(const BwdParams p) {
       }
       __syncthreads();
       // kIlp rows at a time: their dot products, exchanges and exponentials are independent chains
-      for (int r0 = 0; r0 < kTile; r0 += kIlp) {
+      auto rows = [&](int r0) {
         float s[kIlp], dp[kIlp];
 #pragma unroll
         for (int u = 0; u < kIlp; ++u) {
@@ -140,7 +145,11 @@ __global__ __launch_bounds__(kBT) void attn_bwd_dkdv_kernel(const BwdParams p) {
             dk[t] += ds * s_q[r][part * DS + t];
           }
         }
-      }
+      };
+      if (kWholeTiles<DS> || p.Sq - i0 >= kTile)
+        for (int r0 = 0; r0 < kTile; r0 += kIlp) rows(r0);
+      else
+        for (int r0 = 0; r0 < p.Sq - i0; r0 += kIlp) rows(r0);
     }
   }
   if (!jv) return;
@@ -195,7 +204,7 @@ __global__ __launch_bounds__(kBT) void attn_bwd_dq_kernel(const BwdParams p) {
       s_v[r][d] = ok ? to_f<T>(static_cast<const T*>(p.v)[(kv_base + j) * D + d]) : 0.f;
     }
     __syncthreads();
-    for (int r0 = 0; r0 < kTile; r0 += kIlp) {
+    auto rows = [&](int r0) {
       float s[kIlp], dp[kIlp];
 #pragma unroll
       for (int u = 0; u < kIlp; ++u) {
@@ -220,7 +229,11 @@ __global__ __launch_bounds__(kBT) void attn_bwd_dq_kernel(const BwdParams p) {
 #pragma unroll
         for (int t = 0; t < DS; ++t) dq[t] += ds * s_k[r][part * DS + t];
       }
-    }
+    };
+    if (kWholeTiles<DS> || j_end - j0 >= kTile)
+      for (int r0 = 0; r0 < kTile; r0 += kIlp) rows(r0);
+    else
+      for (int r0 = 0; r0 < j_end - j0; r0 += kIlp) rows(r0);
   }
   if (!iv) return;
   T* dqp = static_cast<T*>(p.dq) + q_row * D;

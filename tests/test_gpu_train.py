@@ -411,6 +411,26 @@ def test_flash_attention_backward_reference_shapes_fp32(Hq, Hkv, causal):
         assert_close(a, r, atol=5e-3, what=f"flash {n}")
 
 
+@pytest.mark.parametrize("Sq,Sk,D", [(1, 1, 8), (33, 17, 40), (17, 33, 32), (15, 31, 100), (47, 48, 72), (65, 64, 64)])
+@pytest.mark.parametrize("causal", [True, False])
+def test_flash_attention_backward_partial_tiles_fp32(Sq, Sk, D, causal):
+    """Query and key counts around the SIMT kernels' 16-row tiles, every width of their lanes' share, against float64:
+    fp32 sums of at most 65 terms of products of at most |6|, (65 + D) 2^-24 of the largest gradient and of dP."""
+    q, k, v, dy = rnd(2, 4, Sq, D, seed=60), rnd(2, 2, Sk, D, seed=61), rnd(2, 2, Sk, D, seed=62), rnd(2, 4, Sq, D, seed=63)
+    s = D ** -0.5
+    _, got = run_grads(_fa(2, causal, s), [q, k, v], dy)
+    with torch.enable_grad():
+        xs = [t.double().requires_grad_(True) for t in (q, k, v)]
+        a = xs[0] * s @ xs[1].repeat_interleave(2, 1).transpose(-1, -2)
+        if causal:
+            a = a.masked_fill(~torch.ones(Sq, Sk, dtype=torch.bool).tril(), float("-inf"))
+        ref = torch.autograd.grad(a.softmax(-1) @ xs[2].repeat_interleave(2, 1), xs, dy.double())
+    dp = float((dy @ v.repeat_interleave(2, 1).transpose(-1, -2)).abs().max())
+    for a, r, n in zip(got, ref, ("dq", "dk", "dv")):
+        tol = (65 + D) * 2.0 ** -24 * (4 * float(r.abs().max()) + dp)
+        assert float((a.double().cpu() - r).abs().max()) <= tol, n
+
+
 @pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,D,causal", [
     (1, 8, 2, 300, 300, 128, True),    # text GQA, ragged key tiles
     (2, 4, 4, 100, 100, 72, False),    # vision head dim, non-causal
