@@ -682,16 +682,23 @@ __global__ __launch_bounds__(64 * BW) void flash_decode_kernel(const AttnParams 
   q3::vm_wait<0>();  // no DMA may still target this block's LDS when the wave retires
 }
 
-// Merges the per-wave records of the pairs split between waves. A block takes
-// one head of one pair (2 outputs per lane), its 4 waves every fourth record
-// each, kB of them with all loads (m, l and the outputs) in flight together,
-// and the waves' (max, sum, acc) are merged in wave order. Bound by latency: a
-// pair has as many records as waves share it (1500 keys of one sequence: 47 per
-// pair, which one thread per output of one block per pair walked in 6 dependent
-// rounds).
+// Merges the per-wave records of the pairs split between waves, 2 outputs per
+// lane, kB records with all loads (m, l and the outputs) in flight together. Bound
+// by latency: a pair has as many records as waves share it (1500 keys of one
+// sequence: 47 per pair, which one thread per output of one block per pair walked
+// in 6 dependent rounds).
+// A block takes one head of one pair, its 4 waves every fourth record each, and
+// the waves' (max, sum, acc) are merged in wave order. BY_WAVE, for many pairs,
+// which have few records or are finished by one wave: a block takes one pair, each
+// wave a head at a time with all its records, and nothing is exchanged.
 // One sequence of 1500 keys x 8 KV heads 11.4 -> 4.8 us, 16 paged sequences x 4 KV
-// heads 13.1 -> 4.8 us; 32 sequences x 8 KV heads (few records a pair) 4.8 -> 5.0 us.
-template <int D>
+// heads 13.1 -> 4.8 us.
+// From 256 pairs on BY_WAVE. Whole decode attention, us, by wave / by head: 64
+// sequences of up to 1000 keys x 8 KV heads 32.3 / 34.4, 32 of 300 13.0 / 13.5, 32
+// of 2500 x 4 (128 pairs) 26.6 / 24.0, 24 of 1500 x 8 (192 pairs) 22.1 / 21.7.
+constexpr int64_t kCombineByWave = 256;
+
+template <int D, bool BY_WAVE>
 __global__ __launch_bounds__(256) void flash_decode_combine(const AttnParams p) {
   static_assert(D == 128, "two outputs per lane");
   __shared__ float s_m[4], s_l[4];
@@ -701,14 +708,15 @@ __global__ __launch_bounds__(256) void flash_decode_combine(const AttnParams p) 
   const int Hkv = p.Hkv, G = p.groups;
   const int b = pair / Hkv, kvh = pair % Hkv;
   const int lane = threadIdx.x & 63, rl = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int qc = blockIdx.y;
   // Advance the sequence's cache length (one block per sequence; nothing in
   // this launch reads the lengths).
-  if (p.lens_inc && kvh == 0 && qc == 0 && threadIdx.x == 0) p.lens_inc[b] += 1;
+  if (p.lens_inc && kvh == 0 && blockIdx.y == 0 && threadIdx.x == 0) p.lens_inc[b] += 1;
   const int nb = s_pre[b + 1] - s_pre[b];
-  bf16* out = p.o + (int64_t)b * p.ob + ((int64_t)kvh * G + qc) * p.oh + 2 * lane;
+  auto out_of = [&](int qc) { return p.o + (int64_t)b * p.ob + ((int64_t)kvh * G + qc) * p.oh + 2 * lane; };
+  const int qc0 = BY_WAVE ? rl : (int)blockIdx.y, qstep = BY_WAVE ? 4 : G;
   if (nb == 0) {  // empty sequence: zeros
-    if (rl == 0) out[0] = out[1] = f2bf(0.f);
+    for (int qc = qc0; qc < G; qc += qstep)
+      if (BY_WAVE || rl == 0) out_of(qc)[0] = out_of(qc)[1] = f2bf(0.f);
     return;
   }
   const int64_t U = (int64_t)Hkv * s_pre[p.B];
@@ -717,35 +725,51 @@ __global__ __launch_bounds__(256) void flash_decode_combine(const AttnParams p) 
   if (wf == wl) return;  // finished by its wave
   constexpr int kB = 4;
   const int PF = dec_partial_floats(G, D);
-  float mm = -INFINITY, l = 0.f, a0 = 0.f, a1 = 0.f;
-  for (int w0 = wf + rl; w0 <= wl; w0 += 4 * kB) {
-    float mv[kB], lv[kB];
-    float2 ov[kB];
+  float mm, l, a0, a1;
+  auto merge = [&](int qc, int first, int step) {  // records first, first + step, .. of head qc
+    mm = -INFINITY;
+    l = a0 = a1 = 0.f;
+    for (int w0 = first; w0 <= wl; w0 += step * kB) {
+      float mv[kB], lv[kB];
+      float2 ov[kB];
 #pragma unroll
-    for (int u = 0; u < kB; ++u) {
-      const int w = w0 + 4 * u;
-      const float* rec = p.partial + (int64_t)(min(w, wl) + pair) * PF;
-      mv[u] = w <= wl ? rec[qc] : -INFINITY;
-      lv[u] = rec[G + qc];
-      ov[u] = *reinterpret_cast<const float2*>(rec + 2 * G + qc * D + 2 * lane);
+      for (int u = 0; u < kB; ++u) {
+        const int w = w0 + step * u;
+        const float* rec = p.partial + (int64_t)(min(w, wl) + pair) * PF;
+        mv[u] = w <= wl ? rec[qc] : -INFINITY;
+        lv[u] = rec[G + qc];
+        ov[u] = *reinterpret_cast<const float2*>(rec + 2 * G + qc * D + 2 * lane);
+      }
+      float mb = mm;
+#pragma unroll
+      for (int u = 0; u < kB; ++u) mb = fmaxf(mb, mv[u]);
+      const float base = mb == -INFINITY ? 0.f : mb;  // every score so far -inf: weights 0, not NaN
+      const float sc = fast_exp2(mm - base);          // 0 on the first batch (mm = -inf)
+      l *= sc;
+      a0 *= sc;
+      a1 *= sc;
+#pragma unroll
+      for (int u = 0; u < kB; ++u) {
+        const float wt = fast_exp2(mv[u] - base);  // 0 for the padding records
+        l += lv[u] * wt;
+        a0 += ov[u].x * wt;
+        a1 += ov[u].y * wt;
+      }
+      mm = mb;
     }
-    float mb = mm;
-#pragma unroll
-    for (int u = 0; u < kB; ++u) mb = fmaxf(mb, mv[u]);
-    const float base = mb == -INFINITY ? 0.f : mb;  // every score so far -inf: weights 0, not NaN
-    const float sc = fast_exp2(mm - base);  // 0 on the first batch (mm = -inf)
-    l *= sc;
-    a0 *= sc;
-    a1 *= sc;
-#pragma unroll
-    for (int u = 0; u < kB; ++u) {
-      const float wt = fast_exp2(mv[u] - base);  // 0 for the padding records
-      l += lv[u] * wt;
-      a0 += ov[u].x * wt;
-      a1 += ov[u].y * wt;
+  };
+  auto store = [&](int qc) {
+    out_of(qc)[0] = f2bf(l > 0.f ? a0 / l : 0.f);
+    out_of(qc)[1] = f2bf(l > 0.f ? a1 / l : 0.f);
+  };
+  if constexpr (BY_WAVE) {
+    for (int qc = rl; qc < G; qc += 4) {
+      merge(qc, wf, 1);
+      store(qc);
     }
-    mm = mb;
+    return;
   }
+  merge(qc0, wf + rl, 4);
   if (lane == 0) {
     s_m[rl] = mm;
     s_l[rl] = l;
@@ -764,8 +788,7 @@ __global__ __launch_bounds__(256) void flash_decode_combine(const AttnParams p) 
     a0 += s_acc[u][lane].x * wt;
     a1 += s_acc[u][lane].y * wt;
   }
-  out[0] = f2bf(l > 0.f ? a0 / l : 0.f);
-  out[1] = f2bf(l > 0.f ? a1 / l : 0.f);
+  store(qc0);
 }
 
 // ----------------------------------------------------------------- prefill, pipelined (D = 128)
@@ -1746,8 +1769,11 @@ int decode_impl(const void* q, const void* k_cache, const void* v_cache, const i
     else
       hipLaunchKernelGGL((flash_decode_kernel<8, 3, 2>), grid, dim3(128), 0, st, p);
     Q3_LAUNCH_CHECK();
-    hipLaunchKernelGGL(flash_decode_combine<128>, dim3((unsigned)(B * Hkv), (unsigned)p.groups),
-                       dim3(256), 0, st, p);
+    if (B * Hkv >= kCombineByWave)
+      hipLaunchKernelGGL((flash_decode_combine<128, true>), dim3((unsigned)(B * Hkv)), dim3(256), 0, st, p);
+    else
+      hipLaunchKernelGGL((flash_decode_combine<128, false>), dim3((unsigned)(B * Hkv), (unsigned)p.groups), dim3(256), 0,
+                         st, p);
     Q3_LAUNCH_CHECK();
     return Q3_OK;
   }

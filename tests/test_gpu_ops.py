@@ -509,6 +509,25 @@ def test_decode_attention_c3_lengths():
             assert_bf16_close(o[b], ref, what=f"C3 decode b={b} L={L}")
 
 
+@pytest.mark.parametrize("B,Hkv,groups", [(51, 5, 4), (32, 8, 4), (64, 4, 1), (37, 7, 3), (43, 6, 8)])
+def test_decode_attention_many_pairs(B, Hkv, groups):
+    """(sequence, KV head) pairs on both sides of the 256 from which each wave merges whole heads: empty sequences, ones
+    inside a wave and ones over several, with appended lengths."""
+    D, cap = 128, 700
+    g = torch.Generator().manual_seed(B)
+    lens = torch.randint(0, 60, (B,), generator=g, dtype=torch.int32)
+    lens[::5] = torch.randint(300, cap, (len(lens[::5]),), generator=g, dtype=torch.int32)
+    lens[1], lens[2] = 0, cap
+    q = rnd(B, Hkv * groups, D, seed=32)
+    kc, vc = rnd(B, Hkv, cap, D, seed=33), rnd(B, Hkv, cap, D, seed=34)
+    ref = O.decode_attention(f32(q)[:, :, None], f32(kc), f32(vc), lens, D ** -0.5, groups)[:, :, 0]
+    assert_bf16_close(K.decode_attention(gpu(q), gpu(kc), gpu(vc), gpu(lens), D ** -0.5), ref, what="many pairs")
+    before = (lens - 1).clamp(min=0)
+    lens_d = gpu(before)
+    K.decode_attention(gpu(q), gpu(kc), gpu(vc), lens_d, D ** -0.5, append=True)
+    assert torch.equal(lens_d.cpu(), before + 1)
+
+
 # ------------------------------------------------------------------ rotary
 def test_apply_mrope_matches_oracle():
     B, H, S, D = 2, 4, 50, 128
