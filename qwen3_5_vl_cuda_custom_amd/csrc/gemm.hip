@@ -295,8 +295,9 @@ int launch_tiled_cfg(GemmParams p, int64_t batch, hipStream_t st) {
 // chip holds a higher clock. Same-box A/B, bit-identical outputs: the S=4096
 // decoder layer 1464.9 -> 1395.1 us (gate/up 633 -> 608, down 326 -> 307, o
 // 121 -> 116, q/k/v on 256x192); S=1024 475.7 -> 469.2 us. The MoE expert
-// tiles stay on 32x32x16: no faster with it. (The 128x128 deep ring and the
-// 128x256 tiles take it in their own forms: launch_c, launch_d.)
+// tiles on weights as (N, K) stay on 32x32x16: no faster with it (those of its
+// training backward, on untransposed weights, run it). (The 128x128 deep ring
+// and the 128x256 tiles take it in their own forms: launch_c, launch_d.)
 //
 // The 128x256 tiles on that loop keep a fourth W slot (2 X + 4 W slots of 64-wide
 // stages, 160 KB): M=1024 gate/up 185.1 -> 181.5 us, q/k/v 56.6 -> 55.2 us, the

@@ -4,8 +4,8 @@ from __future__ import annotations
 import torch
 from torch import nn
 
-from ..kernels import (cuda_index_add, cuda_topk, matmul, moe_experts, moe_experts_train, moe_route, moe_router, residual_add, softmax,
-                       swiglu)
+from ..kernels import (cuda_index_add, cuda_topk, matmul, moe_experts, moe_experts_train, moe_route, moe_router,
+                       residual_add, softmax, swiglu)
 from ..kernels.backward import needs_grad
 
 
